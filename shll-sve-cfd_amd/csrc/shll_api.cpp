@@ -83,6 +83,7 @@ static Consts make_consts(int64_t nx, int64_t ny, double lx, double ly, double t
         const float DX = L / (float)nx, DY = H / (float)ny;
         const float DT = (CFL / (R + 1.0f)) * DX;
         k.f_cv = (float)((double)R / ((double)GAMMA - 1.0));
+        k.f_rcv = 1.0 / (double)k.f_cv;
         k.f_gR = GAMMA * R;
         k.f_R = R;
         k.f_lamx = CFL / (R + 1.0f);

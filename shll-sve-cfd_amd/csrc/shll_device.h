@@ -12,8 +12,8 @@
 //
 // The library is compiled with -ffp-contract=off: every + - * below is one IEEE-754
 // operation in source order (fused multiply-adds only where written), and division
-// and square root are correctly rounded (div_rn, sqrt_rn), so the F64 and REF32
-// kernels reproduce the CPU results bit for bit (F64F alone uses faithful sequences).
+// and square root are correctly rounded, so the F64 and REF32 kernels reproduce the CPU
+// results bit for bit (F64F alone uses faithful sequences).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -100,13 +100,13 @@ __device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirs
 // pass of v_div_fixup, the square roots' pre-scaling of tiny radicands and their
 // pass-through of 0 and inf.  With operands and results of moderate size (no
 // intermediate leaves the normal range) they give the same bits as the operators.
-// div_rn and sqrt_rn check the result or radicand (a quotient of at least 2^-64 in
-// float or 2^-900 in double, a radicand of at least 2^-90 / 2^-760) and hand every
-// other case -- zero, tiny, denormal, NaN -- to the operators themselves, so they
-// are always bitwise '/' and sqrt.  The compensated scheme calls the fast paths
-// directly: its divisors (density, sound speed) and radicand (gamma*R*T) are of order
-// one, and its one possibly tiny quotient, the Mach number M, only enters as M/2 +-
-// 1/2 and 1 - M^2, which absorb any last-place difference of a tiny M.
+// The reference forms (F64, REF32) call them through RefArith::prim1_fast / prim2_fast, which
+// say per cell whether every intermediate stayed in that range (one test per cell, below), and
+// hand the other cells -- a vacuum, a tiny velocity, a non-finite state -- to the operators
+// themselves (prim1_exact / prim2_exact), so they are always bitwise '/' and sqrt.  The
+// compensated scheme calls the fast paths directly: its divisors (density, sound speed) and
+// radicand (gamma*R*T) are of order one, and its one possibly tiny quotient, the Mach number
+// M, only enters as M/2 +- 1/2 and 1 - M^2, which absorb any last-place difference of a tiny M.
 // ---------------------------------------------------------------------------
 // rcp_fast(b): 1/b correctly rounded -- v_rcp_f32 (within 1 ulp) and one Newton step with
 // fused multiply-adds.  Checked against IEEE 1.0f/b on the MI355X for every normal float b
@@ -155,18 +155,40 @@ __device__ __forceinline__ double sqrt_fast(double x) {
     d = __builtin_fma(-g, g, x);
     return __builtin_fma(d, h, g);
 }
-__device__ __forceinline__ float div_rn(float a, float b) {
-    float q = div_fast(a, b);
-    if (__builtin_expect(!(fabsf(q) >= 0x1p-64f), 0)) q = a / b;
-    return q;
+// a/b given y = 1/b correctly rounded (the last three operations of div_fast)
+template <class RT>
+__device__ __forceinline__ RT quot(RT a, RT b, RT y) {
+    const RT q = a * y;
+    const RT d = __builtin_elementwise_fma(-b, q, a);
+    return __builtin_elementwise_fma(d, y, q);
 }
-__device__ __forceinline__ double div_rn(double a, double b) {
-    double q = div_fast(a, b);
-    if (__builtin_expect(!(fabs(q) >= 0x1p-900), 0)) q = a / b;
-    return q;
+// 1/b as div_fast's two Newton steps give it
+__device__ __forceinline__ double rcp_2n(double b) {
+    double r = __builtin_amdgcn_rcp(b);
+    double e = __builtin_fma(-b, r, 1.0);
+    r = __builtin_fma(r, e, r);
+    e = __builtin_fma(-b, r, 1.0);
+    return __builtin_fma(r, e, r);
 }
-__device__ __forceinline__ double sqrt_rn(double x) {
-    return __builtin_expect(!(x >= 0x1p-760), 0) ? sqrt(x) : sqrt_fast(x);
+// s = sqrt(x) as sqrt_fast gives it, and y = 1/s: the square root's iteration already holds
+// h = 1/(2 sqrt(x)) to about 2^-46, so one Newton step on 2h replaces a reciprocal seed and two
+__device__ __forceinline__ void sqrt_rcp(double x, double& s, double& y) {
+    const double q = __builtin_amdgcn_rsq(x);
+    double g = x * q, h = q * 0.5;
+    const double r = __builtin_fma(-h, g, 0.5);
+    g = __builtin_fma(g, r, g);
+    h = __builtin_fma(h, r, h);
+    double d = __builtin_fma(-g, g, x);
+    g = __builtin_fma(d, h, g);
+    d = __builtin_fma(-g, g, x);
+    s = __builtin_fma(d, h, g);
+    const double w = h + h;
+    const double e = __builtin_fma(-s, w, 1.0);
+    y = __builtin_fma(w, e, w);
+}
+__device__ __forceinline__ void sqrt_rcp(float x, float& s, float& y) {
+    s = sqrt_fast(x);
+    y = rcp_fast(s);
 }
 
 // Faithful FP64 reciprocal and reciprocal square root (the F64F form): the hardware seeds
@@ -196,40 +218,105 @@ __device__ __forceinline__ double rsq_nr2(double x) {
 // (double) conversions sit where the reference's double literals and its double
 // sqrt() put them (base_shll.c:135-139, :172-175; base_shll_2d.c:313-317).
 // For RT = double every conversion is the identity.
+//
+// prim*_fast give the bits of prim*_exact in about half the instructions, and *ok = false
+// where they may not:
+//   - quotients with one divisor share its reciprocal (u1/u0, u2/u0, u3/u0; vx/a, vy/a); 1/cv
+//     is a constant (Consts::d_rcv, f_rcv, correctly rounded by the host);
+//   - e - kin is one fused multiply-add: kin/2's product is exact (a power of two times a
+//     rounded square, or in REF32 1D first order a 48-bit square in double);
+//   - (float)sqrt((double)x) of a float x is the float square root (rounding twice is
+//     harmless from 53 to 24 bits), so REF32 takes it in float;
+//   - a quotient of +-0 comes out as +0, a zero whose sign no sum here keeps.
+// One test per cell covers all of it: the radicand x = gamma R T in [XLO, XHI] and |M| >= MLO
+// or a zero velocity.  T > 0 then bounds e = cv T + kin below, x and M bound |vx| = |M| a, so
+// every quotient and residual is normal (or exactly zero); non-finite states fail the test on x.
+// Before, each of the five (2D: seven) operations carried its own compare and branch, and a
+// gas at rest (u = 0) took the slow path of two of them: 1D first order FP64, 1024 cells,
+// 5.43 us per 8-step launch, 4.2 us now; second order, 4 cells per lane: 894 VALU instructions per
+// step, 582 now; the whole 2D second-order REF32 run at 1024^2 1.12x.
 // ---------------------------------------------------------------------------
+template <class RT> struct RefRange;
+template <> struct RefRange<double> {
+    static constexpr double XLO = 0x1p-700, XHI = 0x1p+700, MLO = 0x1p-500;
+};
+template <> struct RefRange<float> {
+    static constexpr float XLO = 0x1p-30f, XHI = 0x1p+60f, MLO = 0x1p-45f;
+};
+
 template <class RT>
 struct RefArith {
-    // Compute_P_from_U, 1D.  ke = 0: (0.5*u)*u (base_shll.c:174); ke = 1: 0.5*(u*u)
+    static constexpr bool F32 = sizeof(RT) == 4;
+    // Compute_P_from_U, 1D.  KE = 0: (0.5*u)*u (base_shll.c:174); KE = 1: 0.5*(u*u)
     // (the 2D files' association, used by the derived 1D second-order scheme).
-    __device__ static __forceinline__ void prim1(RT u0, RT u1, RT u2, int ke, RT cv, RT gR, RT& vx, RT& T,
-                                                 RT& a) {
-        vx = div_rn(u1, u0);
+    // M = vx/a (base_shll.c:136).
+    __device__ static __forceinline__ void prim1_exact(RT u0, RT u1, RT u2, int ke, RT cv, RT gR, RT& vx, RT& T,
+                                                       RT& a, RT& M) {
+        vx = u1 / u0;
         double kin = ke == 0 ? (0.5 * (double)vx) * (double)vx : 0.5 * (double)(vx * vx);
-        T = (RT)div_rn((double)div_rn(u2, u0) - kin, (double)cv);
-        a = (RT)sqrt_rn((double)(gR * T));
+        T = (RT)(((double)(u2 / u0) - kin) / (double)cv);
+        a = (RT)sqrt((double)(gR * T));
+        M = vx / a;
     }
-    // Compute_P_from_U, 2D (base_shll_2d.c:313-317)
-    __device__ static __forceinline__ void prim2(RT u0, RT u1, RT u2, RT u3, RT cv, RT gR, RT& vx, RT& vy,
-                                                 RT& T, RT& a) {
-        vx = div_rn(u1, u0);
-        vy = div_rn(u2, u0);
-        T = (RT)div_rn((double)div_rn(u3, u0) - 0.5 * (double)(vx * vx + vy * vy), (double)cv);
-        a = (RT)sqrt_rn((double)(gR * T));
+    __device__ static __forceinline__ bool prim1_fast(RT u0, RT u1, RT u2, int ke, RT cv, double rcv, RT gR, RT& vx,
+                                                      RT& T, RT& a, RT& M) {
+        RT y;
+        if constexpr (F32) y = rcp_fast(u0);
+        else y = rcp_2n(u0);
+        vx = quot(u1, u0, y);
+        const double e = (double)quot(u2, u0, y);
+        const double vv = ke == 0 && F32 ? (double)vx * (double)vx : (double)(vx * vx);
+        T = (RT)quot(__builtin_fma(-0.5, vv, e), (double)cv, rcv);
+        return sound(u1, T, gR, vx, a, M, y);
     }
-    // Z invariants (base_shll.c:137-139)
+    // a = sqrt(gamma R T), y = 1/a, M = v/a and the range test (um: the momentum of v)
+    __device__ static __forceinline__ bool sound(RT um, RT T, RT gR, RT v, RT& a, RT& M, RT& y) {
+        using R = RefRange<RT>;
+        const RT x = gR * T;
+        sqrt_rcp(x, a, y);
+        M = quot(v, a, y);
+        return x >= R::XLO && x <= R::XHI && (fabs(M) >= R::MLO || um == (RT)0);
+    }
+    // Compute_P_from_U, 2D (base_shll_2d.c:313-317), and the two Mach numbers
+    __device__ static __forceinline__ void prim2_exact(RT u0, RT u1, RT u2, RT u3, RT cv, RT gR, RT& vx, RT& vy,
+                                                       RT& T, RT& a, RT& Mx, RT& My) {
+        vx = u1 / u0;
+        vy = u2 / u0;
+        T = (RT)(((double)(u3 / u0) - 0.5 * (double)(vx * vx + vy * vy)) / (double)cv);
+        a = (RT)sqrt((double)(gR * T));
+        Mx = vx / a;
+        My = vy / a;
+    }
+    __device__ static __forceinline__ bool prim2_fast(RT u0, RT u1, RT u2, RT u3, RT cv, double rcv, RT gR, RT& vx,
+                                                      RT& vy, RT& T, RT& a, RT& Mx, RT& My) {
+        using R = RefRange<RT>;
+        RT y;
+        if constexpr (F32) y = rcp_fast(u0);
+        else y = rcp_2n(u0);
+        vx = quot(u1, u0, y);
+        vy = quot(u2, u0, y);
+        const double e = (double)quot(u3, u0, y);
+        T = (RT)quot(__builtin_fma(-0.5, (double)(vx * vx + vy * vy), e), (double)cv, rcv);
+        const bool ok = sound(u1, T, gR, vx, a, Mx, y);
+        My = quot(vy, a, y);
+        return ok && (fabs(My) >= R::MLO || u2 == (RT)0);
+    }
+    // Z invariants (base_shll.c:137-139): 0.5*(M +- 1) in double, stored to RT, is M/2 +- 1/2
+    // rounded once: M/2 is exact, and for a float M the double sum is exact or nowhere near the
+    // middle of two floats
     __device__ static __forceinline__ void zinv(RT M, RT a, RT& z1, RT& z2, RT& z3) {
-        z1 = (RT)(0.5 * ((double)M + 1.0));
+        z1 = __builtin_elementwise_fma((RT)0.5, M, (RT)0.5);
         z2 = (RT)((0.5 * (double)a) * (1.0 - (double)(M * M)));
-        z3 = (RT)(0.5 * ((double)M - 1.0));
+        z3 = __builtin_elementwise_fma((RT)0.5, M, (RT)-0.5);
     }
     // minmod (2nd_order_base_shll.c:191-201): product sign test, ties -> right
     __device__ static __forceinline__ RT mm(RT l, RT r) {
-        RT pick = fabs((double)l) < fabs((double)r) ? l : r;
-        return (double)(l * r) < 0.0 ? (RT)0 : pick;
+        RT pick = fabs(l) < fabs(r) ? l : r;
+        return l * r < (RT)0 ? (RT)0 : pick;
     }
     // 0.5*(difference) with the double literal of base-omp/2nd_order_base_shll.c:317,
-    // rounded to RT as minmod's argument
-    __device__ static __forceinline__ RT half(RT x) { return (RT)(0.5 * (double)x); }
+    // rounded to RT as minmod's argument (halving is exact, or rounds once, in either type)
+    __device__ static __forceinline__ RT half(RT x) { return (RT)0.5 * x; }
 };
 
 // FP32-compensated arithmetic: float, with explicit fused multiply-adds where a

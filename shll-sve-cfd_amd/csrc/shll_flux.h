@@ -13,6 +13,46 @@ template <> struct Real<PREC_REF32> { using T = float; };
 template <> struct Real<PREC_C32> { using T = float; };
 template <> struct Real<PREC_C32K> { using T = float; };
 
+// constants of the reference forms, by type
+template <class RT>
+__device__ __forceinline__ void ref_consts(const Inst& in, RT& cv, double& rcv, RT& gR) {
+    if constexpr (sizeof(RT) == 8) {
+        cv = in.k.d_cv;
+        rcv = in.k.d_rcv;
+        gR = in.k.d_gR;
+    } else {
+        cv = in.k.f_cv;
+        rcv = in.k.f_rcv;
+        gR = in.k.f_gR;
+    }
+}
+// Compute_P_from_U of one cell: the fast form (false: take the exact one), the exact form
+template <class RT>
+__device__ __forceinline__ bool ref_prim1(RT u0, RT u1, RT u2, const Inst& in, RT& vx, RT& T, RT& a, RT& M) {
+    RT cv, gR;
+    double rcv;
+    ref_consts<RT>(in, cv, rcv, gR);
+    return RefArith<RT>::prim1_fast(u0, u1, u2, in.ke, cv, rcv, gR, vx, T, a, M);
+}
+template <class RT>
+__device__ __forceinline__ void ref_prim1_exact(RT u0, RT u1, RT u2, const Inst& in, RT& vx, RT& T, RT& a, RT& M) {
+    RT cv, gR;
+    double rcv;
+    ref_consts<RT>(in, cv, rcv, gR);
+    RefArith<RT>::prim1_exact(u0, u1, u2, in.ke, cv, gR, vx, T, a, M);
+}
+// Compute_F_from_P of one cell (base_shll.c:134-157)
+template <class RT>
+__device__ __forceinline__ void ref_flux1(RT u0, RT u1, RT u2, RT vx, RT T, RT a, RT M, RT (&fp)[3], RT (&fm)[3]) {
+    RT z1, z2, z3;
+    RefArith<RT>::zinv(M, a, z1, z2, z3);
+    const RT P = u0 * T;  // (rho*R)*T with R = 1 (base_shll.c:17, :141)
+    const RT f0 = u1, f1 = u1 * vx + P, f2 = vx * (u2 + P);
+    split<RT>(f0, u0, z1, z2, z3, fp[0], fm[0]);
+    split<RT>(f1, u1, z1, z2, z3, fp[1], fm[1]);
+    split<RT>(f2, u2, z1, z2, z3, fp[2], fm[2]);
+}
+
 // 1D, F64F: F+ and F- of the three variables scaled by sc, and the sound speed a
 // (base_shll.c:134-157 in the compensated forms' arrangement).  The step kernels pass
 // sc = DT/DX, so that their face term is G + d/2 with no product by DT/DX (the minmod and
@@ -55,15 +95,9 @@ __device__ __forceinline__ void flux1(RT u0, RT u1, RT u2, const Inst& in, RT (&
         split_c32(f1, u1, z1, z2, z3, fp[1], fm[1]);
         split_c32(f2, u2, z1, z2, z3, fp[2], fm[2]);
     } else {
-        const RT cv = PREC == PREC_F64 ? (RT)in.k.d_cv : (RT)in.k.f_cv;
-        const RT gR = PREC == PREC_F64 ? (RT)in.k.d_gR : (RT)in.k.f_gR;
-        RefArith<RT>::prim1(u0, u1, u2, in.ke, cv, gR, vx, T, a);
-        RefArith<RT>::zinv(div_rn(vx, a), a, z1, z2, z3);
-        const RT P = u0 * T;  // (rho*R)*T with R = 1 (base_shll.c:17, :141)
-        const RT f0 = u1, f1 = u1 * vx + P, f2 = vx * (u2 + P);
-        split<RT>(f0, u0, z1, z2, z3, fp[0], fm[0]);
-        split<RT>(f1, u1, z1, z2, z3, fp[1], fm[1]);
-        split<RT>(f2, u2, z1, z2, z3, fp[2], fm[2]);
+        RT M;
+        if (!ref_prim1<RT>(u0, u1, u2, in, vx, T, a, M)) ref_prim1_exact<RT>(u0, u1, u2, in, vx, T, a, M);
+        ref_flux1<RT>(u0, u1, u2, vx, T, a, M, fp, fm);
     }
 }
 
@@ -72,13 +106,15 @@ __device__ __forceinline__ void flux1(RT u0, RT u1, RT u2, const Inst& in, RT (&
 template <int PREC, class RT>
 __device__ __forceinline__ void fluxes2(const RT (&U)[4], const Inst& in, RT (&xp)[4], RT (&xm)[4], RT (&yp)[4],
                                         RT (&ym)[4], RT& a) {
-    RT vx, vy, T, z1, z2, z3;
+    RT vx, vy, T, z1, z2, z3, Mx, My;
     if constexpr (PREC == PREC_C32 || PREC == PREC_C32K) {
         C32Arith::prim2(U[0], U[1], U[2], U[3], in.k.c_rcv, in.k.c_gR, vx, vy, T, a);
     } else {
-        const RT cv = PREC == PREC_F64 ? (RT)in.k.d_cv : (RT)in.k.f_cv;
-        const RT gR = PREC == PREC_F64 ? (RT)in.k.d_gR : (RT)in.k.f_gR;
-        RefArith<RT>::prim2(U[0], U[1], U[2], U[3], cv, gR, vx, vy, T, a);
+        RT cv, gR;
+        double rcv;
+        ref_consts<RT>(in, cv, rcv, gR);
+        if (!RefArith<RT>::prim2_fast(U[0], U[1], U[2], U[3], cv, rcv, gR, vx, vy, T, a, Mx, My))
+            RefArith<RT>::prim2_exact(U[0], U[1], U[2], U[3], cv, gR, vx, vy, T, a, Mx, My);
     }
     const RT P = U[0] * T;  // (rho*R)*T with R = 1 (base_shll_2d.c:24, :246)
     if constexpr (PREC == PREC_C32 || PREC == PREC_C32K) {
@@ -95,13 +131,13 @@ __device__ __forceinline__ void fluxes2(const RT (&U)[4], const Inst& in, RT (&x
         split_c32(vy * (U[3] + P), U[3], z1, z2, z3, yp[3], ym[3]);
     } else {
         // x direction (base_shll_2d.c:249-272)
-        RefArith<RT>::zinv(div_rn(vx, a), a, z1, z2, z3);
+        RefArith<RT>::zinv(Mx, a, z1, z2, z3);
         split<RT>(U[1], U[0], z1, z2, z3, xp[0], xm[0]);
         split<RT>(U[1] * vx + P, U[1], z1, z2, z3, xp[1], xm[1]);
         split<RT>(U[1] * vy, U[2], z1, z2, z3, xp[2], xm[2]);
         split<RT>(vx * (U[3] + P), U[3], z1, z2, z3, xp[3], xm[3]);
         // y direction (base_shll_2d.c:275-298)
-        RefArith<RT>::zinv(div_rn(vy, a), a, z1, z2, z3);
+        RefArith<RT>::zinv(My, a, z1, z2, z3);
         split<RT>(U[2], U[0], z1, z2, z3, yp[0], ym[0]);
         split<RT>(U[2] * vx, U[1], z1, z2, z3, yp[1], ym[1]);
         split<RT>(U[2] * vy + P, U[2], z1, z2, z3, yp[2], ym[2]);

@@ -254,21 +254,39 @@ __device__ __forceinline__ void ghost_cells(RT (&q)[3][C], int gl, int n, bool r
 // ---------------------------------------------------------------------------
 // F64 / REF32: the reference association, cell by cell
 // ---------------------------------------------------------------------------
+// u - k*x in one fused multiply-add: for k a power of two (k*x is exact) the bits of the two
+// operations
+template <class RT>
+__device__ __forceinline__ RT fms(RT k, RT x, RT u) { return __builtin_elementwise_fma(-k, x, u); }
+
 template <int PREC, int ORDER, int C, int WM, int LIM, int XW>
 __device__ __forceinline__ void step_ref(typename Real<PREC>::T (&u)[3][C], const Inst& in, int gl,
                                          const Coop<typename Real<PREC>::T, XW>& x, int parity) {
     using RT = typename Real<PREC>::T;
     using A = RefArith<RT>;
-    const RT lam = PREC == PREC_F64 ? (RT)in.k.d_lamx : (RT)in.k.f_lamx;
+    // DT/DX = CFL/(R + 1) = 1/8 (base_shll.c:18,84): products with it and its half are exact, so
+    // u - lam*x and the second-order term (formed in double by the reference, then stored to
+    // float: harmless twice-rounding of a sum of two floats) are fused multiply-adds
+    constexpr RT lam = (RT)0.125, hlam = (RT)0.0625;
     const RT th = PREC == PREC_F64 ? (RT)in.k.d_theta : (RT)in.k.f_theta;
     const int n = in.nx;
     const bool refl = in.bc == BC_REFLECT;
     if constexpr (WM != WM_NONE) ghost_cells<C>(u, gl, n, refl);
     RT fp[3][C], fm[3][C];
+    // primitives of all cells, then one branch for the lanes with a cell outside the fast
+    // form's range, so the cells' dependent chains overlap
+    RT vx[C], T[C], sa[C], M[C];
+    bool ok = true;
+#pragma unroll
+    for (int m = 0; m < C; ++m) ok &= ref_prim1<RT>(u[0][m], u[1][m], u[2][m], in, vx[m], T[m], sa[m], M[m]);
+    if (__builtin_expect(!ok, 0)) {
+#pragma unroll
+        for (int m = 0; m < C; ++m) ref_prim1_exact<RT>(u[0][m], u[1][m], u[2][m], in, vx[m], T[m], sa[m], M[m]);
+    }
 #pragma unroll
     for (int m = 0; m < C; ++m) {
-        RT p[3], q[3], a;
-        flux1<PREC, RT>(u[0][m], u[1][m], u[2][m], in, p, q, a);
+        RT p[3], q[3];
+        ref_flux1<RT>(u[0][m], u[1][m], u[2][m], vx[m], T[m], sa[m], M[m], p, q);
 #pragma unroll
         for (int v = 0; v < 3; ++v) {
             fp[v][m] = p[v];
@@ -284,9 +302,8 @@ __device__ __forceinline__ void step_ref(typename Real<PREC>::T (&u)[3][C], cons
             for (int m = 0; m < C; ++m) {
                 // F+ of the left neighbour, F- of the right one; own slopes, the left
                 // neighbour's F+ slope and the right neighbour's F- slope
-                RT uu = u[v][m] - lam * (fp[v][m] - fm[v][m] + w.FM[m + 2] - w.FP[m]);
-                uu = (RT)((double)uu - 0.5 * (double)lam * (double)(w.sp(m + 1) + w.sm(m) - w.sm(m + 1) - w.sp(m)));
-                u[v][m] = uu;
+                const RT uu = fms(lam, fp[v][m] - fm[v][m] + w.FM[m + 2] - w.FP[m], u[v][m]);
+                u[v][m] = fms(hlam, w.sp(m + 1) + w.sm(m) - w.sm(m + 1) - w.sp(m), uu);
             }
         }
         return;
@@ -308,7 +325,7 @@ __device__ __forceinline__ void step_ref(typename Real<PREC>::T (&u)[3][C], cons
         for (int m = 0; m < C; ++m) {
             const int g = gl + m;
             // FL = F+ of the left neighbour, FR = F- of the right one (ghosts at the walls)
-            RT uu = u[v][m] - lam * (fp[v][m] - fm[v][m] + FM[m + 3] - FP[m + 1]);
+            RT uu = fms(lam, fp[v][m] - fm[v][m] + FM[m + 3] - FP[m + 1], u[v][m]);
             if constexpr (ORDER == 2) {
                 // own slopes, the left neighbour's F+ slope and the right neighbour's F-
                 // slope; every slope of a boundary or ghost cell is zero
@@ -316,7 +333,7 @@ __device__ __forceinline__ void step_ref(typename Real<PREC>::T (&u)[3][C], cons
                 RT dm = slope_at<A, WM, LIM>(FM, m, g, n, th);
                 RT Ldf = slope_at<A, WM, LIM>(FP, m - 1, g - 1, n, th);
                 RT Rdf = slope_at<A, WM, LIM>(FM, m + 1, g + 1, n, th);
-                uu = (RT)((double)uu - 0.5 * (double)lam * (double)(dp + dm - Rdf - Ldf));
+                uu = fms(hlam, dp + dm - Rdf - Ldf, uu);
             }
             u[v][m] = uu;
         }

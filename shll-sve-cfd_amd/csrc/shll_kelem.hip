@@ -97,13 +97,14 @@ __global__ __launch_bounds__(256) void k_output(const Inst* insts, const void* s
         load_cons<PREC, DIM>(s0, s1, plane, o, U);
         if constexpr (PREC == PREC_REF32) {
             const float* u = (const float*)s0;
-            float vx, vy = 0.f, T, a;
+            float vx, vy = 0.f, T, a, M;
             if constexpr (DIM == 1) {
-                RefArith<float>::prim1(u[o], u[plane + o], u[2 * plane + o], in.ke, in.k.f_cv, in.k.f_gR, vx, T, a);
+                RefArith<float>::prim1_exact(u[o], u[plane + o], u[2 * plane + o], in.ke, in.k.f_cv, in.k.f_gR, vx, T, a,
+                                             M);
                 p[0] = u[o]; p[1] = vx; p[2] = T;
             } else {
-                RefArith<float>::prim2(u[o], u[plane + o], u[2 * plane + o], u[3 * plane + o], in.k.f_cv, in.k.f_gR,
-                                       vx, vy, T, a);
+                RefArith<float>::prim2_exact(u[o], u[plane + o], u[2 * plane + o], u[3 * plane + o], in.k.f_cv,
+                                             in.k.f_gR, vx, vy, T, a, M, M);
                 p[0] = u[o]; p[1] = vx; p[2] = vy; p[3] = T;
             }
         } else {
