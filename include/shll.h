@@ -174,8 +174,9 @@ shll_status shll_compare_host(shll_ctx *ctx, const double *ref_prim_soa, shll_er
 void shll_free(shll_ctx *ctx);
 
 /* Launch shape of the step kernels.  cells_per_lane: 1D in {1,2,4,8}; 2D the owned rows
- * of a work item, the cells of its column each lane owns (2-4096; 0 or 1: 16, 32 or 64
- * rows for 1, 2 or more steps per launch), steps_per_launch >= 1 (temporal blocking; 2D:
+ * of a work item, the cells of its column each lane owns (2-4096; 0 or 1: the library's
+ * choice, 32 or 64 rows for 2 or more steps per launch, and for 1 step 16 or, in second
+ * order, 2-16 by the size of the domain), steps_per_launch >= 1 (temporal blocking; 2D:
  * 1, 2, 3, 4 or 8 in first order; 1, or 2 for SHLL_C32/SHLL_C32K in second order),
  * waves_per_block in {1,4} (1D, 4 with 2+ cells per lane: the block's wavefronts hold
  * one segment and share their edge fluxes), graph_steps: steps captured per HIP graph

@@ -174,10 +174,10 @@ struct Launch {
     int rows = 16;      // owned rows per 2D item
 };
 
-// Default owned rows per 2D item for k steps per launch: an item recomputes order*k halo
-// rows on each side, so longer items waste less; 16 rows at one step per launch.  In 2D the
-// launch's cells_per_lane sets the rows instead (each lane owns that many cells of its
-// column); 0 or 1 selects this default.
+// Owned rows per 2D item for k steps per launch: an item recomputes order*k halo rows on each
+// side, so longer items waste less; 16 rows at one step per launch (second order chooses by
+// size, default_rows2d).  In 2D the launch's cells_per_lane sets the rows instead (each lane
+// owns that many cells of its column); 0 or 1 selects this default.
 static int rows2d(int k) { return k <= 1 ? 16 : (k == 2 ? 32 : 64); }
 static constexpr int kMaxRows2d = 4096;
 static constexpr int kMaxGraphLaunches = 4096;  // launches per captured graph
@@ -219,21 +219,25 @@ static bool tile1d(int32_t inst, int64_t nx, int order, int C, int XW, int k, st
     return true;
 }
 
+// Owned columns of a strip of 64 with `rest` columns left: H fewer on each side that is cut.  The
+// last strip reaches the wall, so it has no halo there (1024 columns in second order: 62 +
+// 15 x 60 + 62, 17 strips; with a halo past the wall it took 18, the last with 2 columns).
+static int64_t strip_cols(int64_t rest, int64_t H, bool first) {
+    const int64_t left = first ? 0 : H;
+    return rest <= 64 - left ? rest : 64 - left - H;
+}
+
 // 2D tiling: strips of 64 columns (one wavefront) whose outer H = order*k columns on a
 // cut side are recomputed halo, times runs of `rows` owned rows (H halo rows each side).
 static void tile2d(int32_t inst, int64_t nx, int64_t ny, int order, int k, int rows, std::vector<Item2>& out) {
     struct Strip { int32_t j0, jx0, jw; };
     std::vector<Strip> strips;
     const int64_t H = (int64_t)order * k;
-    {
-        int64_t jw = std::min<int64_t>(ny, 64 - H);
-        strips.push_back(Strip{0, 0, (int32_t)jw});
-        int64_t jx0 = jw;
-        while (jx0 < ny) {
-            int64_t w = std::min<int64_t>(ny - jx0, 64 - 2 * H);
-            strips.push_back(Strip{(int32_t)(jx0 - H), (int32_t)jx0, (int32_t)w});
-            jx0 += w;
-        }
+    for (int64_t jx0 = 0, j0 = 0; jx0 < ny;) {
+        const int64_t w = strip_cols(ny - jx0, H, jx0 == 0);
+        strips.push_back(Strip{(int32_t)j0, (int32_t)jx0, (int32_t)w});
+        jx0 += w;
+        j0 = jx0 - H;
     }
     for (int64_t ix0 = 0; ix0 < nx; ix0 += rows) {
         const int64_t iw = std::min<int64_t>(rows, nx - ix0);
@@ -301,6 +305,51 @@ struct Engine {
     int64_t last_launches = 0;
     bool batch = false;
 };
+
+// 2D work items of every instance at k steps per launch and `rows` owned rows per item
+// (the counts tile2d produces)
+static int64_t items2d(const Engine* E, int k, int rows) {
+    const int64_t H = (int64_t)E->order * k;
+    int64_t n = 0;
+    for (const Inst& in : E->h_inst) {
+        int64_t strips = 0;
+        for (int64_t jx0 = 0; jx0 < in.ny; ++strips) jx0 += strip_cols(in.ny - jx0, H, jx0 == 0);
+        n += strips * ((in.nx + rows - 1) / rows);
+    }
+    return n;
+}
+
+static int64_t simd_count(const Engine* E) {
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, E->device) != hipSuccess) return 1024;
+    return 4LL * cus;
+}
+
+// Owned rows per item when the launch shape leaves them to the library.  Second order, one
+// step per launch: a wavefront walks its rows one after another, so a launch lasts about
+//   (rows + 3.3) x max(L, wavefronts of the fullest SIMD)
+// in units of a row's issue time: the halo rows and start-up of an item cost about 3.3 rows, and
+// a SIMD with few wavefronts waits on the latency of a row, L = 1.5 (FP64) or 2.5 (32-bit forms)
+// issue times.  Rows of 2 to 16 that minimise this.  Measured, us per step: FP64 777x613 4 rows
+// 16.8, 6 rows 16.2, 8 rows 19.6, 9 rows 15.4 (one wavefront per SIMD), 13 rows 19.9; REF32 MC
+// 1024^2 3 rows 22.8, 5 rows 21.2, 8 rows 23.4, 12 rows 25.2; FP64 2048^2 8 or 16 rows 72, 32
+// rows 84; REF32 MC 4096^2 16 or 32 rows 191, 60 rows 211.
+static int default_rows2d(const Engine* E, int k) {
+    if (E->order != 2 || k != 1) return rows2d(k);
+    const int64_t simds = simd_count(E);
+    const double lat = word_bytes(E->prec) == 8 ? 1.5 : 2.5;
+    int best = 16;
+    double cost = 1e300;
+    for (int rows = 16; rows >= 2; --rows) {
+        const double waves = (double)((items2d(E, k, rows) + simds - 1) / simds);
+        const double c = (rows + 3.3) * std::max(lat, waves);
+        if (c < cost) {
+            cost = c;
+            best = rows;
+        }
+    }
+    return best;
+}
 
 static void engine_drop_graphs(Engine* E) {
     for (int p = 0; p < 2; ++p)
@@ -794,15 +843,19 @@ static void default_launch(Engine* E, int64_t max_cells) {
     if (E->dim == 2) {
         // First order: several steps per launch (row-pipelined stages); measured on a
         // 4096^2 domain and a 64-domain batch, the FP32 forms peak at 4 steps per launch,
-        // FP64 (twice the registers per stage) at 2.  Second order: C32K 2 steps per launch
-        // (7.5e10 vs 5.9e10 cell-updates/s at 4096^2); the TwoSum form's two-row stages
-        // overflow the registers (4.4e10 vs 5.3e10), so it and FP64/REF32 take one step per
-        // launch in 16-row items (a 4096^2 domain in 64-row items leaves ~4 wavefronts per
-        // SIMD, too few to cover the row loads).
+        // FP64 (twice the registers per stage) at 2.  Second order: one step per launch, but
+        // C32K takes two on domains whose two state buffers exceed the 256 MiB last-level
+        // cache, where one step is bound by HBM (us per step, 1 and 2 steps per launch: 1024^2
+        // 16.4 and 32.2, 2048^2 55 and 58, 3072^2 163 and 108); the TwoSum form's two-row
+        // stages overflow the registers (3072^2 162 and 183).
+        int64_t cells = 0;
+        for (int64_t c : E->inst_cells) cells += c;
+        const bool in_cache = cells * 64 <= (256LL << 20);
         E->L.C = 1;
-        E->L.k = E->order == 1 ? (E->prec == PREC_C32 || E->prec == PREC_C32K ? 4 : 2) : (E->prec == PREC_C32K ? 2 : 1);
+        E->L.k = E->order == 1 ? (E->prec == PREC_C32 || E->prec == PREC_C32K ? 4 : 2)
+                               : (E->prec == PREC_C32K && !in_cache ? 2 : 1);
         E->L.wpb = 4;
-        E->L.rows = rows2d(E->L.k);
+        E->L.rows = default_rows2d(E, E->L.k);
         E->L.graph = 64;
         return;
     }
@@ -1158,7 +1211,7 @@ static shll_status set_launch(Engine* E, int32_t C, int32_t k, int32_t wpb, int3
     Launch old = E->L;
     E->L.C = E->dim == 1 ? C : (C <= 1 ? 1 : C);
     E->L.k = k;
-    if (E->dim == 2) E->L.rows = C <= 1 ? rows2d(k) : C;
+    if (E->dim == 2) E->L.rows = C <= 1 ? default_rows2d(E, k) : C;
     E->L.wpb = wpb;
     E->L.graph = graph;
     E->items_valid = false;
@@ -1250,25 +1303,6 @@ static void tune_cache_store(const std::string& key, const Launch& L) {
     if (!f) return;
     std::fprintf(f, "%s|%d %d %d %d\n", key.c_str(), L.C, L.k, L.wpb, L.graph);
     std::fclose(f);
-}
-
-// 2D work items of every instance at k steps per launch and `rows` owned rows per item
-// (the counts tile2d produces)
-static int64_t items2d(const Engine* E, int k, int rows) {
-    const int64_t H = (int64_t)E->order * k;
-    int64_t n = 0;
-    for (const Inst& in : E->h_inst) {
-        int64_t strips = 1;
-        if (in.ny > 64 - H) strips += (in.ny - (64 - H) + (64 - 2 * H) - 1) / (64 - 2 * H);
-        n += strips * ((in.nx + rows - 1) / rows);
-    }
-    return n;
-}
-
-static int64_t simd_count(const Engine* E) {
-    hipDeviceProp_t prop;
-    if (hipGetDeviceProperties(&prop, E->device) != hipSuccess) return 1024;
-    return 4LL * prop.multiProcessorCount;
 }
 
 static shll_status engine_autotune(Engine* E, int32_t trial_steps, int64_t shape_class,

@@ -101,24 +101,73 @@ __device__ __forceinline__ void flux1(RT u0, RT u1, RT u2, const Inst& in, RT (&
     }
 }
 
+// 2D reference forms: Compute_P_from_U of one cell and the Mach numbers (as ref_prim1)
+template <class RT>
+struct Prim2 {
+    RT vx, vy, T, a, Mx, My;
+};
+template <class RT>
+__device__ __forceinline__ bool ref_prim2(const RT (&U)[4], const Inst& in, Prim2<RT>& q) {
+    RT cv, gR;
+    double rcv;
+    ref_consts<RT>(in, cv, rcv, gR);
+    return RefArith<RT>::prim2_fast(U[0], U[1], U[2], U[3], cv, rcv, gR, q.vx, q.vy, q.T, q.a, q.Mx, q.My);
+}
+template <class RT>
+__device__ __forceinline__ void ref_prim2_exact(const RT (&U)[4], const Inst& in, Prim2<RT>& q) {
+    RT cv, gR;
+    double rcv;
+    ref_consts<RT>(in, cv, rcv, gR);
+    RefArith<RT>::prim2_exact(U[0], U[1], U[2], U[3], cv, gR, q.vx, q.vy, q.T, q.a, q.Mx, q.My);
+}
+// Compute_F_from_P of one cell, x and y (base_shll_2d.c:239-298)
+template <class RT>
+__device__ __forceinline__ void ref_flux2(const RT (&U)[4], const Prim2<RT>& q, RT (&xp)[4], RT (&xm)[4], RT (&yp)[4],
+                                          RT (&ym)[4]) {
+    RT z1, z2, z3;
+    const RT P = U[0] * q.T;  // (rho*R)*T with R = 1 (base_shll_2d.c:24, :246)
+    RefArith<RT>::zinv(q.Mx, q.a, z1, z2, z3);
+    split<RT>(U[1], U[0], z1, z2, z3, xp[0], xm[0]);
+    split<RT>(U[1] * q.vx + P, U[1], z1, z2, z3, xp[1], xm[1]);
+    split<RT>(U[1] * q.vy, U[2], z1, z2, z3, xp[2], xm[2]);
+    split<RT>(q.vx * (U[3] + P), U[3], z1, z2, z3, xp[3], xm[3]);
+    RefArith<RT>::zinv(q.My, q.a, z1, z2, z3);
+    split<RT>(U[2], U[0], z1, z2, z3, yp[0], ym[0]);
+    split<RT>(U[2] * q.vx, U[1], z1, z2, z3, yp[1], ym[1]);
+    split<RT>(U[2] * q.vy + P, U[2], z1, z2, z3, yp[2], ym[2]);
+    split<RT>(q.vy * (U[3] + P), U[3], z1, z2, z3, yp[3], ym[3]);
+}
+
+// The reference's 2D update terms: u - lam*x, and the second-order u - 0.5*lam*x formed in
+// double and stored to RT.  EIGHTH: lam = CFL/(R + 1) = 1/8 (DT/DX always, base_shll.c:18,84;
+// DT/DY on square cells), whose products are exact, so one fused multiply-add gives the same
+// bits (for a float u the second rounding of the double sum is harmless).  The transverse
+// momentum's fluxes are products of two velocities and reach the denormal range ahead of a
+// front, where a product with 1/8 rounds: it keeps the two operations.
+template <class RT>
+struct RefUpdate {
+    template <bool EIGHTH>
+    __device__ static __forceinline__ RT first(bool transverse, RT u, RT lam, RT x) {
+        if (EIGHTH && !transverse) return __builtin_elementwise_fma((RT)-0.125, x, u);
+        return u - lam * x;
+    }
+    template <bool EIGHTH>
+    __device__ static __forceinline__ RT second(bool transverse, RT u, RT lam, RT x) {
+        if (EIGHTH && (sizeof(RT) == 4 || !transverse)) return __builtin_elementwise_fma((RT)-0.0625, x, u);
+        return (RT)((double)u - 0.5 * (double)lam * (double)x);
+    }
+};
+
 // x and y split fluxes of one cell (Compute_P_from_U + Compute_F_from_P, base_shll_2d.c:239-319)
 // and its sound speed a.  U: conserved (F64/REF32: the state; C32: hi).
 template <int PREC, class RT>
 __device__ __forceinline__ void fluxes2(const RT (&U)[4], const Inst& in, RT (&xp)[4], RT (&xm)[4], RT (&yp)[4],
                                         RT (&ym)[4], RT& a) {
-    RT vx, vy, T, z1, z2, z3, Mx, My;
-    if constexpr (PREC == PREC_C32 || PREC == PREC_C32K) {
-        C32Arith::prim2(U[0], U[1], U[2], U[3], in.k.c_rcv, in.k.c_gR, vx, vy, T, a);
-    } else {
-        RT cv, gR;
-        double rcv;
-        ref_consts<RT>(in, cv, rcv, gR);
-        if (!RefArith<RT>::prim2_fast(U[0], U[1], U[2], U[3], cv, rcv, gR, vx, vy, T, a, Mx, My))
-            RefArith<RT>::prim2_exact(U[0], U[1], U[2], U[3], cv, gR, vx, vy, T, a, Mx, My);
-    }
-    const RT P = U[0] * T;  // (rho*R)*T with R = 1 (base_shll_2d.c:24, :246)
     if constexpr (PREC == PREC_C32 || PREC == PREC_C32K) {
         // the compensated scheme's float form: fused multiply-adds (split_c32)
+        RT vx, vy, T, z1, z2, z3;
+        C32Arith::prim2(U[0], U[1], U[2], U[3], in.k.c_rcv, in.k.c_gR, vx, vy, T, a);
+        const RT P = U[0] * T;
         C32Arith::zinv(div_fast(vx, a), a, z1, z2, z3);
         split_c32(U[1], U[0], z1, z2, z3, xp[0], xm[0]);
         split_c32(__builtin_fmaf(U[1], vx, P), U[1], z1, z2, z3, xp[1], xm[1]);
@@ -130,18 +179,10 @@ __device__ __forceinline__ void fluxes2(const RT (&U)[4], const Inst& in, RT (&x
         split_c32(__builtin_fmaf(U[2], vy, P), U[2], z1, z2, z3, yp[2], ym[2]);
         split_c32(vy * (U[3] + P), U[3], z1, z2, z3, yp[3], ym[3]);
     } else {
-        // x direction (base_shll_2d.c:249-272)
-        RefArith<RT>::zinv(Mx, a, z1, z2, z3);
-        split<RT>(U[1], U[0], z1, z2, z3, xp[0], xm[0]);
-        split<RT>(U[1] * vx + P, U[1], z1, z2, z3, xp[1], xm[1]);
-        split<RT>(U[1] * vy, U[2], z1, z2, z3, xp[2], xm[2]);
-        split<RT>(vx * (U[3] + P), U[3], z1, z2, z3, xp[3], xm[3]);
-        // y direction (base_shll_2d.c:275-298)
-        RefArith<RT>::zinv(My, a, z1, z2, z3);
-        split<RT>(U[2], U[0], z1, z2, z3, yp[0], ym[0]);
-        split<RT>(U[2] * vx, U[1], z1, z2, z3, yp[1], ym[1]);
-        split<RT>(U[2] * vy + P, U[2], z1, z2, z3, yp[2], ym[2]);
-        split<RT>(vy * (U[3] + P), U[3], z1, z2, z3, yp[3], ym[3]);
+        Prim2<RT> q;
+        if (!ref_prim2<RT>(U, in, q)) ref_prim2_exact<RT>(U, in, q);
+        ref_flux2<RT>(U, q, xp, xm, yp, ym);
+        a = q.a;
     }
 }
 

@@ -26,8 +26,277 @@ namespace shll {
 __device__ __forceinline__ int sgn_x(int v) { return v == 1 ? 1 : -1; }
 __device__ __forceinline__ int sgn_y(int v) { return v == 2 ? 1 : -1; }
 
-template <int PREC, int ORDER, int WPB, int LIM>
+// A lane's y walls, as per-lane flags (lane-varying, so the wall choices are selects
+// rather than branches): lo / hi = the lane is column 0 / ny-1, *_refl = and reflective;
+// edge = on or beyond such a column (no slope)
+struct LaneWalls {
+    bool lo, hi, lo_refl, hi_refl, refl, edge;
+};
+
+// ---------------------------------------------------------------------------
+// Second order, one step per launch: a wavefront streams a strip of 64 columns down the rows.
+//
+// Row t's state is loaded two rows ahead; its fluxes, its y terms and the limited x slopes of
+// row t-1 complete when it arrives, and row c = t-2 is advanced.  Between rows a wavefront
+// keeps rows c and c+1 (state, x fluxes, y terms), the slopes of row c and, of row c-1, what
+// row c's lower face needs; every slope is limited once.  Inner rows run one straight-line
+// body (walls only enter where an item starts, and in the two drain rows past the last one).
+// Bound: VALU issue, and on small domains the latency of an item's rows (default_rows2d in
+// shll_api.cpp).  Before, each row re-limited half of its x slopes and walked through some
+// thirty branch blocks and 100 register moves (REF32 MC: about 700 VALU instructions per row,
+// now about 500).  Measured, us per step before and now at the best item heights of each: REF32
+// MC 1024^2 28 and 19.6, 4096^2 273 and 191; FP64 minmod 777x613 25.3 and 15.1, 2048^2 118 and
+// 70 (268 MB read and written: 48% of the copy rate); C32K 1024^2 24.3 and 15.5.
+// ---------------------------------------------------------------------------
+template <int PREC>
+struct Row2 {
+    using RT = typename Real<PREC>::T;
+    RT u[4], l[4];          // state (C32: hi, lo)
+    RT xp[4], xm[4];        // x split fluxes
+    RT y1[4], y2[4];        // y terms (y_terms2)
+};
+
+// y terms of a row: reference forms y1 = hp - hm + T - B and y2 = the same of the slopes; C32
+// the lower and upper face terms, C32K their difference in y1
+template <int PREC, int LIM, bool YW, class A, class RT>
+__device__ __forceinline__ void y_terms2(const RT (&yp)[4], const RT (&ym)[4], const LaneWalls& w, RT lamy, RT th,
+                                         RT (&y1)[4], RT (&y2)[4]) {
+    constexpr bool CMP = PREC == PREC_C32 || PREC == PREC_C32K;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        const RT sy = (RT)sgn_y(v);
+        const RT hp = yp[v], hm = ym[v];
+        RT B = from_left_z(hp), T = from_right_z(hm);
+        RT dhp = limited_slope<A, LIM>(B, hp, from_right_z(hp), th);
+        RT dhm = limited_slope<A, LIM>(from_left_z(hm), hm, T, th);
+        if constexpr (YW) {
+            dhp = w.edge ? (RT)0 : dhp;
+            dhm = w.edge ? (RT)0 : dhm;
+        }
+        if constexpr (YW) B = w.lo ? (w.lo_refl ? sy * hm : hp) : B;
+        if constexpr (!CMP) {
+            if constexpr (YW) T = w.hi ? (w.hi_refl ? sy * hp : hm) : T;
+            y1[v] = hp - hm + T - B;
+            RT Bd = from_left_z(dhp), Td = from_right_z(dhm);
+            if constexpr (YW) {
+                Bd = w.lo ? (RT)0 : Bd;
+                Td = w.hi ? (RT)0 : Td;
+            }
+            y2[v] = dhp + dhm - Td - Bd;
+        } else {
+            RT d = from_left_z(dhp) - dhm;
+            if constexpr (YW) d = w.lo ? (RT)0 : d;
+            const RT tb = __builtin_fmaf((RT)0.5 * lamy, d, lamy * (B + hm));
+            RT tt = from_right_z(tb);
+            if constexpr (YW) tt = w.hi ? lamy * (hp + (w.hi_refl ? sy * hp : hm)) : tt;
+            if constexpr (PREC == PREC_C32K) {
+                y1[v] = tb - tt;
+                y2[v] = 0;
+            } else {
+                y1[v] = tb;
+                y2[v] = tt;
+            }
+        }
+    }
+}
+
+template <int PREC, int LIM, bool YW, bool SQ>
+__device__ __forceinline__ void rows2(const StepArgs& a, const Item2& it, const Inst& in, int lane) {
+    using RT = typename Real<PREC>::T;
+    constexpr bool CMP = PREC == PREC_C32 || PREC == PREC_C32K;
+    using A = typename std::conditional<CMP, C32Arith, RefArith<RT>>::type;
+    const int nx = in.nx, ny = in.ny;
+    const int64_t P = a.plane;
+    const int j = it.j0 + lane;
+    const int jc = j < 0 ? 0 : (j < ny ? j : ny - 1);  // lanes off the domain hold a copy of its edge
+    const bool jown = j >= it.jx0 && j < it.jx0 + it.jw;
+    const bool refl = in.bc == BC_REFLECT;
+    const LaneWalls w{j == 0, j == ny - 1, j == 0 && refl, j == ny - 1 && refl, refl, j <= 0 || j >= ny - 1};
+    const RT lamx = PREC == PREC_F64 ? (RT)in.k.d_lamx : (PREC == PREC_REF32 ? (RT)in.k.f_lamx : (RT)in.k.c_lamx);
+    const RT lamy = PREC == PREC_F64 ? (RT)in.k.d_lamy : (PREC == PREC_REF32 ? (RT)in.k.f_lamy : (RT)in.k.c_lamy);
+    const RT th = PREC == PREC_F64 ? (RT)in.k.d_theta : (PREC == PREC_REF32 ? (RT)in.k.f_theta : (RT)in.k.c_theta);
+    const RT hlx = (RT)0.5 * lamx;
+    const RT* __restrict__ p0 = (const RT*)a.in0 + in.off + jc;
+    const RT* __restrict__ p1 = CMP ? (const RT*)a.in1 + in.off + jc : nullptr;
+    RT* __restrict__ q0 = (RT*)a.out0 + in.off + jc;
+    RT* __restrict__ q1 = CMP ? (RT*)a.out1 + in.off + jc : nullptr;
+
+    auto load = [&](int t, Row2<PREC>& r) {
+        const int64_t o = (int64_t)(t < nx ? t : nx - 1) * ny;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            r.u[v] = p0[v * P + o];
+            if constexpr (CMP) r.l[v] = p1[v * P + o];
+        }
+    };
+    const int end = it.ix0 + it.iw;
+    // fluxes of row t, and the y terms of an owned row
+    auto take = [&](int t, Row2<PREC>& r) {
+        RT yp[4], ym[4];
+        fluxes2<PREC, RT>(r.u, in, r.xp, r.xm, yp, ym);
+        RT y1[4] = {0, 0, 0, 0}, y2[4] = {0, 0, 0, 0};
+        if (t >= it.ix0 && t < end) y_terms2<PREC, LIM, YW, A, RT>(yp, ym, w, lamy, th, y1, y2);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            r.y1[v] = y1[v];
+            r.y2[v] = y2[v];
+        }
+    };
+
+    // of row c-1 the upper-face parts (reference forms: F+ and its slope; C32: the face term);
+    // the slopes of row c
+    RT L[4], sPl[4], sP[4], sM[4];
+    // iteration t advances row c = t - 2 from rows c, c+1 and t (ra, rb, rn), whose arrival
+    // completes the slopes of row t-1; INNER false: t = nx, nx + 1, the last rows at the wall
+    auto advance = [&](int t, const Row2<PREC>& ra, const Row2<PREC>& rb, const Row2<PREC>& rn, auto inner) {
+        constexpr bool INNER = decltype(inner)::value;
+        const int c = t - 2;
+        RT nP[4], nM[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            nP[v] = INNER ? limited_slope<A, LIM>(ra.xp[v], rb.xp[v], rn.xp[v], th) : (RT)0;
+            nM[v] = INNER ? limited_slope<A, LIM>(ra.xm[v], rb.xm[v], rn.xm[v], th) : (RT)0;
+        }
+        const int64_t o = (int64_t)c * ny;
+        RT tr[4];
+        if constexpr (CMP) {
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                RT R = rb.xm[v];
+                if constexpr (!INNER) R = c == nx - 1 ? (refl ? (RT)sgn_x(v) * ra.xp[v] : ra.xm[v]) : R;
+                tr[v] = __builtin_fmaf(hlx, sP[v] - nM[v], lamx * (ra.xp[v] + R));
+            }
+        }
+        if (c >= it.ix0) {
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                if constexpr (!CMP) {
+                    using U = RefUpdate<RT>;
+                    RT R = rb.xm[v];
+                    if constexpr (!INNER) R = c == nx - 1 ? (refl ? (RT)sgn_x(v) * ra.xp[v] : ra.xm[v]) : R;
+                    RT uu = U::template first<true>(v == 2, ra.u[v], lamx, ra.xp[v] - ra.xm[v] + R - L[v]);
+                    uu = U::template second<true>(v == 2, uu, lamx, sP[v] + sM[v] - nM[v] - sPl[v]);
+                    uu = U::template first<SQ>(v == 1, uu, lamy, ra.y1[v]);
+                    uu = U::template second<SQ>(v == 1, uu, lamy, ra.y2[v]);
+                    if (jown) q0[v * P + o] = uu;
+                } else {
+                    RT hi = ra.u[v], lo = ra.l[v], e;
+                    if constexpr (PREC == PREC_C32K) {
+                        const RT y = ((L[v] - tr[v]) + ra.y1[v]) + lo;
+                        const RT s = hi + y;
+                        e = y - (s - hi);
+                        hi = s;
+                    } else {
+                        two_sum(hi, L[v], hi, e);
+                        lo = lo + e;
+                        two_sum(hi, -tr[v], hi, e);
+                        lo = lo + e;
+                        two_sum(hi, ra.y1[v], hi, e);
+                        lo = lo + e;
+                        two_sum(hi, -ra.y2[v], hi, e);
+                        lo = lo + e;
+                        fast_two_sum(hi, lo, hi, e);
+                    }
+                    if (jown) {
+                        q0[v * P + o] = hi;
+                        q1[v * P + o] = e;
+                    }
+                }
+            }
+        }
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            if constexpr (CMP) {
+                L[v] = tr[v];
+            } else {
+                L[v] = ra.xp[v];
+                sPl[v] = sP[v];
+            }
+            sP[v] = nP[v];
+            sM[v] = nM[v];
+        }
+    };
+    auto drain = [&](int t, const Row2<PREC>& ra, const Row2<PREC>& rb) {
+        if (t < end + 2) advance(t, ra, rb, rb, std::false_type{});
+        if (t + 1 < end + 2) advance(t + 1, rb, rb, rb, std::false_type{});
+    };
+    // four rows in rotation (so none is ever moved): c, c+1, t, and t+1 on its way from memory
+    Row2<PREC> r0, r1, r2, r3;
+    const int first = it.ix0 - 2 < 0 ? 0 : it.ix0 - 2;
+    load(first, r0);
+    load(first + 1, r1);
+    load(first + 2, r2);
+    take(first, r0);
+    take(first + 1, r1);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        // the first row's lower face: the wall (at a cut: spoils rows that are not stored)
+        const RT f = refl ? (RT)sgn_x(v) * r0.xm[v] : r0.xp[v];
+        L[v] = CMP ? lamx * (f + r0.xm[v]) : f;
+        sPl[v] = sP[v] = sM[v] = (RT)0;
+    }
+    int t = first + 2;
+    const int tin = end + 2 < nx ? end + 2 : nx;  // iterations below this take a row
+    // unrolled by four only where that keeps the wavefronts per SIMD: REF32 needs 152 registers
+    // unrolled (3 per SIMD) and 128 rolled, and ran 4% slower unrolled at 4096^2; FP64 ran 7%
+    // faster.  (Leaving the unrolled loop from its middle cost 100 registers.)
+    for (; PREC != PREC_REF32 && t + 4 <= tin; t += 4) {
+        load(t + 1, r3);
+        take(t, r2);
+        advance(t, r0, r1, r2, std::true_type{});
+        load(t + 2, r0);
+        take(t + 1, r3);
+        advance(t + 1, r1, r2, r3, std::true_type{});
+        load(t + 3, r1);
+        take(t + 2, r0);
+        advance(t + 2, r2, r3, r0, std::true_type{});
+        load(t + 4, r2);
+        take(t + 3, r1);
+        advance(t + 3, r3, r0, r1, std::true_type{});
+    }
+    for (; t < tin; ++t) {
+        load(t + 1, r3);
+        take(t, r2);
+        advance(t, r0, r1, r2, std::true_type{});
+        r0 = r1;
+        r1 = r2;
+        r2 = r3;
+    }
+    drain(t, r0, r1);
+}
+
+template <int PREC, int WPB, int LIM>
+__global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(PREC == PREC_F64 ? 2 : 1)))
+void k_row2d(StepArgs a) {
+    const LaunchView lv = launch_view(a);
+    const int blk = xcd_work((int)blockIdx.x, (lv.n_items + WPB - 1) / WPB);
+    const int wave = blk * WPB + uniform((int)threadIdx.x >> 6);
+    if (blk < 0 || wave >= lv.n_items) return;
+    const int lane = (int)threadIdx.x & 63;
+    const Item2 it = ((const Item2*)a.items)[wave];
+    const Inst in = a.inst[it.inst];
+    if (in.nsteps - lv.step_base <= 0) return;
+    // strips away from both y walls take the copy without wall choices, square cells the one
+    // with DT/DY = 1/8
+    const bool yw = it.j0 <= 0 || it.j0 + 64 >= in.ny;
+    if constexpr (PREC == PREC_F64 || PREC == PREC_REF32) {
+        const bool sq = PREC == PREC_F64 ? in.k.d_lamy == 0.125 : in.k.f_lamy == 0.125f;
+        if (yw) {
+            if (sq) rows2<PREC, LIM, true, true>(a, it, in, lane);
+            else rows2<PREC, LIM, true, false>(a, it, in, lane);
+        } else {
+            if (sq) rows2<PREC, LIM, false, true>(a, it, in, lane);
+            else rows2<PREC, LIM, false, false>(a, it, in, lane);
+        }
+    } else {
+        if (yw) rows2<PREC, LIM, true, false>(a, it, in, lane);
+        else rows2<PREC, LIM, false, false>(a, it, in, lane);
+    }
+}
+
+template <int PREC, int WPB>
 __global__ __launch_bounds__(64 * WPB) void k_step2d(StepArgs a) {
+    constexpr int ORDER = 1, LIM = LIM_MINMOD;
     using RT = typename Real<PREC>::T;
     using A = typename std::conditional<PREC == PREC_C32 || PREC == PREC_C32K, C32Arith, RefArith<RT>>::type;
     constexpr int NW = 2 * ORDER + 1;  // rows of x fluxes kept: c-ORDER .. c+ORDER
@@ -238,12 +507,6 @@ struct Held2 {
                       // F64/REF32: yb = (hp - hm) + T - B
 };
 
-// A lane's y walls, as per-lane flags (lane-varying, so the wall choices are selects
-// rather than branches): lo / hi = the lane is column 0 / ny-1, *_refl = and reflective
-struct LaneWalls {
-    bool lo, hi, lo_refl, hi_refl, refl;
-};
-
 enum { ST_TAKE_FIRST = 0, ST_TAKE = 1, ST_DRAIN = 2 };
 
 // One stage, one row.  io: the incoming row (ST_TAKE_FIRST / ST_TAKE); on return the
@@ -364,7 +627,7 @@ __device__ __forceinline__ void pipeline2(const StepArgs& a, const Item2& it, co
     const RT lamx = PREC == PREC_F64 ? (RT)in.k.d_lamx : (PREC == PREC_REF32 ? (RT)in.k.f_lamx : (RT)in.k.c_lamx);
     const RT lamy = PREC == PREC_F64 ? (RT)in.k.d_lamy : (PREC == PREC_REF32 ? (RT)in.k.f_lamy : (RT)in.k.c_lamy);
     const bool refl = in.bc == BC_REFLECT;
-    const LaneWalls w{j == 0, j == ny - 1, j == 0 && refl, j == ny - 1 && refl, refl};
+    const LaneWalls w{j == 0, j == ny - 1, j == 0 && refl, j == ny - 1 && refl, refl, j <= 0 || j >= ny - 1};
 
     // rows taken by every stage: [r0, r1), then a drain
     const int r0 = it.ix0 - K < 0 ? 0 : it.ix0 - K;
@@ -660,7 +923,7 @@ __device__ __forceinline__ void pipeline2o2(const StepArgs& a, const Item2& it, 
     float* __restrict__ o1p = (float*)a.out1 + in.off;
     const float lamx = in.k.c_lamx, lamy = in.k.c_lamy, th = in.k.c_theta;
     const bool refl = in.bc == BC_REFLECT;
-    const LaneWalls w{j == 0, j == ny - 1, j == 0 && refl, j == ny - 1 && refl, refl};
+    const LaneWalls w{j == 0, j == ny - 1, j == 0 && refl, j == ny - 1 && refl, refl, j <= 0 || j >= ny - 1};
     const bool yedge = j <= 0 || j >= ny - 1;  // zero y slopes (2nd_order_base_shll.c:293-344)
 
     constexpr int H = 2 * K;
@@ -806,21 +1069,19 @@ static hipError_t launch2_tb(int k, int wpb, int nblocks, hipStream_t s, const S
     return wpb == 1 ? launch2_tb_w<PREC, 1>(k, nblocks, s, a) : launch2_tb_w<PREC, 4>(k, nblocks, s, a);
 }
 
-template <int PREC, int ORDER, int LIM>
-static hipError_t launch2_o(int wpb, int nblocks, hipStream_t s, const StepArgs& a) {
-    if (wpb == 1) hipLaunchKernelGGL((k_step2d<PREC, ORDER, 1, LIM>), dim3(nblocks), dim3(64), 0, s, a);
-    else hipLaunchKernelGGL((k_step2d<PREC, ORDER, 4, LIM>), dim3(nblocks), dim3(256), 0, s, a);
+template <int PREC, int WPB>
+static hipError_t launch2_w(int order, int lim, int nblocks, hipStream_t s, const StepArgs& a) {
+    const dim3 grid(nblocks), block(64 * WPB);
+    if (order == 1 && lim == LIM_MINMOD) hipLaunchKernelGGL((k_step2d<PREC, WPB>), grid, block, 0, s, a);
+    else if (order == 2 && lim == LIM_MINMOD) hipLaunchKernelGGL((k_row2d<PREC, WPB, LIM_MINMOD>), grid, block, 0, s, a);
+    else if (order == 2 && lim == LIM_MC) hipLaunchKernelGGL((k_row2d<PREC, WPB, LIM_MC>), grid, block, 0, s, a);
+    else return hipErrorInvalidValue;
     return hipGetLastError();
 }
 
-// first order; second order with minmod; second order with the MC limiter
 template <int PREC>
 static hipError_t launch2_p(int order, int lim, int wpb, int nblocks, hipStream_t s, const StepArgs& a) {
-    if (order == 1) return lim == LIM_MINMOD ? launch2_o<PREC, 1, LIM_MINMOD>(wpb, nblocks, s, a) : hipErrorInvalidValue;
-    if (order != 2) return hipErrorInvalidValue;
-    if (lim == LIM_MINMOD) return launch2_o<PREC, 2, LIM_MINMOD>(wpb, nblocks, s, a);
-    if (lim == LIM_MC) return launch2_o<PREC, 2, LIM_MC>(wpb, nblocks, s, a);
-    return hipErrorInvalidValue;
+    return wpb == 1 ? launch2_w<PREC, 1>(order, lim, nblocks, s, a) : launch2_w<PREC, 4>(order, lim, nblocks, s, a);
 }
 
 bool step2d_supported(int prec, int order, int k) {

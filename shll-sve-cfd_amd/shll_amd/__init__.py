@@ -291,7 +291,7 @@ class Solver:
 
     def set_launch(self, cells_per_lane=None, steps_per_launch=8, waves_per_block=4, graph_steps=128):
         """cells_per_lane: 1D cells per lane (default 2); 2D owned rows per work item (default 1:
-        16, 32 or 64 rows for 1, 2 or more steps per launch)."""
+        the library's choice by steps per launch and size)."""
         if cells_per_lane is None:
             cells_per_lane = 2 if self.pb.dim == 1 else 1
         _check(lib().shll_set_launch(self.h, cells_per_lane, steps_per_launch, waves_per_block, graph_steps))
