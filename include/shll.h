@@ -175,9 +175,10 @@ void shll_free(shll_ctx *ctx);
 
 /* Launch shape of the step kernels.  cells_per_lane: 1D in {1,2,4,8}; 2D the owned rows
  * of a work item, the cells of its column each lane owns (2-4096; 0 or 1: the library's
- * choice, 32 or 64 rows for 2 or more steps per launch, and for 1 step 16 or, in second
- * order, 2-16 by the size of the domain), steps_per_launch >= 1 (temporal blocking; 2D:
- * 1, 2, 3, 4 or 8 in first order; 1, or 2 for SHLL_C32/SHLL_C32K in second order),
+ * choice; first-order items are register tiles of the library's height whatever is asked
+ * for, except in SHLL_F64 at 1 or 2 steps per launch on more than about 4e6 cells),
+ * steps_per_launch >= 1 (temporal blocking; 2D: 1, 2, 3, 4 or 8 in first order; 1, or 2 for
+ * SHLL_C32/SHLL_C32K in second order),
  * waves_per_block in {1,4} (1D, 4 with 2+ cells per lane: the block's wavefronts hold
  * one segment and share their edge fluxes), graph_steps: steps captured per HIP graph
  * (0 = no graph; at most 4096 launches per graph; a single instance's graphs are captured

@@ -26,6 +26,8 @@ int step1d_items_per_block(int C, int wpb);
 hipError_t launch_step2d(int prec, int order, int lim, int k, int wpb, int n_items, hipStream_t s,
                          const StepArgs& a);
 bool step2d_supported(int prec, int order, int k);
+int tile2d_rows(int prec, int k, int64_t (*tiles)(const void*, int), const void* arg);
+hipError_t launch_tile2d(int prec, int rows, int n_items, hipStream_t s, const StepArgs& a);
 hipError_t launch_init(int prec, int dim, int nblocks, int n_inst, hipStream_t st, const Inst* insts,
                        const double* prim, void* o0, void* o1, int64_t plane);
 hipError_t launch_stage(int prec, int dim, int nblocks, hipStream_t st, const Inst* inst, const void* s0,
@@ -262,6 +264,7 @@ struct Engine {
     std::vector<int64_t> inst_cells;   // cells per instance
     std::vector<int64_t> order_idx;    // instances sorted by nsteps descending
     Launch L;
+    int tile = 0;       // 2D first order: rows of the register tiles (0: the row kernels)
     // work list for the current launch shape (instances in order_idx order)
     void* d_items = nullptr;
     size_t d_items_cap = 0;
@@ -351,6 +354,23 @@ static int default_rows2d(const Engine* E, int k) {
     return best;
 }
 
+// 2D first order: rows of the register tiles, 0 for the row pipelines, which FP64 keeps at 1 and
+// 2 steps per launch on domains whose two state buffers exceed the last-level cache (4096^2, us
+// per step at k = 2: pipeline 172, tiles 192; 2048^2, in the cache: 58 and 51).  An item is one
+// tile, whatever rows the launch shape asks for.
+static bool in_cache(const Engine* E) {
+    int64_t cells = 0;
+    for (int64_t c : E->inst_cells) cells += c;
+    return cells * 2 * E->nv * (int64_t)(word_bytes(E->prec) * nwords(E->prec)) <= (256LL << 20);
+}
+static int pick_tile2d(const Engine* E) {
+    if (E->dim != 2 || E->order != 1) return 0;
+    if (E->prec == SHLL_F64 && E->L.k <= 2 && !in_cache(E)) return 0;
+    return tile2d_rows(
+        E->prec, E->L.k,
+        [](const void* e, int rows) { return items2d((const Engine*)e, ((const Engine*)e)->L.k, rows); }, E);
+}
+
 static void engine_drop_graphs(Engine* E) {
     for (int p = 0; p < 2; ++p)
         if (E->gexec[p]) {
@@ -403,6 +423,7 @@ static shll_status engine_build_items(Engine* E) {
     engine_drop_graphs(E);
     std::vector<Item1> it1;
     std::vector<Item2> it2;
+    E->tile = pick_tile2d(E);
     E->inst_first_item.assign(E->order_idx.size() + 1, 0);
     for (size_t r = 0; r < E->order_idx.size(); ++r) {
         const int64_t i = E->order_idx[r];
@@ -414,7 +435,7 @@ static shll_status engine_build_items(Engine* E) {
                 return fail(SHLL_EINVAL, "launch shape C=%d k=%d leaves no owned cells (order %d)", E->L.C, E->L.k,
                             E->order);
         } else {
-            tile2d((int32_t)i, in.nx, in.ny, E->order, E->L.k, E->L.rows, it2);
+            tile2d((int32_t)i, in.nx, in.ny, E->order, E->L.k, E->tile ? E->tile - 2 * E->L.k : E->L.rows, it2);
         }
     }
     E->inst_first_item[E->order_idx.size()] = E->dim == 1 ? (int64_t)it1.size() : (int64_t)it2.size();
@@ -484,11 +505,13 @@ static StepArgs make_args(const Engine* E, int64_t step_base, int parity, int64_
 
 // work items per block of a launch
 static int items_per_block(const Engine* E) {
+    if (E->tile) return 1;
     return E->dim == 1 ? step1d_items_per_block(E->L.C, E->L.wpb) : E->L.wpb;
 }
 
 static hipError_t launch_one(const Engine* E, const StepArgs& a, int64_t n_items) {
     if (E->dim == 1) return launch_step1d(E->prec, E->order, E->lim, E->L.C, E->L.wpb, (int)n_items, E->stream, a);
+    if (E->tile) return launch_tile2d(E->prec, E->tile, (int)n_items, E->stream, a);
     return launch_step2d(E->prec, E->order, E->lim, E->L.k, E->L.wpb, (int)n_items, E->stream, a);
 }
 
@@ -841,19 +864,22 @@ static shll_status engine_create_stream(Engine* E) {
 
 static void default_launch(Engine* E, int64_t max_cells) {
     if (E->dim == 2) {
-        // First order: several steps per launch (row-pipelined stages); measured on a
-        // 4096^2 domain and a 64-domain batch, the FP32 forms peak at 4 steps per launch,
-        // FP64 (twice the registers per stage) at 2.  Second order: one step per launch, but
-        // C32K takes two on domains whose two state buffers exceed the 256 MiB last-level
-        // cache, where one step is bound by HBM (us per step, 1 and 2 steps per launch: 1024^2
-        // 16.4 and 32.2, 2048^2 55 and 58, 3072^2 163 and 108); the TwoSum form's two-row
-        // stages overflow the registers (3072^2 162 and 183).
+        // First order: the compensated forms take 4 steps per launch; F64 and REF32 4 on small
+        // domains, where a launch costs as much as its steps, and 2 (F64 in between 3) on large
+        // ones, whose halo costs more than the traffic it saves.  Measured, us per step at 2, 3
+        // and 4: REF32 256^2 2.6, 2.2, 1.9, 400^2 2.8, 3.0, 2.8, 800^2 5.6, 5.7, -; F64 300^2
+        // 3.5, 2.9, 2.7, 500^2 4.5, 3.9, 5.7, 1024^2 13.8, 13.4, -, 1531x2049 38, 39, 41.
+        // Second order: one step per launch, but C32K takes two on domains whose state exceeds
+        // the last-level cache, where one step is bound by HBM (us per step, 1 and 2 steps per
+        // launch: 1024^2 16.4 and 32.2, 2048^2 55 and 58, 3072^2 163 and 108); the TwoSum form's
+        // two-row stages overflow the registers (3072^2 162 and 183).
         int64_t cells = 0;
         for (int64_t c : E->inst_cells) cells += c;
-        const bool in_cache = cells * 64 <= (256LL << 20);
+        const bool comp = E->prec == SHLL_C32 || E->prec == SHLL_C32K;
         E->L.C = 1;
-        E->L.k = E->order == 1 ? (E->prec == PREC_C32 || E->prec == PREC_C32K ? 4 : 2)
-                               : (E->prec == PREC_C32K && !in_cache ? 2 : 1);
+        if (E->order == 2) E->L.k = E->prec == SHLL_C32K && !in_cache(E) ? 2 : 1;
+        else if (comp || cells < 150000) E->L.k = 4;
+        else E->L.k = E->prec == SHLL_F64 && cells < 1500000 ? 3 : 2;
         E->L.wpb = 4;
         E->L.rows = default_rows2d(E, E->L.k);
         E->L.graph = 64;
@@ -1353,8 +1379,9 @@ static shll_status engine_autotune(Engine* E, int32_t trial_steps, int64_t shape
                 // SIMD: each wavefront walks its rows one after another, so a launch of few
                 // items is latency-bound, and more items trade halo rows for parallelism
                 const int rd = rows2d(k);
-                std::vector<int> rows = {1, rd * 3 / 4, rd * 5 / 4, rd * 3 / 2};
-                if (items2d(E, k, rd) < 4 * simd_count(E))
+                std::vector<int> rows = {1};
+                if (E->order == 2 || E->prec == SHLL_F64) rows = {1, rd * 3 / 4, rd * 5 / 4, rd * 3 / 2};
+                if (E->order == 2 && items2d(E, k, rd) < 4 * simd_count(E))
                     for (int r : {rd / 2, rd * 3 / 8, rd / 4, rd * 3 / 16, rd / 8})
                         if (r >= 2) rows.push_back(r);
                 std::vector<int> graphs = {std::max(64, 2 * k)};

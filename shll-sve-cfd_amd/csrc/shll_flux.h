@@ -180,7 +180,7 @@ __device__ __forceinline__ void fluxes2(const RT (&U)[4], const Inst& in, RT (&x
         split_c32(vy * (U[3] + P), U[3], z1, z2, z3, yp[3], ym[3]);
     } else {
         Prim2<RT> q;
-        if (!ref_prim2<RT>(U, in, q)) ref_prim2_exact<RT>(U, in, q);
+        if (__builtin_expect(!ref_prim2<RT>(U, in, q), 0)) ref_prim2_exact<RT>(U, in, q);
         ref_flux2<RT>(U, q, xp, xm, yp, ym);
         a = q.a;
     }

@@ -1,4 +1,4 @@
-// shll_k2t.hip -- 2D SHLL step kernel on register tiles (first and second order) for gfx950.
+// shll_k2t.hip -- 2D first-order SHLL step kernel on register tiles for gfx950.
 //
 // A block of W wavefronts holds a tile of W*RW rows by 64 columns in registers: wavefront w
 // has RW consecutive rows, lane = column.  A step is
@@ -6,14 +6,21 @@
 //   the y terms of each row, from the adjacent lanes (DPP wave shifts),
 //   one exchange of the edge rows' x fluxes with the wavefronts above and below (LDS, one
 //   barrier, double-buffered by step parity),
-//   limited x slopes (second order) and the conservative update, all in registers,
-// so a launch of k steps reads the state once and writes it once; the outer order*k rows and
-// columns of a tile are recomputed halo.  The RW rows of a wavefront are independent chains,
-// where a wavefront that walks down its rows one after another (the row pipelines of
-// shll_k2d.hip) has only one.
+//   the conservative update, all in registers,
+// so a launch of k steps reads the state once and writes it once; the outer k rows and columns
+// of a tile are recomputed halo.  Bound: VALU issue and latency on small domains, HBM traffic
+// (halo included) together with the blocks a CU holds on large ones.
 //
-// Layout, update order, walls and limiters as in shll_k2d.hip (base_shll_2d.c:139-319,
-// 2nd_order_base_shll.c:203-541, base-omp/2nd_order_base_shll.c:317-325,385-392).
+// Why tiles: a wavefront that walks down its rows (the pipelines of shll_k2d.hip) has one serial
+// chain of k stages per row and few wavefronts on a small domain; the RW rows of a tile's
+// wavefront are independent chains, and a domain gives a wavefront per RW rows and strip.
+// Measured, us per step before (row pipelines, their default items) and now: REF32 128^2 27 and
+// 1.9, 2048^2 45 and 26; FP64 700^2 32 and 7.1, 1531x2049 45 and 38; C32K 600^2 28 and 4.6,
+// 1500^2 29 and 13, 4096^2 104 and 74; C32 4096^2 151 and 112.  A pipeline of k wavefronts that
+// hand rows on through LDS (one stage each, a barrier per row) was slower: C32K 4096^2 107,
+// FP64 1531x2049 48.
+//
+// Layout, update order and walls as in shll_k2d.hip (base_shll_2d.c:139-319).
 #include "shll_flux.h"
 
 namespace shll {
@@ -24,78 +31,42 @@ __device__ __forceinline__ RT wall_x(int v, RT f) { return v == 1 ? f : -f; }
 template <class RT>
 __device__ __forceinline__ RT wall_y(int v, RT f) { return v == 2 ? f : -f; }
 
-// Edge rows' x fluxes in LDS, per buffer, wavefront and slot: 4 variables x 64 lanes.
-// Slots for the wavefront below: F- of the first row (second order: and of the second, and F+
-// of the first); for the one above: F+ of the last row (and of the last but one, and F- of the
-// last).  First order double-buffers them by step parity, one barrier per step; second order,
-// with three times the slots, keeps one buffer and takes a second barrier before it is
-// written again.
-template <int ORDER>
-struct TileSlots {
-    static constexpr int SIDE = ORDER == 1 ? 1 : 3, N = 2 * SIDE, NBUF = ORDER == 1 ? 2 : 1;
-};
-
-template <int PREC, int ORDER, int LIM, int RW, int W, bool EDGE, bool SQ>
+// One wavefront's rows.  EDGE: the tile touches a wall; SQ: DT/DY = 1/8 (reference forms).
+template <int PREC, int RW, int W, bool EDGE, bool SQ>
 struct Tile2 {
     using RT = typename Real<PREC>::T;
     static constexpr bool CMP = PREC == PREC_C32 || PREC == PREC_C32K;  // (hi, lo) state
     static constexpr bool KAHAN = PREC == PREC_C32K;
-    using A = typename std::conditional<CMP, C32Arith, RefArith<RT>>::type;
-    using Up = RefUpdate<RT>;
-    static constexpr int SIDE = TileSlots<ORDER>::SIDE, SLOTS = TileSlots<ORDER>::N;
 
     const Inst& in;
-    RT* lds;        // [NBUF][W][SLOTS][4][64]
+    RT* lds;        // [2 parity][W][2: F- of the first row, F+ of the last][4][64]
     int wib, lane;  // wavefront in block
-    int g0, j;      // the wavefront's first row, the lane's column
+    int g0;         // the wavefront's first row
     bool jlo, jhi, refl;
-    RT lamy, hlamx, hlamy, lamx, th;
+    RT lamx, lamy;
 
     RT u[RW][4], l[CMP ? RW : 1][4];
     RT xp[RW][4], xm[RW][4];
-    // y terms: reference forms Y1 = hp - hm + T - B and Y2 = the same of the slopes; C32 the
-    // lower and upper face terms, C32K their difference in Y1
-    RT Y1[RW][4], Y2[ORDER == 2 || PREC == PREC_C32 ? RW : 1][4];
+    // y terms: reference forms Y1 = hp - hm + T - B; C32 the lower and upper face terms, C32K
+    // their difference in Y1
+    RT Y1[RW][4], Y2[PREC == PREC_C32 ? RW : 1][4];
 
     __device__ __forceinline__ RT* slot(int parity, int w, int s, int v) const {
-        const int b = TileSlots<ORDER>::NBUF == 2 ? parity : 0;
-        return lds + (((b * W + w) * SLOTS + s) * 4 + v) * 64 + lane;
+        return lds + (((parity * W + w) * 2 + s) * 4 + v) * 64 + lane;
     }
 
-    // F and the y terms of row r
     __device__ __forceinline__ void y_terms(int r, const RT (&yp)[4], const RT (&ym)[4]) {
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             const RT hp = yp[v], hm = ym[v];
-            RT B = from_left_z(hp), dhp = 0, dhm = 0;
-            if constexpr (ORDER == 2) {
-                dhp = limited_slope<A, LIM>(B, hp, from_right_z(hp), th);
-                dhm = limited_slope<A, LIM>(from_left_z(hm), hm, from_right_z(hm), th);
-                if constexpr (EDGE) {
-                    dhp = jlo || jhi ? (RT)0 : dhp;
-                    dhm = jlo || jhi ? (RT)0 : dhm;
-                }
-            }
+            RT B = from_left_z(hp);
             if constexpr (EDGE) B = jlo ? (refl ? wall_y(v, hm) : hp) : B;
             if constexpr (!CMP) {
                 RT T = from_right_z(hm);
                 if constexpr (EDGE) T = jhi ? (refl ? wall_y(v, hp) : hm) : T;
                 Y1[r][v] = hp - hm + T - B;
-                if constexpr (ORDER == 2) {
-                    RT Bd = from_left_z(dhp), Td = from_right_z(dhm);
-                    if constexpr (EDGE) {
-                        Bd = jlo ? (RT)0 : Bd;
-                        Td = jhi ? (RT)0 : Td;
-                    }
-                    Y2[r][v] = dhp + dhm - Td - Bd;
-                }
             } else {
-                RT tb = lamy * (B + hm);
-                if constexpr (ORDER == 2) {
-                    RT d = from_left_z(dhp) - dhm;
-                    if constexpr (EDGE) d = jlo ? (RT)0 : d;
-                    tb = __builtin_fmaf(hlamy, d, tb);
-                }
+                const RT tb = lamy * (B + hm);
                 RT tt = from_right_z(tb);
                 if constexpr (EDGE) tt = jhi ? lamy * (hp + (refl ? wall_y(v, hp) : hm)) : tt;
                 if constexpr (KAHAN) {
@@ -118,7 +89,7 @@ struct Tile2 {
             }
         } else {
             // primitives of all rows, then one branch for the lanes with a cell outside the
-            // fast form's range
+            // fast form's range, so the rows' dependent chains overlap
             Prim2<RT> q[RW];
             bool ok = true;
 #pragma unroll
@@ -136,71 +107,30 @@ struct Tile2 {
         }
     }
 
-    // limited slope of row g from its three values; zero on the domain's first and last rows
-    __device__ __forceinline__ RT xslope(RT a, RT b, RT c, int g) const {
-        RT s = limited_slope<A, LIM>(a, b, c, th);
-        if constexpr (EDGE) s = g <= 0 || g >= in.nx - 1 ? (RT)0 : s;
-        return s;
-    }
-
-    // the conservative update of all rows, variable by variable
-    __device__ __forceinline__ void update(int parity, bool again) {
-        if constexpr (TileSlots<ORDER>::NBUF == 1) {
-            if (again) __syncthreads();  // every wavefront has read the last step's rows
-        }
-        // publish the edge rows, wait, read the neighbours'; the block's end wavefronts read
-        // their own rows for the missing ones (halo)
+    // publish the edge rows, wait, read the neighbours', update all rows; the block's end
+    // wavefronts read their own rows for the missing ones (halo)
+    __device__ __forceinline__ void update(int parity) {
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             *slot(parity, wib, 0, v) = xm[0][v];
-            *slot(parity, wib, SIDE, v) = xp[RW - 1][v];
-            if constexpr (ORDER == 2) {
-                *slot(parity, wib, 1, v) = xm[1][v];
-                *slot(parity, wib, 2, v) = xp[0][v];
-                *slot(parity, wib, SIDE + 1, v) = xp[RW - 2][v];
-                *slot(parity, wib, SIDE + 2, v) = xm[RW - 1][v];
-            }
+            *slot(parity, wib, 1, v) = xp[RW - 1][v];
         }
         __syncthreads();
         const int wb = wib > 0 ? wib - 1 : 0, wa = wib + 1 < W ? wib + 1 : W - 1;
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            // window rows -1 .. RW (second order: F+ also at -2, F- at RW+1), index r + 2
-            RT P[RW + 4], M[RW + 4];
-#pragma unroll
-            for (int r = 0; r < RW; ++r) {
-                P[r + 2] = xp[r][v];
-                M[r + 2] = xm[r][v];
-            }
-            P[0] = P[RW + 2] = P[RW + 3] = M[0] = M[1] = M[RW + 3] = (RT)0;
-            P[1] = *slot(parity, wb, SIDE, v);
-            M[RW + 2] = *slot(parity, wa, 0, v);
-            RT sP[RW + 1], sM[RW + 1];  // sP[f] = F+ slope of row f-1, sM[f] = F- slope of row f
-            if constexpr (ORDER == 2) {
-                P[0] = *slot(parity, wb, SIDE + 1, v);
-                M[1] = *slot(parity, wb, SIDE + 2, v);
-                M[RW + 3] = *slot(parity, wa, 1, v);
-                P[RW + 2] = *slot(parity, wa, 2, v);
-#pragma unroll
-                for (int f = 0; f <= RW; ++f) {
-                    sP[f] = xslope(P[f], P[f + 1], P[f + 2], g0 + f - 1);
-                    sM[f] = xslope(M[f + 1], M[f + 2], M[f + 3], g0 + f);
-                }
-            }
+            const RT below = *slot(parity, wb, 1, v), above = *slot(parity, wa, 0, v);
             if constexpr (CMP) {
                 RT t[RW + 1];  // face terms between rows f-1 and f
 #pragma unroll
                 for (int f = 0; f <= RW; ++f) {
-                    RT L = P[f + 1], R = M[f + 2];
+                    RT L = f > 0 ? xp[f > 0 ? f - 1 : 0][v] : below;
+                    RT R = f < RW ? xm[f < RW ? f : 0][v] : above;
                     if constexpr (EDGE) {
-                        const int g = g0 + f;
-                        L = g == 0 ? (refl ? wall_x(v, R) : P[f + 2]) : L;
-                        R = g == in.nx ? (refl ? wall_x(v, L) : M[f + 1]) : R;
+                        if (f < RW) L = g0 + f == 0 ? (refl ? wall_x(v, R) : xp[f < RW ? f : 0][v]) : L;
+                        if (f > 0) R = g0 + f == in.nx ? (refl ? wall_x(v, L) : xm[f > 0 ? f - 1 : 0][v]) : R;
                     }
                     t[f] = lamx * (L + R);
-                    if constexpr (ORDER == 2) {
-                        t[f] = __builtin_fmaf(hlamx, sP[f] - sM[f], t[f]);
-                    }
                 }
 #pragma unroll
                 for (int r = 0; r < RW; ++r) {
@@ -226,28 +156,26 @@ struct Tile2 {
             } else {
 #pragma unroll
                 for (int r = 0; r < RW; ++r) {
-                    RT L = P[r + 1], R = M[r + 3];
+                    RT L = r > 0 ? xp[r > 0 ? r - 1 : 0][v] : below;
+                    RT R = r + 1 < RW ? xm[r + 1 < RW ? r + 1 : 0][v] : above;
                     if constexpr (EDGE) {
                         L = g0 + r == 0 ? (refl ? wall_x(v, xm[r][v]) : xp[r][v]) : L;
                         R = g0 + r == in.nx - 1 ? (refl ? wall_x(v, xp[r][v]) : xm[r][v]) : R;
                     }
-                    RT uu = Up::template first<true>(v == 2, u[r][v], lamx, xp[r][v] - xm[r][v] + R - L);
-                    if constexpr (ORDER == 2)
-                        uu = Up::template second<true>(v == 2, uu, lamx, sP[r + 1] + sM[r] - sM[r + 1] - sP[r]);
-                    uu = Up::template first<SQ>(v == 1, uu, lamy, Y1[r][v]);
-                    if constexpr (ORDER == 2) uu = Up::template second<SQ>(v == 1, uu, lamy, Y2[r][v]);
-                    u[r][v] = uu;
+                    using U = RefUpdate<RT>;
+                    const RT uu = U::template first<true>(v == 2, u[r][v], lamx, xp[r][v] - xm[r][v] + R - L);
+                    u[r][v] = U::template first<SQ>(v == 1, uu, lamy, Y1[r][v]);
                 }
             }
         }
     }
 };
 
-// One item: its owned rows in tiles of at most W*RW rows
-template <int PREC, int ORDER, int LIM, int RW, int W, bool EDGE, bool SQ>
-__device__ __forceinline__ void tile_steps(const StepArgs& a, const Item2& it, const Inst& in, int i0, int ns, int x0,
-                                           int x1, typename Real<PREC>::T* lds, int& parity) {  // parity: steps this block has taken
-    using T = Tile2<PREC, ORDER, LIM, RW, W, EDGE, SQ>;
+// ns steps of rows [i0, i0 + W*RW), of which the item's are stored
+template <int PREC, int RW, int W, bool EDGE, bool SQ>
+__device__ __forceinline__ void tile_steps(const StepArgs& a, const Item2& it, const Inst& in, int i0, int ns,
+                                           typename Real<PREC>::T* lds) {
+    using T = Tile2<PREC, RW, W, EDGE, SQ>;
     using RT = typename T::RT;
     constexpr bool CMP = T::CMP;
     const int wib = uniform((int)threadIdx.x >> 6), lane = (int)threadIdx.x & 63;
@@ -255,22 +183,15 @@ __device__ __forceinline__ void tile_steps(const StepArgs& a, const Item2& it, c
     const int jc = j < 0 ? 0 : (j < ny ? j : ny - 1);
     const int64_t P = a.plane;
     const int g0 = i0 + wib * RW;
-    T t{in, lds, wib, lane, g0, j, j <= 0, j >= ny - 1, in.bc == BC_REFLECT};
-    if constexpr (CMP) {
-        t.lamx = in.k.c_lamx; t.lamy = in.k.c_lamy; t.th = in.k.c_theta;
-    } else if constexpr (PREC == PREC_F64) {
-        t.lamx = in.k.d_lamx; t.lamy = in.k.d_lamy; t.th = in.k.d_theta;
-    } else {
-        t.lamx = in.k.f_lamx; t.lamy = in.k.f_lamy; t.th = in.k.f_theta;
-    }
-    t.hlamx = (RT)0.5 * t.lamx;
-    t.hlamy = (RT)0.5 * t.lamy;
+    T t{in, lds, wib, lane, g0, j <= 0, j >= ny - 1, in.bc == BC_REFLECT};
+    t.lamx = PREC == PREC_F64 ? (RT)in.k.d_lamx : (PREC == PREC_REF32 ? (RT)in.k.f_lamx : (RT)in.k.c_lamx);
+    t.lamy = PREC == PREC_F64 ? (RT)in.k.d_lamy : (PREC == PREC_REF32 ? (RT)in.k.f_lamy : (RT)in.k.c_lamy);
     // rows and columns off the domain hold copies of its edge
     const RT* __restrict__ p0 = (const RT*)a.in0 + in.off;
     const RT* __restrict__ p1 = CMP ? (const RT*)a.in1 + in.off : nullptr;
 #pragma unroll
     for (int r = 0; r < RW; ++r) {
-        const int g = g0 + r < 0 ? 0 : (g0 + r < nx ? g0 + r : nx - 1);
+        const int g = g0 + r < nx ? g0 + r : nx - 1;
         const int64_t o = (int64_t)g * ny + jc;
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
@@ -280,8 +201,7 @@ __device__ __forceinline__ void tile_steps(const StepArgs& a, const Item2& it, c
     }
     for (int s = 0; s < ns; ++s) {
         t.fluxes();
-        t.update(parity & 1, parity > 0);
-        ++parity;
+        t.update(s & 1);
     }
     RT* __restrict__ o0 = (RT*)a.out0 + in.off;
     RT* __restrict__ o1 = CMP ? (RT*)a.out1 + in.off : nullptr;
@@ -289,7 +209,7 @@ __device__ __forceinline__ void tile_steps(const StepArgs& a, const Item2& it, c
 #pragma unroll
     for (int r = 0; r < RW; ++r) {
         const int g = g0 + r;
-        if (g >= x0 && g < x1 && jown) {
+        if (g >= it.ix0 && g < it.ix0 + it.iw && jown) {
             const int64_t o = (int64_t)g * ny + j;
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
@@ -300,15 +220,10 @@ __device__ __forceinline__ void tile_steps(const StepArgs& a, const Item2& it, c
     }
 }
 
-#ifndef T_EU32
-#define T_EU32 1
-#define T_EU64 1
-#endif
-template <int PREC, int ORDER, int LIM, int RW, int W>
-__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(PREC == PREC_F64 ? T_EU64 : T_EU32)))
-void k_tile2d(StepArgs a) {
+template <int PREC, int RW, int W>
+__global__ __launch_bounds__(64 * W) void k_tile2d(StepArgs a) {
     using RT = typename Real<PREC>::T;
-    __shared__ RT lds[TileSlots<ORDER>::NBUF * W * TileSlots<ORDER>::N * 4 * 64];
+    __shared__ RT lds[2 * W * 2 * 4 * 64];
     const LaunchView lv = launch_view(a);
     const int item = xcd_work((int)blockIdx.x, lv.n_items);
     if (item < 0) return;
@@ -317,71 +232,77 @@ void k_tile2d(StepArgs a) {
     const int64_t left = in.nsteps - lv.step_base;
     const int ns = left < (int64_t)a.ksteps ? (int)left : a.ksteps;
     if (ns <= 0) return;
-    // tiles of the item: halo rows on the sides that are not walls
-    const int H = ORDER * a.ksteps, end = it.ix0 + it.iw;
-    int parity = 0;
-    for (int x0 = it.ix0; x0 < end;) {
-        const int i0 = x0 - H < 0 ? 0 : x0 - H;
-        int x1 = i0 + W * RW >= in.nx ? in.nx : i0 + W * RW - H;
-        x1 = x1 < end ? x1 : end;
-        const bool edge = i0 <= 0 || i0 + W * RW >= in.nx || it.j0 <= 0 || it.j0 + 64 >= in.ny;
-        if constexpr (PREC == PREC_F64 || PREC == PREC_REF32) {
-            const bool sq = PREC == PREC_F64 ? in.k.d_lamy == 0.125 : in.k.f_lamy == 0.125f;
-            if (edge) {
-                if (sq) tile_steps<PREC, ORDER, LIM, RW, W, true, true>(a, it, in, i0, ns, x0, x1, lds, parity);
-                else tile_steps<PREC, ORDER, LIM, RW, W, true, false>(a, it, in, i0, ns, x0, x1, lds, parity);
-            } else {
-                if (sq) tile_steps<PREC, ORDER, LIM, RW, W, false, true>(a, it, in, i0, ns, x0, x1, lds, parity);
-                else tile_steps<PREC, ORDER, LIM, RW, W, false, false>(a, it, in, i0, ns, x0, x1, lds, parity);
-            }
+    // the tile's rows: the item's owned rows [ix0, ix0 + iw) and, on the sides that are not
+    // walls, the halo (the host makes no item of more than W*RW - 2k rows)
+    const int i0 = it.ix0 - a.ksteps < 0 ? 0 : it.ix0 - a.ksteps;
+    const bool edge = i0 <= 0 || i0 + W * RW >= in.nx || it.j0 <= 0 || it.j0 + 64 >= in.ny;
+    if constexpr (PREC == PREC_F64 || PREC == PREC_REF32) {
+        const bool sq = PREC == PREC_F64 ? in.k.d_lamy == 0.125 : in.k.f_lamy == 0.125f;
+        if (edge) {
+            if (sq) tile_steps<PREC, RW, W, true, true>(a, it, in, i0, ns, lds);
+            else tile_steps<PREC, RW, W, true, false>(a, it, in, i0, ns, lds);
         } else {
-            if (edge) tile_steps<PREC, ORDER, LIM, RW, W, true, false>(a, it, in, i0, ns, x0, x1, lds, parity);
-            else tile_steps<PREC, ORDER, LIM, RW, W, false, false>(a, it, in, i0, ns, x0, x1, lds, parity);
+            if (sq) tile_steps<PREC, RW, W, false, true>(a, it, in, i0, ns, lds);
+            else tile_steps<PREC, RW, W, false, false>(a, it, in, i0, ns, lds);
         }
-        x0 = x1;
+    } else {
+        if (edge) tile_steps<PREC, RW, W, true, false>(a, it, in, i0, ns, lds);
+        else tile_steps<PREC, RW, W, false, false>(a, it, in, i0, ns, lds);
     }
 }
 
-// rows per wavefront and wavefronts per block, by precision and order
-#ifndef T_RW32
-#define T_RW32 4
-#define T_W32 4
-#define T_RW64 4
-#define T_W64 4
-#endif
-template <int PREC, int ORDER>
-struct TileShape {
-    static constexpr int RW = PREC == PREC_F64 ? T_RW64 : T_RW32, W = PREC == PREC_F64 ? T_W64 : T_W32;
+// ---------------------------------------------------------------------------
+// Tile heights (rows = RW * W), by precision.  A taller tile recomputes less halo, a shorter one
+// gives more blocks: the tallest whose tiles number at least `blocks` is taken, else the
+// shortest (16 rows; with 8 steps per launch the next one, since 2k halo rows must leave owned
+// ones).  Measured, us per step: C32K, k = 4: 300^2 16 rows 2.0, 32 rows 2.9; 500^2 3.6 and 3.1;
+// 1024^2 32 rows 8.2, 40 rows 8.5; 1500^2 13.9 and 13.0; 4096^2 82 and 74.  FP64, k = 2-4: 300^2
+// 16 rows 2.7, 24 rows 3.4; 500^2 5.1 and 3.9.  REF32: 24 rows gain nothing up to 4096^2 (97 and
+// 96); C32 spills at 40 rows (4096^2 32 rows 112, 40 rows 142), FP64 at 32.
+// ---------------------------------------------------------------------------
+struct TileRows {
+    int rows, blocks;
 };
-
-int tile2d_rows(int prec, int order) {
-    (void)order;
-    return prec == PREC_F64 ? TileShape<PREC_F64, 1>::RW * TileShape<PREC_F64, 1>::W
-                            : TileShape<PREC_REF32, 1>::RW * TileShape<PREC_REF32, 1>::W;
+static const TileRows* tile_rows(int prec) {
+    static const TileRows f64[] = {{24, 200}, {16, 0}, {0, 0}};
+    static const TileRows ref32[] = {{24, 1 << 30}, {16, 0}, {0, 0}};
+    static const TileRows c32[] = {{32, 150}, {16, 0}, {0, 0}};
+    static const TileRows c32k[] = {{40, 1000}, {32, 150}, {16, 0}, {0, 0}};
+    return prec == PREC_F64 ? f64 : prec == PREC_REF32 ? ref32 : prec == PREC_C32 ? c32 : c32k;
 }
 
-template <int PREC, int ORDER, int LIM>
+// rows of the tiles for k steps per launch, 0 if none fits; tiles(owned): the number of tiles
+// that own that many rows
+int tile2d_rows(int prec, int k, int64_t (*tiles)(const void*, int), const void* arg) {
+    int rows = 0;
+    for (const TileRows* t = tile_rows(prec); t->rows > 0; ++t) {
+        if (t->rows <= 2 * k) break;
+        rows = t->rows;
+        if (tiles(arg, rows - 2 * k) >= t->blocks) break;
+    }
+    return rows;
+}
+
+template <int PREC, int RW, int W>
 static hipError_t launch_tile(int nblocks, hipStream_t s, const StepArgs& a) {
-    constexpr int RW = TileShape<PREC, ORDER>::RW, W = TileShape<PREC, ORDER>::W;
-    hipLaunchKernelGGL((k_tile2d<PREC, ORDER, LIM, RW, W>), dim3(nblocks), dim3(64 * W), 0, s, a);
+    hipLaunchKernelGGL((k_tile2d<PREC, RW, W>), dim3(nblocks), dim3(64 * W), 0, s, a);
     return hipGetLastError();
 }
 
-template <int PREC>
-static hipError_t launch_tile_p(int order, int lim, int nblocks, hipStream_t s, const StepArgs& a) {
-    if (order == 1) return launch_tile<PREC, 1, LIM_MINMOD>(nblocks, s, a);
-    return lim == LIM_MC ? launch_tile<PREC, 2, LIM_MC>(nblocks, s, a) : launch_tile<PREC, 2, LIM_MINMOD>(nblocks, s, a);
-}
-
-// one block per item
-hipError_t launch_tile2d(int prec, int order, int lim, int n_items, hipStream_t s, const StepArgs& a) {
+// one block per item; rows as tile2d_rows gives them
+hipError_t launch_tile2d(int prec, int rows, int n_items, hipStream_t s, const StepArgs& a) {
     const int nblocks = xcd_grid(n_items);
     if (nblocks <= 0) return hipSuccess;
-    switch (prec) {
-    case PREC_F64: return launch_tile_p<PREC_F64>(order, lim, nblocks, s, a);
-    case PREC_REF32: return launch_tile_p<PREC_REF32>(order, lim, nblocks, s, a);
-    case PREC_C32: return launch_tile_p<PREC_C32>(order, lim, nblocks, s, a);
-    case PREC_C32K: return launch_tile_p<PREC_C32K>(order, lim, nblocks, s, a);
+    switch (prec * 64 + rows) {
+    case PREC_F64 * 64 + 16: return launch_tile<PREC_F64, 2, 8>(nblocks, s, a);
+    case PREC_F64 * 64 + 24: return launch_tile<PREC_F64, 2, 12>(nblocks, s, a);
+    case PREC_REF32 * 64 + 16: return launch_tile<PREC_REF32, 2, 8>(nblocks, s, a);
+    case PREC_REF32 * 64 + 24: return launch_tile<PREC_REF32, 2, 12>(nblocks, s, a);
+    case PREC_C32 * 64 + 16: return launch_tile<PREC_C32, 2, 8>(nblocks, s, a);
+    case PREC_C32 * 64 + 32: return launch_tile<PREC_C32, 4, 8>(nblocks, s, a);
+    case PREC_C32K * 64 + 16: return launch_tile<PREC_C32K, 2, 8>(nblocks, s, a);
+    case PREC_C32K * 64 + 32: return launch_tile<PREC_C32K, 4, 8>(nblocks, s, a);
+    case PREC_C32K * 64 + 40: return launch_tile<PREC_C32K, 5, 8>(nblocks, s, a);
     default: return hipErrorInvalidValue;
     }
 }

@@ -1,0 +1,32 @@
+"""GPU: the 2D first-order register tiles at the edges of their tiling: domains of a few rows and
+columns, one row or column more or less than tiles and strips hold, every number of steps per
+launch, rectangular cells (DT/DY not 1/8), both walls, a last launch of fewer steps; and each
+tile height on a domain large enough to take it.  Bitwise against the oracle."""
+import pytest
+
+import icgen
+import shll_amd as S
+from test_gpu_parity import assert_same, banner, gpu_run, oracle_run
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("prec", [S.F64, S.REF32, S.C32, S.C32K])
+@pytest.mark.parametrize("shape,k", [((2, 2), 1), ((3, 5), 8), ((14, 62), 1), ((15, 63), 1), ((13, 124), 2), ((25, 125), 2),
+                                     ((10, 64), 3), ((23, 117), 3), ((8, 57), 4), ((13, 121), 4), ((33, 65), 4),
+                                     ((17, 49), 8), ((41, 97), 8)])
+def test_edges(orc, prec, shape, k):
+    for bc, dy in ((S.BC_REFLECT, 1.0), (S.BC_OUTFLOW, 0.9)):
+        pb = S.problem(2, 1, *shape, precision=prec, bc=bc, lx=1.0, ly=dy * shape[1] / shape[0])
+        ic = icgen.random_2d(*shape, 3 + k, block=3)
+        banner("tile2d", prec, shape, k, bc)
+        assert_same(pb, gpu_run(pb, ic, 2 * k + 1, (1, k, 4, 0)), oracle_run(orc, pb, ic, 2 * k + 1), "tile edges")
+
+
+@pytest.mark.parametrize("prec,shape,k", [(S.F64, (410, 600), 2), (S.REF32, (60, 100), 8), (S.C32, (310, 700), 4),
+                                          (S.C32K, (310, 700), 4), (S.C32K, (1610, 1100), 4)])
+def test_taller_tiles(orc, prec, shape, k):
+    pb = S.problem(2, 1, *shape, precision=prec, lx=1.0, ly=shape[1] / shape[0])
+    ic = icgen.random_2d(*shape, 11, block=7)
+    banner("tall tiles", prec, shape, k)
+    assert_same(pb, gpu_run(pb, ic, k + 2, (1, k, 4, 0)), oracle_run(orc, pb, ic, k + 2), "tall tiles")
