@@ -101,6 +101,10 @@ static Consts make_consts(int64_t nx, int64_t ny, double lx, double ly, double t
         k.d_lamx = CFL / (R + 1.0);
         k.d_lamy = DT / DY;
         k.d_rcv = 1.0 / k.d_cv;
+        k.d_sc = std::sqrt(k.d_gR / k.d_cv);
+        k.d_rsc = std::sqrt(k.d_cv / k.d_gR);
+        k.u_hsc = std::ldexp(k.d_sc, -513);
+        k.u_hrc = std::ldexp(k.d_rsc, -513);
     }
     k.c_rcv = (float)(1.0 / k.d_cv);
     k.c_gR = (float)k.d_gR;

@@ -192,10 +192,13 @@ __device__ __forceinline__ void sqrt_rcp(float x, float& s, float& y) {
 }
 
 // Faithful FP64 reciprocal and reciprocal square root (the F64F form): the hardware seeds
-// (v_rcp_f64, v_rsq_f64; relative error about 2^-24, measured) and two Newton steps each.
+// (v_rcp_f64, v_rsq_f64; relative error about 2^-24, measured) and a correction each.
 //   rcp_nr2(b): r <- r + r(1 - b r); equal to the correctly rounded 1/b on each of 8e8
 //               random arguments with exponents -1000..1000 (MI355X)
-//   rsq_nr2(x): y <- y (3/2 - (x/2) y^2); within 2 ulp of 1.0/sqrt(x) on the same arguments
+//   rsq_nr2(x): one third-order step y <- y (1 + e/2 + 3 e^2/8), e = 1 - x y^2 (its remainder
+//               is 5/16 e^3, about 2^-73; two Newton steps took one operation more and rounded
+//               twice); within 2 ulp of 1.0/sqrt(x) on the same arguments.  rsq_sqrt also
+//               gives sqrt(x) from the same correction, in one operation
 // Neither is correctly rounded by construction, and the seeds are the hardware's, so the
 // F64F results are reproduced on a CPU to within round-off, not bit for bit.  A zero argument
 // gives NaN (not inf); negative and NaN arguments give NaN.
@@ -206,11 +209,18 @@ __device__ __forceinline__ double rcp_nr2(double b) {
     e = __builtin_fma(-b, r, 1.0);
     return __builtin_fma(r, e, r);
 }
+__device__ __forceinline__ void rsq_sqrt(double x, double& y, double& s) {
+    const double q = __builtin_amdgcn_rsq(x);
+    const double g = x * q;
+    const double e = __builtin_fma(-g, q, 1.0);
+    const double c = __builtin_fma(0.375, e, 0.5) * e;
+    y = __builtin_fma(q, c, q);
+    s = __builtin_fma(g, c, g);
+}
 __device__ __forceinline__ double rsq_nr2(double x) {
-    const double nhx = -0.5 * x;
-    double y = __builtin_amdgcn_rsq(x);
-    y = y * __builtin_fma(nhx, y * y, 1.5);
-    return y * __builtin_fma(nhx, y * y, 1.5);
+    double y, s;
+    rsq_sqrt(x, y, s);
+    return y;
 }
 
 // ---------------------------------------------------------------------------
@@ -357,12 +367,31 @@ struct C32Arith {
 };
 
 // FP64 in the compensated scheme's arrangement (PREC_F64F): the limiter of the C32 forms in
-// double (the split fluxes are flux1_f64f in shll_flux.h)
+// double (the split fluxes are flux1_f64f in shll_flux.h), on fluxes scaled by SC.
+// minmod is the median of (l, r, 0): the smaller magnitude when the signs agree, zero otherwise
+// (sign of a zero result unspecified, as in C32Arith::mm).
+//   UNIT   SC = 2^-512, so that every |l|, |r| < 1: max(min(l, r), 0) and max(min(-l, -r), 0) are
+//          one v_min_f64 each, whose result the output clamp limits to [0, 1] for free; one of
+//          the two is zero.  Three instructions instead of four, the same values.
+//   else   SC = 1, any magnitude.
+template <bool UNIT>
 struct F64FArith {
-    // minmod as the median of (l, r, 0): the smaller magnitude when the signs agree, zero
-    // otherwise (sign of a zero result unspecified, as in C32Arith::mm)
+    static constexpr double SC = UNIT ? 0x1p-512 : 1.0;
+    // min(l, r) and min(-l, -r), each limited to [0, 1] (the compiler turns the second into a
+    // negated maximum, which takes the clamp as an instruction of its own)
+    __device__ static __forceinline__ double min01(double l, double r) {
+        double d;
+        asm("v_min_f64 %0, %1, %2 clamp" : "=v"(d) : "v"(l), "v"(r));
+        return d;
+    }
+    __device__ static __forceinline__ double nmin01(double l, double r) {
+        double d;
+        asm("v_min_f64 %0, -%1, -%2 clamp" : "=v"(d) : "v"(l), "v"(r));
+        return d;
+    }
     __device__ static __forceinline__ double mm(double l, double r) {
-        return __builtin_fmax(__builtin_fmin(l, r), __builtin_fmin(__builtin_fmax(l, r), 0.0));
+        if constexpr (UNIT) return min01(l, r) - nmin01(l, r);
+        else return __builtin_fmax(__builtin_fmin(l, r), __builtin_fmin(__builtin_fmax(l, r), 0.0));
     }
     __device__ static __forceinline__ double half(double x) { return 0.5 * x; }
 };

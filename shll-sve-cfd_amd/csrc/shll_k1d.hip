@@ -426,22 +426,24 @@ __device__ __forceinline__ void step_c32(float (&hi)[3][C], float (&lo)[3][C], c
 
 // ---------------------------------------------------------------------------
 // F64F: the C32 face-term arrangement with every value a double (no compensation: the
-// face terms are added to the FP64 state directly, u += t[m] - t[m+1]).  The split fluxes
-// come scaled by DT/DX, so a face term is G + d/2 (G = F+ of the left cell + F- of the
-// right cell, d = the difference of their limited slopes).
+// face terms are added to the FP64 state directly).  The split fluxes come scaled by SC
+// (F64FArith); a face term is G + d/2 (G = F+ of the left cell + F- of the right cell, d = the
+// difference of their limited slopes), and u += (DT/DX / SC)(t[m] - t[m+1]) in one fused
+// multiply-add, DT/DX = 1/8.
 // ---------------------------------------------------------------------------
-template <int ORDER, int C, int WM, int LIM, int XW>
+template <int ORDER, int C, int WM, int LIM, int XW, bool UNIT>
 __device__ __forceinline__ void step_f64f(double (&u)[3][C], const Inst& in, int gl, const Coop<double, XW>& x,
                                           int parity) {
-    using A = F64FArith;
-    const double lam = in.k.d_lamx, th = in.k.d_theta;
+    using A = F64FArith<UNIT>;
+    constexpr double lam = 0.125 / A::SC;
+    const double th = in.k.d_theta;
     const int n = in.nx;
     if constexpr (WM != WM_NONE) ghost_cells<C>(u, gl, n, in.bc == BC_REFLECT);
     double fp[3][C], fm[3][C];
 #pragma unroll
     for (int m = 0; m < C; ++m) {
         double p[3], q[3], a;
-        flux1_f64f(u[0][m], u[1][m], u[2][m], in, lam, p, q, a);  // scaled by DT/DX
+        flux1_f64f<UNIT>(u[0][m], u[1][m], u[2][m], in, p, q, a);
 #pragma unroll
         for (int v = 0; v < 3; ++v) {
             fp[v][m] = p[v];
@@ -457,7 +459,7 @@ __device__ __forceinline__ void step_f64f(double (&u)[3][C], const Inst& in, int
             for (int f = 0; f <= C; ++f)  // face f lies between cells gl+f-1 and gl+f
                 t[f] = __builtin_fma(0.5, w.sp(f) - w.sm(f), w.FP[f] + w.FM[f + 1]);  // G + d/2
 #pragma unroll
-            for (int m = 0; m < C; ++m) u[v][m] = u[v][m] + (t[m] - t[m + 1]);
+            for (int m = 0; m < C; ++m) u[v][m] = __builtin_fma(lam, t[m] - t[m + 1], u[v][m]);
         }
         return;
     }
@@ -487,7 +489,7 @@ __device__ __forceinline__ void step_f64f(double (&u)[3][C], const Inst& in, int
             }
         }
 #pragma unroll
-        for (int m = 0; m < C; ++m) u[v][m] = u[v][m] + (t[m] - t[m + 1]);
+        for (int m = 0; m < C; ++m) u[v][m] = __builtin_fma(lam, t[m] - t[m + 1], u[v][m]);
     }
 }
 
@@ -519,7 +521,18 @@ __device__ __forceinline__ void advance_c32(float (&hi)[3][C], float (&lo)[3][C]
 template <int ORDER, int C, int WM, int LIM, int XW>
 __device__ __forceinline__ void advance_f64f(double (&u)[3][C], const Inst& in, const Item1& it, int gl, int ns,
                                              const StepArgs& a, const Coop<double, XW>& x) {
-    for (int s = 0; s < ns; ++s) step_f64f<ORDER, C, WM, LIM, XW>(u, in, gl, x, s & 1);
+    // the limiter's clamped form (F64FArith) where it holds for the whole launch: second order,
+    // density and energy of every cell in [2^-200, 2^400] and at most 64 steps, so that no flux
+    // reaches 2^512 or falls where scaling it by 2^-512 costs digits
+    bool unit = ORDER == 2 && ns <= 64;
+#pragma unroll
+    for (int m = 0; m < C; ++m)
+        unit = unit && u[0][m] >= 0x1p-200 && u[0][m] <= 0x1p400 && u[2][m] >= 0x1p-200 && u[2][m] <= 0x1p400;
+    if (ORDER == 2 && __all(unit)) {
+        for (int s = 0; s < ns; ++s) step_f64f<ORDER, C, WM, LIM, XW, ORDER == 2>(u, in, gl, x, s & 1);
+    } else {
+        for (int s = 0; s < ns; ++s) step_f64f<ORDER, C, WM, LIM, XW, false>(u, in, gl, x, s & 1);
+    }
     double* __restrict__ ou = (double*)a.out0 + in.off;
     const int64_t P = a.plane;
 #pragma unroll

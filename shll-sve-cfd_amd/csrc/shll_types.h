@@ -17,11 +17,12 @@ enum Lim : int { LIM_MINMOD = 0, LIM_MC = 1 };
 //   F64   : d_*  (gamma = 1.4, CV = R/(gamma-1), lam = DT/DX)
 //   REF32 : f_*  (the reference's float constants, base_shll.c:17-22,83-84)
 //   C32   : c_*  (the F64 constants rounded once to float; rcv = 1/CV)
-//   F64F  : d_*, and d_rcv = 1/CV in double
+//   F64F  : d_*, d_rcv = 1/CV in double, and of c = gamma R/CV: d_sc = sqrt(c), d_rsc =
+//           1/sqrt(c), u_hsc = 2^-513 sqrt(c), u_hrc = 2^-513/sqrt(c)
 // f_rcv: 1/(double)f_cv, correctly rounded (as d_rcv is for d_cv)
 // theta: the MC limiter's weight (the reference's float alpha = 1.25 in REF32)
 struct Consts {
-    double d_cv, d_gR, d_R, d_lamx, d_lamy, d_theta, d_rcv, f_rcv;
+    double d_cv, d_gR, d_R, d_lamx, d_lamy, d_theta, d_rcv, f_rcv, d_sc, d_rsc, u_hsc, u_hrc;
     float f_cv, f_gR, f_R, f_lamx, f_lamy, f_theta;
     float c_rcv, c_gR, c_R, c_lamx, c_lamy, c_theta;
 };
