@@ -866,6 +866,72 @@ static shll_status engine_create_stream(Engine* E) {
     return SHLL_OK;
 }
 
+// Default launch shape in 1D.  Up to 65536 cells in all, a launch lasts as long as one wavefront
+// (or the few that share a SIMD): about 1.7 us and, per step, T(C) for C cells per lane.  So the
+// shape minimises T(C) x max(1, 0.85 x wavefronts of the fullest SIMD) + t0 / k over the cells
+// per lane and the owned cells W of a segment (16, or whole lines of 32), whose halo leaves
+// k = (64 C - W) / (2 order) steps per launch.  T and t0 in units of T(1): 1, 1.45 (second
+// order 1.3), 2.4, 4.3 and 4 (F64 first order 0.31 and 1.7 us, second order 0.61 and 1.7).
+// Measured, us per step: F64 first order, 1024 cells: C 1, k 8 0.52, k 16 0.41, k 24 0.37, C 2,
+// k 32 0.56; REF32 20000 cells: C 1, k 16 0.36, k 24 (more segments than SIMDs) 0.43; C32K MC
+// 9973 cells: C 1, k 12 0.55, C 2, k 16 0.66; F64F 65536 cells: C 2, k 16 0.63, C 1, k 8 0.97.
+// Single instances launch directly: a launch of 6 us or more outlasts its submission, and graph
+// nodes start 2-3% later.
+// Beyond, throughput decides (shape C,k,waves per block): batches of 4.2e5 and 5.9e6 cells, ms:
+//   second order  F64 2,16,4 15.2, 2,8,1 13.1; 2,16,4 74.5, 4,8,1 62.3
+//                 F64F 2,16,4 11.9, 2,8,1 9.5; 2,16,4 104.6, 4,8,1 79.7 (another end time)
+//                 C32K 2,16,4 9.2, 2,8,1 9.4; 4,8,1 41.1, 4,16,4 35.3
+//                 REF32 2,16,4 11.4, 2,8,1 11.6; 2,16,4 53.0, 4,8,1 48.2, 4,16,4 42.6
+//   first order   F64 2,16,4 10.5, 2,16,1 7.9; 2,16,4 40.0, 4,16,1 36.0
+//                 C32K 2,16,4 6.8, 2,16,1 6.1; 2,16,4 23.7, 4,16,1 27.8
+// and the largest batches take the autotuner's choices for the 4.7e7-cell one.
+static void default_launch1d(Engine* E, int64_t max_cells) {
+    int64_t cells = 0;
+    for (int64_t c : E->inst_cells) cells += c;
+    const bool f64 = word_bytes(E->prec) == 8;
+    E->L.graph = E->batch ? 128 : 256;
+    if (cells <= 65536) {
+        const double T[4] = {1.0, E->order == 1 ? 1.45 : 1.3, 2.4, 4.3};
+        const int64_t simds = simd_count(E);
+        double best = 1e300;
+        E->L.wpb = 1;
+        for (int c = 0; c < 4; ++c) {
+            const int C = 1 << c;
+            for (int W = 16; W < 64 * C; W += W < 32 ? 16 : 32) {  // whole 128-byte lines (tile1d)
+                const int k = std::min(64, (64 * C - W) / (2 * E->order));
+                if (k < 1) break;
+                int64_t waves = 0;
+                for (int64_t n : E->inst_cells) waves += n + 2 <= 64 * C ? 1 : (n + W - 1) / W;
+                const double cost = T[c] * std::max(1.0, 0.85 * (double)((waves + simds - 1) / simds)) + 4.0 / k;
+                if (cost < best) {
+                    best = cost;
+                    E->L.C = C;
+                    E->L.k = k;
+                }
+            }
+        }
+        if (!E->batch) E->L.graph = 0;
+        return;
+    }
+    if (!E->batch) {
+        E->L.C = 2;
+        E->L.k = 16;
+        E->L.wpb = max_cells <= 65536 ? 1 : 4;
+        return;
+    }
+    // {C, k, waves per block} for up to 1e6, up to 2e7 and more cells
+    struct S { int C, k, w; };
+    static const S o1f64[3] = {{2, 16, 1}, {4, 16, 1}, {4, 16, 1}}, o1f32[3] = {{2, 16, 1}, {2, 16, 4}, {2, 16, 4}},
+                   o2f64[3] = {{2, 8, 1}, {4, 8, 1}, {4, 8, 1}}, o2f64f[3] = {{2, 8, 1}, {4, 8, 1}, {8, 8, 1}},
+                   o2f32[3] = {{2, 16, 4}, {4, 16, 4}, {4, 16, 4}}, o2c32k[3] = {{2, 16, 4}, {4, 16, 4}, {8, 16, 1}};
+    const int z = cells <= 1000000 ? 0 : (cells <= 20000000 ? 1 : 2);
+    const S* t = E->order == 1 ? (f64 ? o1f64 : o1f32)
+                               : (E->prec == SHLL_F64F ? o2f64f : f64 ? o2f64 : E->prec == SHLL_C32K ? o2c32k : o2f32);
+    E->L.C = t[z].C;
+    E->L.k = t[z].k;
+    E->L.wpb = t[z].w;
+}
+
 static void default_launch(Engine* E, int64_t max_cells) {
     if (E->dim == 2) {
         // First order: the compensated forms take 4 steps per launch; F64 and REF32 4 on small
@@ -889,11 +955,7 @@ static void default_launch(Engine* E, int64_t max_cells) {
         E->L.graph = 64;
         return;
     }
-    // small instances: short segments and a few steps per launch keep many wavefronts busy
-    E->L.C = max_cells <= 4096 ? 1 : 2;
-    E->L.k = max_cells <= 4096 ? 8 : 16;
-    E->L.wpb = max_cells <= 65536 ? 1 : 4;
-    E->L.graph = 256;
+    default_launch1d(E, max_cells);
 }
 
 extern "C" shll_status shll_init(const shll_problem* pb, const double* prim_soa, shll_ctx** out) {
@@ -1500,12 +1562,6 @@ extern "C" shll_status shll_batch_init(const shll_problem* items, const double* 
     std::stable_sort(E->order_idx.begin(), E->order_idx.end(),
                      [&](int64_t a, int64_t b) { return E->h_inst[a].nsteps > E->h_inst[b].nsteps; });
     default_launch(E, maxcells);
-    if (E->dim == 1) {
-        E->L.C = 2;
-        E->L.k = 16;
-        E->L.wpb = 4;
-        E->L.graph = 128;
-    }
     if ((st = engine_alloc(E, off)) != SHLL_OK) { engine_free(E); return st; }
     if ((st = engine_init_state(E, prims)) != SHLL_OK) { engine_free(E); return st; }
     if ((st = engine_snapshot(E, true)) != SHLL_OK) { engine_free(E); return st; }
