@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstdarg>
@@ -13,7 +14,9 @@
 #include <cstdlib>
 #include <cstring>
 #include <limits>
+#include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "shll.h"
@@ -33,7 +36,8 @@ hipError_t launch_init(int prec, int dim, int nblocks, int n_inst, hipStream_t s
 hipError_t launch_stage(int prec, int dim, int nblocks, hipStream_t st, const Inst* inst, const void* s0,
                         int64_t plane, double* out);
 hipError_t launch_output(int prec, int dim, int nblocks, int n_inst, hipStream_t st, const Inst* insts,
-                         const void* s0, const void* s1, int64_t plane, double* prim, double* cons);
+                         const void* s0, const void* s1, int64_t plane, double* prim, double* cons, int64_t plane_out,
+                         int64_t off_out);
 hipError_t launch_sums(int prec, int dim, int nblocks, int n_inst, hipStream_t st, const Inst* insts,
                        const void* s0, const void* s1, int64_t plane, double* partial);
 hipError_t launch_ctl(hipStream_t st, int64_t* ctl, int64_t v0, int64_t v1, int64_t v2, int add);
@@ -69,6 +73,113 @@ static shll_status fail(shll_status st, const char* fmt, ...) {
 
 extern "C" const char* shll_last_error(void) { return g_err.c_str(); }
 extern "C" const char* shll_version(void) { return "shll_amd 0.1 (gfx950)"; }
+
+// ---------------------------------------------------------------------------
+// host transfers through pinned slabs
+//
+// Callers pass pageable memory.  The runtime's own pageable copies move about 10 GB/s from the
+// device (one thread copying out of its staging buffer) and cost some 10 us each however small;
+// pinning a buffer per call costs 0.1 ms to 40 ms.  So transfers go through pinned slabs of 4
+// MiB that are kept between calls: up to 4 MiB the output kernels write straight into one slab
+// (no copy command, one synchronisation), beyond that up to eight threads each take the next
+// piece, copy it between its slab and the caller's memory, and have a second piece in flight.
+// Measured (16-core host), before and now: 24 KB of primitives 48 and 14 us, 111 MB of 400 tubes
+// one by one 24 and 11.8 ms, 537 MB 51.5 and 12.5 ms; constructing a 128^2 context 183 and 96 us.
+// ---------------------------------------------------------------------------
+namespace {
+constexpr size_t kSlabBytes = 4u << 20;
+constexpr size_t kSlabsKept = 16;
+
+// The slabs not in use: at most kSlabsKept stay allocated for the process, the others are freed
+// when they are returned.  Portable, so any device may use any slab.
+std::mutex g_slab_mu;
+char* g_slabs[kSlabsKept];
+size_t g_nslabs = 0;
+
+struct Slab {
+    char* p = nullptr;
+    Slab() {
+        {
+            std::lock_guard<std::mutex> lock(g_slab_mu);
+            if (g_nslabs > 0) {
+                p = g_slabs[--g_nslabs];
+                return;
+            }
+        }
+        if (hipHostMalloc((void**)&p, kSlabBytes, hipHostMallocPortable) != hipSuccess) p = nullptr;
+    }
+    // its last use by the device must have completed
+    ~Slab() {
+        if (!p) return;
+        {
+            std::lock_guard<std::mutex> lock(g_slab_mu);
+            if (g_nslabs < kSlabsKept) {
+                g_slabs[g_nslabs++] = p;
+                return;
+            }
+        }
+        (void)hipHostFree(p);
+    }
+    Slab(const Slab&) = delete;
+    Slab& operator=(const Slab&) = delete;
+};
+
+// Pieces [0, n) of a transfer.  start(i, slab): enqueue the copy between slab and device (an
+// upload fills the slab first); finish(i, slab): after it has completed.  Every piece is done by
+// the time this returns; the first error wins.
+template <class Start, class Finish>
+hipError_t transfer(int device, hipStream_t stream, size_t n, const Start& start, const Finish& finish) {
+    std::atomic<size_t> next{0};
+    std::atomic<int> error{(int)hipSuccess};
+    auto work = [&]() {
+        hipError_t e = hipSetDevice(device);
+        Slab slab[2];
+        hipEvent_t ev[2] = {nullptr, nullptr};
+        for (int q = 0; q < 2 && e == hipSuccess; ++q) {
+            if (!slab[q].p) e = hipErrorOutOfMemory;
+            else e = hipEventCreateWithFlags(&ev[q], hipEventDisableTiming);
+        }
+        size_t at[2];
+        bool busy[2] = {false, false};
+        for (int q = 0;; q ^= 1) {
+            if (busy[q]) {
+                const hipError_t w = hipEventSynchronize(ev[q]);
+                busy[q] = false;
+                if (w == hipSuccess) finish(at[q], slab[q].p);
+                else if (e == hipSuccess) e = w;
+            }
+            const size_t i = e == hipSuccess && error.load() == (int)hipSuccess ? next.fetch_add(1) : n;
+            if (i < n) {
+                at[q] = i;
+                const hipError_t c = start(i, slab[q].p);
+                const hipError_t r = hipEventRecord(ev[q], stream);
+                busy[q] = true;  // waited for even after an error, so the slab is idle when it goes back
+                e = c != hipSuccess ? c : r;
+            } else if (!busy[q ^ 1]) {
+                break;
+            }
+        }
+        if (e != hipSuccess) {
+            int ok = (int)hipSuccess;
+            error.compare_exchange_strong(ok, (int)e);
+            (void)hipStreamSynchronize(stream);
+        }
+        for (int q = 0; q < 2; ++q)
+            if (ev[q]) (void)hipEventDestroy(ev[q]);
+    };
+    const size_t want = std::min<size_t>(std::min<size_t>(8, std::max(1u, std::thread::hardware_concurrency() / 2)),
+                                         (n + 1) / 2);
+    std::thread helpers[8];
+    size_t made = 0;
+    try {
+        for (; made + 1 < want; ++made) helpers[made] = std::thread(work);
+    } catch (...) {  // no more threads: the others take the pieces
+    }
+    work();
+    for (size_t t = 0; t < made; ++t) helpers[t].join();
+    return (hipError_t)error.load();
+}
+}  // namespace
 
 // ---------------------------------------------------------------------------
 // constants and step counts
@@ -733,38 +844,65 @@ static shll_status engine_alloc(Engine* E, int64_t plane) {
 
 static int elem_blocks(int64_t ncell) { return (int)std::max<int64_t>(1, std::min<int64_t>(2048, (ncell + 255) / 256)); }
 
+// device memory for the primitives (or conserved variables) of all instances as doubles
+static shll_status ensure_prim(Engine* E) {
+    if (!E->d_prim) HIPCHECK(hipMalloc(&E->d_prim, (size_t)E->plane * E->nv * sizeof(double)));
+    return SHLL_OK;
+}
+
 // upload primitives of all instances and convert them (k_init) into buffer 0
 static shll_status engine_init_state(Engine* E, const double* const* prims) {
-    const size_t pbytes = (size_t)E->plane * E->nv * sizeof(double);
-    double* d_p = nullptr;
-    HIPCHECK(hipMalloc(&d_p, pbytes));
-    // gather every instance's primitives into one pinned staging buffer in the device
-    // layout, then one host-to-device copy (instead of nvar copies per instance)
-    double* h_p = nullptr;
-    if (hipHostMalloc((void**)&h_p, pbytes, hipHostMallocDefault) != hipSuccess) {
-        (void)hipFree(d_p);
-        return fail(SHLL_ENOMEM, "hipHostMalloc(%zu) for the initial data", pbytes);
-    }
+    const size_t total = (size_t)E->plane * E->nv * sizeof(double);
     int64_t maxcells = 0;
-    for (size_t i = 0; i < E->h_inst.size(); ++i) {
-        const int64_t nc = E->inst_cells[i];
-        maxcells = std::max(maxcells, nc);
-        for (int v = 0; v < E->nv; ++v)
-            std::memcpy(h_p + v * E->plane + E->h_inst[i].off, prims[i] + (size_t)v * nc, (size_t)nc * sizeof(double));
+    for (int64_t c : E->inst_cells) maxcells = std::max(maxcells, c);
+    // bytes [at, at + len) of the device layout (planes of all instances, each padded to 64 cells)
+    auto gather = [&](char* dst, size_t at, size_t len) {
+        size_t g = at / sizeof(double);
+        const size_t end = (at + len) / sizeof(double);
+        while (g < end) {
+            const size_t v = g / (size_t)E->plane, o = g % (size_t)E->plane;
+            // the instance at offset o: the last one that starts at or before it
+            size_t i = std::upper_bound(E->h_inst.begin(), E->h_inst.end(), (int64_t)o,
+                                        [](int64_t x, const Inst& in) { return x < in.off; }) - E->h_inst.begin() - 1;
+            for (; i < E->h_inst.size() && g < end && g / (size_t)E->plane == v; ++i) {
+                const size_t off = (size_t)E->h_inst[i].off, nc = (size_t)E->inst_cells[i];
+                const size_t stop = i + 1 < E->h_inst.size() ? (size_t)E->h_inst[i + 1].off : (size_t)E->plane;
+                const size_t from = g - v * (size_t)E->plane - off;  // cell within the instance, or its padding
+                const size_t take = from < nc ? std::min(nc - from, end - g) : 0;
+                std::memcpy(dst + g * sizeof(double) - at, prims[i] + v * nc + from, take * sizeof(double));
+                g = std::min(end, v * (size_t)E->plane + stop);
+            }
+        }
+    };
+    auto convert = [&](const double* src) {
+        return launch_init(E->prec, E->dim, elem_blocks(maxcells), (int)E->h_inst.size(), E->stream, E->d_inst, src,
+                           E->buf[0][0], E->buf[0][1], E->plane);
+    };
+    if (total <= kSlabBytes) {
+        Slab slab;
+        if (!slab.p) return fail(SHLL_ENOMEM, "hipHostMalloc(%zu) for the initial data", kSlabBytes);
+        gather(slab.p, 0, total);
+        const hipError_t e = convert((const double*)slab.p);
+        const hipError_t w = hipStreamSynchronize(E->stream);
+        if (e != hipSuccess || w != hipSuccess)
+            return fail(SHLL_EDEVICE, "init kernel: %s", hipGetErrorString(e != hipSuccess ? e : w));
+    } else {
+        shll_status st = ensure_prim(E);
+        if (st != SHLL_OK) return st;
+        auto len = [&](size_t i) { return std::min(kSlabBytes, total - i * kSlabBytes); };
+        hipError_t e = transfer(
+            E->device, E->stream, (total + kSlabBytes - 1) / kSlabBytes,
+            [&](size_t i, char* slab) {
+                gather(slab, i * kSlabBytes, len(i));
+                return hipMemcpyAsync((char*)E->d_prim + i * kSlabBytes, slab, len(i), hipMemcpyHostToDevice, E->stream);
+            },
+            [](size_t, const char*) {});
+        if (e != hipSuccess) return fail(SHLL_EDEVICE, "upload: %s", hipGetErrorString(e));
+        e = convert(E->d_prim);
+        const hipError_t w = hipStreamSynchronize(E->stream);
+        if (e != hipSuccess || w != hipSuccess)
+            return fail(SHLL_EDEVICE, "init kernel: %s", hipGetErrorString(e != hipSuccess ? e : w));
     }
-    hipError_t eu = hipMemcpyAsync(d_p, h_p, pbytes, hipMemcpyHostToDevice, E->stream);
-    hipError_t es = hipStreamSynchronize(E->stream);
-    (void)hipHostFree(h_p);
-    if (eu != hipSuccess || es != hipSuccess) {
-        (void)hipFree(d_p);
-        return fail(SHLL_EDEVICE, "upload: %s", hipGetErrorString(eu != hipSuccess ? eu : es));
-    }
-    hipError_t e = launch_init(E->prec, E->dim, elem_blocks(maxcells), (int)E->h_inst.size(), E->stream, E->d_inst, d_p,
-                               E->buf[0][0], E->buf[0][1], E->plane);
-    hipError_t e2 = hipStreamSynchronize(E->stream);
-    (void)hipFree(d_p);
-    if (e != hipSuccess || e2 != hipSuccess)
-        return fail(SHLL_EDEVICE, "init kernel: %s", hipGetErrorString(e != hipSuccess ? e : e2));
     engine_rewind(E);
     return SHLL_OK;
 }
@@ -784,24 +922,44 @@ static shll_status engine_snapshot(Engine* E, bool save) {
     return SHLL_OK;
 }
 
-// primitives (and conserved) of instance i into host arrays (nv * cells each)
+// contiguous device memory to the caller's
+static shll_status download(Engine* E, void* dst, const void* src, size_t bytes) {
+    const size_t n = (bytes + kSlabBytes - 1) / kSlabBytes;
+    auto len = [&](size_t i) { return std::min(kSlabBytes, bytes - i * kSlabBytes); };
+    HIPCHECK(transfer(
+        E->device, E->stream, n,
+        [&](size_t i, char* slab) {
+            return hipMemcpyAsync(slab, (const char*)src + i * kSlabBytes, len(i), hipMemcpyDeviceToHost, E->stream);
+        },
+        [&](size_t i, const char* slab) { std::memcpy((char*)dst + i * kSlabBytes, slab, len(i)); }));
+    return SHLL_OK;
+}
+
+// primitives or conserved variables of instance i into a host array (nv * cells)
 static shll_status engine_get(Engine* E, int64_t i, double* prim, double* cons) {
     const int64_t nc = E->inst_cells[i];
-    if (!E->d_prim) HIPCHECK(hipMalloc(&E->d_prim, (size_t)E->plane * E->nv * sizeof(double)));
-    if (cons && !E->d_cons) HIPCHECK(hipMalloc(&E->d_cons, (size_t)E->plane * E->nv * sizeof(double)));
+    const size_t bytes = (size_t)nc * E->nv * sizeof(double);
+    double* dst = prim ? prim : cons;
     const int p = inst_parity(E, i);
     // one instance: point the kernel at its Inst record
-    HIPCHECK(launch_output(E->prec, E->dim, elem_blocks(nc), 1, E->stream, E->d_inst + i, E->buf[p][0], E->buf[p][1],
-                           E->plane, E->d_prim, cons ? E->d_cons : nullptr));
-    for (int v = 0; v < E->nv; ++v) {
-        const size_t off = (size_t)v * E->plane + E->h_inst[i].off;
-        if (prim) HIPCHECK(hipMemcpyAsync(prim + (size_t)v * nc, E->d_prim + off, nc * sizeof(double),
-                                          hipMemcpyDeviceToHost, E->stream));
-        if (cons) HIPCHECK(hipMemcpyAsync(cons + (size_t)v * nc, E->d_cons + off, nc * sizeof(double),
-                                          hipMemcpyDeviceToHost, E->stream));
+    auto output = [&](double* o) {
+        return launch_output(E->prec, E->dim, elem_blocks(nc), 1, E->stream, E->d_inst + i, E->buf[p][0], E->buf[p][1],
+                             E->plane, prim ? o : nullptr, prim ? nullptr : o, nc, 0);
+    };
+    if (bytes <= kSlabBytes) {
+        Slab slab;
+        if (!slab.p) return fail(SHLL_ENOMEM, "hipHostMalloc(%zu)", kSlabBytes);
+        const hipError_t e = output((double*)slab.p);
+        const hipError_t w = hipStreamSynchronize(E->stream);
+        HIPCHECK(e);
+        HIPCHECK(w);
+        std::memcpy(dst, slab.p, bytes);
+        return SHLL_OK;
     }
-    HIPCHECK(hipStreamSynchronize(E->stream));
-    return SHLL_OK;
+    shll_status st = ensure_prim(E);
+    if (st != SHLL_OK) return st;
+    HIPCHECK(output(E->d_prim));
+    return download(E, dst, E->d_prim, bytes);
 }
 
 static shll_status ensure_partial(Engine* E, size_t n) {
@@ -819,24 +977,45 @@ static shll_status engine_sums(Engine* E, std::vector<double>& out) {
     int64_t maxcells = 0;
     for (int64_t c : E->inst_cells) maxcells = std::max(maxcells, c);
     const int nb = std::min(elem_blocks(maxcells), 256);
-    shll_status st = ensure_partial(E, (size_t)ninst * nb * 6);
-    if (st != SHLL_OK) return st;
+    const size_t n = (size_t)ninst * nb * 6;
     out.assign((size_t)ninst * 5, 0.0);
-    std::vector<double> part((size_t)ninst * nb * 6);
+    // few partials: the kernel writes them into a pinned slab
+    const bool small = n * sizeof(double) <= kSlabBytes;
+    std::vector<double> part(small ? 0 : n);
     // instances may sit in different buffers: launch per parity group
     for (int p = 0; p < 2; ++p) {
-        HIPCHECK(launch_sums(E->prec, E->dim, nb, (int)ninst, E->stream, E->d_inst, E->buf[p][0], E->buf[p][1],
-                             E->plane, E->d_partial));
-        HIPCHECK(hipMemcpyAsync(part.data(), E->d_partial, part.size() * sizeof(double), hipMemcpyDeviceToHost,
-                                E->stream));
-        HIPCHECK(hipStreamSynchronize(E->stream));
-        for (int64_t i = 0; i < ninst; ++i) {
-            if (inst_parity(E, i) != p) continue;
-            for (int q = 0; q < 5; ++q) {
-                double t = 0;
-                for (int b = 0; b < nb; ++b) t += part[((size_t)i * nb + b) * 6 + q];
-                out[(size_t)i * 5 + q] = t;
+        bool any = false;
+        for (int64_t i = 0; i < ninst && !any; ++i) any = inst_parity(E, i) == p;
+        if (!any) continue;
+        auto sums = [&](double* partial) {
+            return launch_sums(E->prec, E->dim, nb, (int)ninst, E->stream, E->d_inst, E->buf[p][0], E->buf[p][1], E->plane,
+                               partial);
+        };
+        auto add = [&](const double* pt) {
+            for (int64_t i = 0; i < ninst; ++i) {
+                if (inst_parity(E, i) != p) continue;
+                for (int q = 0; q < 5; ++q) {
+                    double t = 0;
+                    for (int b = 0; b < nb; ++b) t += pt[((size_t)i * nb + b) * 6 + q];
+                    out[(size_t)i * 5 + q] = t;
+                }
             }
+        };
+        if (small) {
+            Slab slab;
+            if (!slab.p) return fail(SHLL_ENOMEM, "hipHostMalloc(%zu)", kSlabBytes);
+            const hipError_t e = sums((double*)slab.p);
+            const hipError_t w = hipStreamSynchronize(E->stream);
+            HIPCHECK(e);
+            HIPCHECK(w);
+            add((const double*)slab.p);
+        } else {
+            shll_status st = ensure_partial(E, n);
+            if (st != SHLL_OK) return st;
+            HIPCHECK(sums(E->d_partial));
+            HIPCHECK(hipMemcpyAsync(part.data(), E->d_partial, n * sizeof(double), hipMemcpyDeviceToHost, E->stream));
+            HIPCHECK(hipStreamSynchronize(E->stream));
+            add(part.data());
         }
     }
     return SHLL_OK;
@@ -952,7 +1131,8 @@ static void default_launch(Engine* E, int64_t max_cells) {
         else E->L.k = E->prec == SHLL_F64 && cells < 1500000 ? 3 : 2;
         E->L.wpb = 4;
         E->L.rows = default_rows2d(E, E->L.k);
-        E->L.graph = 64;
+        // first-order launches of a single instance last 7 us or more and are submitted directly
+        E->L.graph = E->batch || E->order == 2 ? 64 : 0;
         return;
     }
     default_launch1d(E, max_cells);
@@ -1047,8 +1227,13 @@ extern "C" shll_status shll_get_state_raw(shll_ctx* ctx, void* out, size_t bytes
     char* o = (char*)out;
     for (int w = 0; w < nwords(E->prec); ++w)
         for (int v = 0; v < E->nv; ++v) {
-            HIPCHECK(hipMemcpyAsync(o, (const char*)E->buf[E->cur][w] + (size_t)v * E->plane * wb, nc * wb,
-                                    hipMemcpyDeviceToHost, E->stream));
+            const char* src = (const char*)E->buf[E->cur][w] + (size_t)v * E->plane * wb;
+            if ((size_t)nc * wb > kSlabBytes) {
+                shll_status st = download(E, o, src, (size_t)nc * wb);
+                if (st != SHLL_OK) return st;
+            } else {
+                HIPCHECK(hipMemcpyAsync(o, src, nc * wb, hipMemcpyDeviceToHost, E->stream));
+            }
             o += nc * wb;
         }
     HIPCHECK(hipStreamSynchronize(E->stream));
@@ -1217,10 +1402,11 @@ extern "C" shll_status shll_stage_fluxes(shll_ctx* ctx, double* a, double* fp, d
 
 // primitives of instance i on the device (E->d_prim at the instance's offset)
 static shll_status engine_prim_dev(Engine* E, int64_t i, const double** out) {
-    if (!E->d_prim) HIPCHECK(hipMalloc(&E->d_prim, (size_t)E->plane * E->nv * sizeof(double)));
+    shll_status st = ensure_prim(E);
+    if (st != SHLL_OK) return st;
     const int p = inst_parity(E, i);
     HIPCHECK(launch_output(E->prec, E->dim, elem_blocks(E->inst_cells[i]), 1, E->stream, E->d_inst + i,
-                           E->buf[p][0], E->buf[p][1], E->plane, E->d_prim, nullptr));
+                           E->buf[p][0], E->buf[p][1], E->plane, E->d_prim, nullptr, E->plane, E->h_inst[i].off));
     HIPCHECK(hipStreamSynchronize(E->stream));
     *out = E->d_prim + E->h_inst[i].off;
     return SHLL_OK;

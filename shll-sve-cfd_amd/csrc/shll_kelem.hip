@@ -85,9 +85,11 @@ __device__ __forceinline__ void load_cons(const void* s0, const void* s1, int64_
     }
 }
 
+// plane_out, off_out: cells per plane of the outputs and where the instance starts in them
 template <int PREC, int DIM>
 __global__ __launch_bounds__(256) void k_output(const Inst* insts, const void* s0, const void* s1, int64_t plane,
-                                                double* __restrict__ prim, double* __restrict__ cons) {
+                                                double* __restrict__ prim, double* __restrict__ cons,
+                                                int64_t plane_out, int64_t off_out) {
     const Inst in = insts[blockIdx.y];
     const int64_t ncell = (int64_t)in.nx * in.ny;
     for (int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; c < ncell;
@@ -121,8 +123,8 @@ __global__ __launch_bounds__(256) void k_output(const Inst* insts, const void* s
         }
 #pragma unroll
         for (int v = 0; v < DIM + 2; ++v) {
-            if (prim) prim[v * plane + o] = p[v];
-            if (cons) cons[v * plane + o] = U[v];
+            if (prim) prim[v * plane_out + off_out + c] = p[v];
+            if (cons) cons[v * plane_out + off_out + c] = U[v];
         }
     }
 }
@@ -335,18 +337,20 @@ hipError_t launch_stage(int prec, int dim, int nblocks, hipStream_t st, const In
 
 template <int PREC>
 static hipError_t output_p(int dim, dim3 g, hipStream_t st, const Inst* insts, const void* s0, const void* s1,
-                           int64_t plane, double* prim, double* cons) {
-    if (dim == 1) hipLaunchKernelGGL((k_output<PREC, 1>), g, dim3(256), 0, st, insts, s0, s1, plane, prim, cons);
-    else hipLaunchKernelGGL((k_output<PREC, 2>), g, dim3(256), 0, st, insts, s0, s1, plane, prim, cons);
+                           int64_t plane, double* prim, double* cons, int64_t po, int64_t oo) {
+    if (dim == 1) hipLaunchKernelGGL((k_output<PREC, 1>), g, dim3(256), 0, st, insts, s0, s1, plane, prim, cons, po, oo);
+    else hipLaunchKernelGGL((k_output<PREC, 2>), g, dim3(256), 0, st, insts, s0, s1, plane, prim, cons, po, oo);
     return hipGetLastError();
 }
 
 hipError_t launch_output(int prec, int dim, int nblocks, int n_inst, hipStream_t st, const Inst* insts,
-                         const void* s0, const void* s1, int64_t plane, double* prim, double* cons) {
+                         const void* s0, const void* s1, int64_t plane, double* prim, double* cons, int64_t plane_out,
+                         int64_t off_out) {
     dim3 g(nblocks, n_inst);
-    if (prec == PREC_F64 || prec == PREC_F64F) return output_p<PREC_F64>(dim, g, st, insts, s0, s1, plane, prim, cons);
-    if (prec == PREC_REF32) return output_p<PREC_REF32>(dim, g, st, insts, s0, s1, plane, prim, cons);
-    return output_p<PREC_C32>(dim, g, st, insts, s0, s1, plane, prim, cons);
+    const int64_t po = plane_out, oo = off_out;
+    if (prec == PREC_F64 || prec == PREC_F64F) return output_p<PREC_F64>(dim, g, st, insts, s0, s1, plane, prim, cons, po, oo);
+    if (prec == PREC_REF32) return output_p<PREC_REF32>(dim, g, st, insts, s0, s1, plane, prim, cons, po, oo);
+    return output_p<PREC_C32>(dim, g, st, insts, s0, s1, plane, prim, cons, po, oo);
 }
 
 template <int PREC>
