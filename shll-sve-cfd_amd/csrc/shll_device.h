@@ -229,8 +229,8 @@ __device__ __forceinline__ double rsq_nr2(double x) {
 // sqrt() put them (base_shll.c:135-139, :172-175; base_shll_2d.c:313-317).
 // For RT = double every conversion is the identity.
 //
-// prim*_fast give the bits of prim*_exact in about half the instructions, and *ok = false
-// where they may not:
+// prim*_fast give the bits of prim*_exact in about half the instructions, and say where they
+// may not:
 //   - quotients with one divisor share its reciprocal (u1/u0, u2/u0, u3/u0; vx/a, vy/a); 1/cv
 //     is a constant (Consts::d_rcv, f_rcv, correctly rounded by the host);
 //   - e - kin is one fused multiply-add: kin/2's product is exact (a power of two times a
@@ -238,9 +238,17 @@ __device__ __forceinline__ double rsq_nr2(double x) {
 //   - (float)sqrt((double)x) of a float x is the float square root (rounding twice is
 //     harmless from 53 to 24 bits), so REF32 takes it in float;
 //   - a quotient of +-0 comes out as +0, a zero whose sign no sum here keeps.
-// One test per cell covers all of it: the radicand x = gamma R T in [XLO, XHI] and |M| >= MLO
-// or a zero velocity.  T > 0 then bounds e = cv T + kin below, x and M bound |vx| = |M| a, so
-// every quotient and residual is normal (or exactly zero); non-finite states fail the test on x.
+// Two tests per cell cover all of it:
+//   - the radicand x = gamma R T in [XLO, XHI] (else false: the cell takes prim*_exact).  T > 0
+//     then bounds e = cv T + kin below and a away from the ends of the range; non-finite states
+//     fail here;
+//   - every velocity |v| >= VLO or exactly zero (else *tiny: the caller divides again with the
+//     operator).  Only the velocity itself needs it: with |v| below VLO, M/2 +- 1/2 is +-1/2
+//     and 1 - M^2 is 1 whatever M's last bits, and v^2 vanishes in kin.  Transverse velocities
+//     ahead of a front square from cell to cell (1e-9, 1e-18, 1e-36, 0), so a wavefront that
+//     holds a front nearly always has such a lane: REF32 at 128^2, four steps per launch, 10.7
+//     us with the whole cell redone there, 8.4 us with the divisions only, 7.6 us once the
+//     fronts are gone.
 // Before, each of the five (2D: seven) operations carried its own compare and branch, and a
 // gas at rest (u = 0) took the slow path of two of them: 1D first order FP64, 1024 cells,
 // 5.43 us per 8-step launch, 4.2 us now; second order, 4 cells per lane: 894 VALU instructions per
@@ -248,10 +256,10 @@ __device__ __forceinline__ double rsq_nr2(double x) {
 // ---------------------------------------------------------------------------
 template <class RT> struct RefRange;
 template <> struct RefRange<double> {
-    static constexpr double XLO = 0x1p-700, XHI = 0x1p+700, MLO = 0x1p-500;
+    static constexpr double XLO = 0x1p-700, XHI = 0x1p+700, VLO = 0x1p-900;
 };
 template <> struct RefRange<float> {
-    static constexpr float XLO = 0x1p-30f, XHI = 0x1p+60f, MLO = 0x1p-45f;
+    static constexpr float XLO = 0x1p-30f, XHI = 0x1p+60f, VLO = 0x1p-64f;
 };
 
 template <class RT>
@@ -269,7 +277,7 @@ struct RefArith {
         M = vx / a;
     }
     __device__ static __forceinline__ bool prim1_fast(RT u0, RT u1, RT u2, int ke, RT cv, double rcv, RT gR, RT& vx,
-                                                      RT& T, RT& a, RT& M) {
+                                                      RT& T, RT& a, RT& M, bool& tiny) {
         RT y;
         if constexpr (F32) y = rcp_fast(u0);
         else y = rcp_2n(u0);
@@ -277,15 +285,20 @@ struct RefArith {
         const double e = (double)quot(u2, u0, y);
         const double vv = ke == 0 && F32 ? (double)vx * (double)vx : (double)(vx * vx);
         T = (RT)quot(__builtin_fma(-0.5, vv, e), (double)cv, rcv);
-        return sound(u1, T, gR, vx, a, M, y);
+        tiny |= small(vx, u1);
+        return sound(T, gR, vx, a, M, y);
     }
-    // a = sqrt(gamma R T), y = 1/a, M = v/a and the range test (um: the momentum of v)
-    __device__ static __forceinline__ bool sound(RT um, RT T, RT gR, RT v, RT& a, RT& M, RT& y) {
+    // a = sqrt(gamma R T), y = 1/a, M = v/a and the range test on x
+    __device__ static __forceinline__ bool sound(RT T, RT gR, RT v, RT& a, RT& M, RT& y) {
         using R = RefRange<RT>;
         const RT x = gR * T;
         sqrt_rcp(x, a, y);
         M = quot(v, a, y);
-        return x >= R::XLO && x <= R::XHI && (fabs(M) >= R::MLO || um == (RT)0);
+        return x >= R::XLO && x <= R::XHI;
+    }
+    // the range test on a velocity (um: its momentum)
+    __device__ static __forceinline__ bool small(RT v, RT um) {
+        return !(fabs(v) >= RefRange<RT>::VLO || um == (RT)0);
     }
     // Compute_P_from_U, 2D (base_shll_2d.c:313-317), and the two Mach numbers
     __device__ static __forceinline__ void prim2_exact(RT u0, RT u1, RT u2, RT u3, RT cv, RT gR, RT& vx, RT& vy,
@@ -298,8 +311,7 @@ struct RefArith {
         My = vy / a;
     }
     __device__ static __forceinline__ bool prim2_fast(RT u0, RT u1, RT u2, RT u3, RT cv, double rcv, RT gR, RT& vx,
-                                                      RT& vy, RT& T, RT& a, RT& Mx, RT& My) {
-        using R = RefRange<RT>;
+                                                      RT& vy, RT& T, RT& a, RT& Mx, RT& My, bool& tiny) {
         RT y;
         if constexpr (F32) y = rcp_fast(u0);
         else y = rcp_2n(u0);
@@ -307,9 +319,10 @@ struct RefArith {
         vy = quot(u2, u0, y);
         const double e = (double)quot(u3, u0, y);
         T = (RT)quot(__builtin_fma(-0.5, (double)(vx * vx + vy * vy), e), (double)cv, rcv);
-        const bool ok = sound(u1, T, gR, vx, a, Mx, y);
+        const bool ok = sound(T, gR, vx, a, Mx, y);
         My = quot(vy, a, y);
-        return ok && (fabs(My) >= R::MLO || u2 == (RT)0);
+        tiny |= small(vx, u1) || small(vy, u2);
+        return ok;
     }
     // Z invariants (base_shll.c:137-139): 0.5*(M +- 1) in double, stored to RT, is M/2 +- 1/2
     // rounded once: M/2 is exact, and for a float M the double sum is exact or nowhere near the

@@ -26,13 +26,15 @@ __device__ __forceinline__ void ref_consts(const Inst& in, RT& cv, double& rcv, 
         gR = in.k.f_gR;
     }
 }
-// Compute_P_from_U of one cell: the fast form (false: take the exact one), the exact form
+// Compute_P_from_U of one cell: the fast form (false: take the exact one; tiny: divide for the
+// velocity again), the exact form
 template <class RT>
-__device__ __forceinline__ bool ref_prim1(RT u0, RT u1, RT u2, const Inst& in, RT& vx, RT& T, RT& a, RT& M) {
+__device__ __forceinline__ bool ref_prim1(RT u0, RT u1, RT u2, const Inst& in, RT& vx, RT& T, RT& a, RT& M,
+                                          bool& tiny) {
     RT cv, gR;
     double rcv;
     ref_consts<RT>(in, cv, rcv, gR);
-    return RefArith<RT>::prim1_fast(u0, u1, u2, in.ke, cv, rcv, gR, vx, T, a, M);
+    return RefArith<RT>::prim1_fast(u0, u1, u2, in.ke, cv, rcv, gR, vx, T, a, M, tiny);
 }
 template <class RT>
 __device__ __forceinline__ void ref_prim1_exact(RT u0, RT u1, RT u2, const Inst& in, RT& vx, RT& T, RT& a, RT& M) {
@@ -105,7 +107,9 @@ __device__ __forceinline__ void flux1(RT u0, RT u1, RT u2, const Inst& in, RT (&
         split_c32(f2, u2, z1, z2, z3, fp[2], fm[2]);
     } else {
         RT M;
-        if (!ref_prim1<RT>(u0, u1, u2, in, vx, T, a, M)) ref_prim1_exact<RT>(u0, u1, u2, in, vx, T, a, M);
+        bool tiny = false;
+        if (!ref_prim1<RT>(u0, u1, u2, in, vx, T, a, M, tiny)) ref_prim1_exact<RT>(u0, u1, u2, in, vx, T, a, M);
+        else if (tiny) vx = u1 / u0;
         ref_flux1<RT>(u0, u1, u2, vx, T, a, M, fp, fm);
     }
 }
@@ -116,11 +120,11 @@ struct Prim2 {
     RT vx, vy, T, a, Mx, My;
 };
 template <class RT>
-__device__ __forceinline__ bool ref_prim2(const RT (&U)[4], const Inst& in, Prim2<RT>& q) {
+__device__ __forceinline__ bool ref_prim2(const RT (&U)[4], const Inst& in, Prim2<RT>& q, bool& tiny) {
     RT cv, gR;
     double rcv;
     ref_consts<RT>(in, cv, rcv, gR);
-    return RefArith<RT>::prim2_fast(U[0], U[1], U[2], U[3], cv, rcv, gR, q.vx, q.vy, q.T, q.a, q.Mx, q.My);
+    return RefArith<RT>::prim2_fast(U[0], U[1], U[2], U[3], cv, rcv, gR, q.vx, q.vy, q.T, q.a, q.Mx, q.My, tiny);
 }
 template <class RT>
 __device__ __forceinline__ void ref_prim2_exact(const RT (&U)[4], const Inst& in, Prim2<RT>& q) {
@@ -128,6 +132,16 @@ __device__ __forceinline__ void ref_prim2_exact(const RT (&U)[4], const Inst& in
     double rcv;
     ref_consts<RT>(in, cv, rcv, gR);
     RefArith<RT>::prim2_exact(U[0], U[1], U[2], U[3], cv, gR, q.vx, q.vy, q.T, q.a, q.Mx, q.My);
+}
+// redo what the fast form could not: ok, tiny as ref_prim2 says
+template <class RT>
+__device__ __forceinline__ void ref_prim2_redo(const RT (&U)[4], const Inst& in, bool ok, Prim2<RT>& q) {
+    if (!ok) {
+        ref_prim2_exact<RT>(U, in, q);
+    } else {
+        q.vx = U[1] / U[0];
+        q.vy = U[2] / U[0];
+    }
 }
 // Compute_F_from_P of one cell, x and y (base_shll_2d.c:239-298)
 template <class RT>
@@ -189,7 +203,9 @@ __device__ __forceinline__ void fluxes2(const RT (&U)[4], const Inst& in, RT (&x
         split_c32(vy * (U[3] + P), U[3], z1, z2, z3, yp[3], ym[3]);
     } else {
         Prim2<RT> q;
-        if (__builtin_expect(!ref_prim2<RT>(U, in, q), 0)) ref_prim2_exact<RT>(U, in, q);
+        bool tiny = false;
+        const bool ok = ref_prim2<RT>(U, in, q, tiny);
+        if (__builtin_expect(!ok || tiny, 0)) ref_prim2_redo<RT>(U, in, ok, q);
         ref_flux2<RT>(U, q, xp, xm, yp, ym);
         a = q.a;
     }
