@@ -1049,11 +1049,11 @@ static shll_status engine_create_stream(Engine* E) {
 // (or the few that share a SIMD): about 1.7 us and, per step, T(C) for C cells per lane.  So the
 // shape minimises T(C) x max(1, 0.85 x wavefronts of the fullest SIMD) + t0 / k over the cells
 // per lane and the owned cells W of a segment (16, or whole lines of 32), whose halo leaves
-// k = (64 C - W) / (2 order) steps per launch.  T and t0 in units of T(1): 1, 1.45 (second
-// order 1.3), 2.4, 4.3 and 4 (F64 first order 0.31 and 1.7 us, second order 0.61 and 1.7).
+// k = (64 C - W) / (2 order) steps per launch.  T and t0 in units of T(1): 1, 1.45, 2.4, 4.3 and
+// 4 (F64 first order 0.31 and 1.7 us, second order 0.43 and 1.7).
 // Measured, us per step: F64 first order, 1024 cells: C 1, k 8 0.52, k 16 0.41, k 24 0.37, C 2,
 // k 32 0.56; REF32 20000 cells: C 1, k 16 0.36, k 24 (more segments than SIMDs) 0.43; C32K MC
-// 9973 cells: C 1, k 12 0.55, C 2, k 16 0.66; F64F 65536 cells: C 2, k 16 0.63, C 1, k 8 0.97.
+// 9973 cells: C 1, k 12 0.42, C 2, k 16 0.55; F64F 65536 cells: C 2, k 16 0.61, C 1, k 8 0.8.
 // Single instances launch directly: a launch of 6 us or more outlasts its submission, and graph
 // nodes start 2-3% later.
 // Beyond, throughput decides (shape C,k,waves per block): batches of 4.2e5 and 5.9e6 cells, ms:
@@ -1070,7 +1070,7 @@ static void default_launch1d(Engine* E, int64_t max_cells) {
     const bool f64 = word_bytes(E->prec) == 8;
     E->L.graph = E->batch ? 128 : 256;
     if (cells <= 65536) {
-        const double T[4] = {1.0, E->order == 1 ? 1.45 : 1.3, 2.4, 4.3};
+        static const double T[4] = {1.0, 1.45, 2.4, 4.3};
         const int64_t simds = simd_count(E);
         double best = 1e300;
         E->L.wpb = 1;
