@@ -469,18 +469,22 @@ static int default_rows2d(const Engine* E, int k) {
     return best;
 }
 
-// 2D first order: rows of the register tiles, 0 for the row pipelines, which FP64 keeps at 1 and
-// 2 steps per launch on domains whose two state buffers exceed the last-level cache (4096^2, us
-// per step at k = 2: pipeline 172, tiles 192; 2048^2, in the cache: 58 and 51).  An item is one
-// tile, whatever rows the launch shape asks for.
-static bool in_cache(const Engine* E) {
+// bytes of the two state buffers
+static int64_t state_bytes(const Engine* E) {
     int64_t cells = 0;
     for (int64_t c : E->inst_cells) cells += c;
-    return cells * 2 * E->nv * (int64_t)(word_bytes(E->prec) * nwords(E->prec)) <= (256LL << 20);
+    return cells * 2 * E->nv * (int64_t)(word_bytes(E->prec) * nwords(E->prec));
 }
+// they fit the last-level cache
+static bool in_cache(const Engine* E) { return state_bytes(E) <= (256LL << 20); }
+// 2D first order: rows of the register tiles, 0 for the row pipelines, which FP64 keeps at 1 and
+// 2 steps per launch on domains well beyond the last-level cache (us per step at k = 2, pipeline
+// and tiles: 2048^2, 256 MB, 58 and 38; 2500^2, 400 MB, 66 and 61; 3072^2, 604 MB, 86 and 90;
+// 4096^2 147 and 151; 8192^2 530 and 588).  An item is one tile, whatever rows the launch shape
+// asks for.
 static int pick_tile2d(const Engine* E) {
     if (E->dim != 2 || E->order != 1) return 0;
-    if (E->prec == SHLL_F64 && E->L.k <= 2 && !in_cache(E)) return 0;
+    if (E->prec == SHLL_F64 && E->L.k <= 2 && state_bytes(E) > (448LL << 20)) return 0;
     return tile2d_rows(
         E->prec, E->L.k,
         [](const void* e, int rows) { return items2d((const Engine*)e, ((const Engine*)e)->L.k, rows); }, E);
@@ -1117,7 +1121,7 @@ static void default_launch(Engine* E, int64_t max_cells) {
         // domains, where a launch costs as much as its steps, and 2 (F64 in between 3) on large
         // ones, whose halo costs more than the traffic it saves.  Measured, us per step at 2, 3
         // and 4: REF32 256^2 2.6, 2.2, 1.9, 400^2 2.8, 3.0, 2.8, 800^2 5.6, 5.7, -; F64 300^2
-        // 3.5, 2.9, 2.7, 500^2 4.5, 3.9, 5.7, 1024^2 13.8, 13.4, -, 1531x2049 38, 39, 41.
+        // 3.3, 2.9, 2.6, 500^2 4.4, 3.8, -, 700^2 6.9, 6.9, 8.0, 1024^2 12.1, 13.1, -, 1531x2049 30, 33, -.
         // Second order: one step per launch, but C32K takes two on domains whose state exceeds
         // the last-level cache, where one step is bound by HBM (us per step, 1 and 2 steps per
         // launch: 1024^2 16.4 and 32.2, 2048^2 55 and 58, 3072^2 163 and 108); the TwoSum form's
@@ -1128,7 +1132,7 @@ static void default_launch(Engine* E, int64_t max_cells) {
         E->L.C = 1;
         if (E->order == 2) E->L.k = E->prec == SHLL_C32K && !in_cache(E) ? 2 : 1;
         else if (comp || cells < 150000) E->L.k = 4;
-        else E->L.k = E->prec == SHLL_F64 && cells < 1500000 ? 3 : 2;
+        else E->L.k = E->prec == SHLL_F64 && cells < 500000 ? 3 : 2;
         E->L.wpb = 4;
         E->L.rows = default_rows2d(E, E->L.k);
         // first-order launches of a single instance last 7 us or more and are submitted directly

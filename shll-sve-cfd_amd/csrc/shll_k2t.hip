@@ -15,7 +15,7 @@
 // chain of k stages per row and few wavefronts on a small domain; the RW rows of a tile's
 // wavefront are independent chains, and a domain gives a wavefront per RW rows and strip.
 // Measured, us per step before (row pipelines, their default items) and now: REF32 128^2 27 and
-// 1.9, 2048^2 45 and 26; FP64 700^2 32 and 7.1, 1531x2049 45 and 38; C32K 600^2 28 and 4.6,
+// 1.8, 2048^2 45 and 24; FP64 700^2 32 and 6.9, 1531x2049 45 and 30; C32K 600^2 28 and 4.6,
 // 1500^2 29 and 13, 4096^2 104 and 74; C32 4096^2 151 and 112.  A pipeline of k wavefronts that
 // hand rows on through LDS (one stage each, a barrier per row) was slower: C32K 4096^2 107,
 // FP64 1531x2049 48.
@@ -117,9 +117,20 @@ struct Tile2 {
         }
         __syncthreads();
         const int wb = wib > 0 ? wib - 1 : 0, wa = wib + 1 < W ? wib + 1 : W - 1;
+        // reference forms: all reads ahead of the updates; read one variable at a time they cost
+        // 143 registers instead of 126 (FP64), and so the second block of 16 rows on a CU
+        RT near[CMP ? 1 : 4][2];
+        if constexpr (!CMP) {
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                near[v][0] = *slot(parity, wb, 1, v);
+                near[v][1] = *slot(parity, wa, 0, v);
+            }
+        }
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            const RT below = *slot(parity, wb, 1, v), above = *slot(parity, wa, 0, v);
+            const RT below = CMP ? *slot(parity, wb, 1, v) : near[CMP ? 0 : v][0];
+            const RT above = CMP ? *slot(parity, wa, 0, v) : near[CMP ? 0 : v][1];
             if constexpr (CMP) {
                 RT t[RW + 1];  // face terms between rows f-1 and f
 #pragma unroll
@@ -256,18 +267,23 @@ __global__ __launch_bounds__(64 * W) void k_tile2d(StepArgs a) {
 // gives more blocks: the tallest whose tiles number at least `blocks` is taken, else the
 // shortest (16 rows; with 8 steps per launch the next one, since 2k halo rows must leave owned
 // ones).  Measured, us per step: C32K, k = 4: 300^2 16 rows 2.0, 32 rows 2.9; 500^2 3.6 and 3.1;
-// 1024^2 32 rows 8.2, 40 rows 8.5; 1500^2 13.9 and 13.0; 4096^2 82 and 74.  FP64, k = 2-4: 300^2
-// 16 rows 2.7, 24 rows 3.4; 500^2 5.1 and 3.9.  REF32: 24 rows gain nothing up to 4096^2 (97 and
-// 96); C32 spills at 40 rows (4096^2 32 rows 112, 40 rows 142), FP64 at 32.
+// 1024^2 32 rows 8.2, 40 rows 8.5; 1500^2 13.9 and 13.0; 4096^2 82 and 74.  REF32: 24 rows gain
+// nothing up to 4096^2 (97 and 96); C32 spills at 40 rows (4096^2 32 rows 112, 40 rows 142).
+// FP64 tiles of 16 rows hold two blocks on a CU (126 registers), of 24 rows one, so 24 rows win
+// where their tiles fill the CUs once or twice (k = 3, 16 and 24 rows: 300^2 2.9 and 3.6, 500^2
+// 4.4 and 3.8, 700^2 7.3 and 6.9) and lose beyond (1024^2 13.0 and 13.6, 2048^2 42 and 44; k = 2:
+// 12.1 and 13.6, 38 and 45), but for the halo of 4 steps, which leaves 8 of 16 rows (4096^2 189
+// and 183).  Tiles of 32 rows, one block of 16 wavefronts, k = 2 and 3: 1024^2 13.7 and 12.7,
+// 2048^2 42 and 40, behind the two blocks of 16 rows at k = 2.
 // ---------------------------------------------------------------------------
 struct TileRows {
-    int rows, blocks;
+    int rows, blocks, most;  // from `blocks` tiles on; up to `most` (0: any) at less than 4 steps
 };
 static const TileRows* tile_rows(int prec) {
-    static const TileRows f64[] = {{24, 200}, {16, 0}, {0, 0}};
-    static const TileRows ref32[] = {{24, 1 << 30}, {16, 0}, {0, 0}};
-    static const TileRows c32[] = {{32, 150}, {16, 0}, {0, 0}};
-    static const TileRows c32k[] = {{40, 1000}, {32, 150}, {16, 0}, {0, 0}};
+    static const TileRows f64[] = {{24, 200, 500}, {16, 0, 0}, {0, 0, 0}};
+    static const TileRows ref32[] = {{24, 1 << 30, 0}, {16, 0, 0}, {0, 0, 0}};
+    static const TileRows c32[] = {{32, 150, 0}, {16, 0, 0}, {0, 0, 0}};
+    static const TileRows c32k[] = {{40, 1000, 0}, {32, 150, 0}, {16, 0, 0}, {0, 0, 0}};
     return prec == PREC_F64 ? f64 : prec == PREC_REF32 ? ref32 : prec == PREC_C32 ? c32 : c32k;
 }
 
@@ -278,7 +294,8 @@ int tile2d_rows(int prec, int k, int64_t (*tiles)(const void*, int), const void*
     for (const TileRows* t = tile_rows(prec); t->rows > 0; ++t) {
         if (t->rows <= 2 * k) break;
         rows = t->rows;
-        if (tiles(arg, rows - 2 * k) >= t->blocks) break;
+        const int64_t n = tiles(arg, rows - 2 * k);
+        if (n >= t->blocks && (t->most == 0 || n <= t->most || k >= 4)) break;
     }
     return rows;
 }

@@ -30,3 +30,12 @@ def test_taller_tiles(orc, prec, shape, k):
     ic = icgen.random_2d(*shape, 11, block=7)
     banner("tall tiles", prec, shape, k)
     assert_same(pb, gpu_run(pb, ic, k + 2, (1, k, 4, 0)), oracle_run(orc, pb, ic, k + 2), "tall tiles")
+
+
+@pytest.mark.parametrize("k", [2, 3, 4])
+def test_f64_heights_on_many_tiles(orc, k):
+    """More tiles of 24 rows than twice the compute units: 16 rows below 4 steps per launch."""
+    pb = S.problem(2, 1, 1003, 701, precision=S.F64, lx=1.0, ly=701 / 1003)
+    ic = icgen.random_2d(1003, 701, 12, block=7)
+    banner("F64 heights", k)
+    assert_same(pb, gpu_run(pb, ic, 2 * k + 1, (1, k, 4, 0)), oracle_run(orc, pb, ic, 2 * k + 1), "F64 heights")
