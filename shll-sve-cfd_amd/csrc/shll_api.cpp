@@ -29,7 +29,7 @@ int step1d_items_per_block(int C, int wpb);
 hipError_t launch_step2d(int prec, int order, int lim, int k, int wpb, int n_items, hipStream_t s,
                          const StepArgs& a);
 bool step2d_supported(int prec, int order, int k);
-int tile2d_rows(int prec, int k, int64_t (*tiles)(const void*, int), const void* arg);
+int tile2d_rows(int prec, int k, int cus, int64_t (*tiles)(const void*, int), const void* arg);
 hipError_t launch_tile2d(int prec, int rows, int n_items, hipStream_t s, const StepArgs& a);
 hipError_t launch_init(int prec, int dim, int nblocks, int n_inst, hipStream_t st, const Inst* insts,
                        const double* prim, void* o0, void* o1, int64_t plane);
@@ -486,7 +486,7 @@ static int pick_tile2d(const Engine* E) {
     if (E->dim != 2 || E->order != 1) return 0;
     if (E->prec == SHLL_F64 && E->L.k <= 2 && state_bytes(E) > (448LL << 20)) return 0;
     return tile2d_rows(
-        E->prec, E->L.k,
+        E->prec, E->L.k, (int)(simd_count(E) / 4),
         [](const void* e, int rows) { return items2d((const Engine*)e, ((const Engine*)e)->L.k, rows); }, E);
 }
 

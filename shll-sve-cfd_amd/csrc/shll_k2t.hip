@@ -15,7 +15,7 @@
 // chain of k stages per row and few wavefronts on a small domain; the RW rows of a tile's
 // wavefront are independent chains, and a domain gives a wavefront per RW rows and strip.
 // Measured, us per step before (row pipelines, their default items) and now: REF32 128^2 27 and
-// 1.8, 2048^2 45 and 24; FP64 700^2 32 and 6.9, 1531x2049 45 and 30; C32K 600^2 28 and 4.6,
+// 1.5, 2048^2 45 and 24; FP64 700^2 32 and 6.9, 1531x2049 45 and 30; C32K 600^2 28 and 4.6,
 // 1500^2 29 and 13, 4096^2 104 and 74; C32 4096^2 151 and 112.  A pipeline of k wavefronts that
 // hand rows on through LDS (one stage each, a barrier per row) was slower: C32K 4096^2 107,
 // FP64 1531x2049 48.
@@ -263,39 +263,48 @@ __global__ __launch_bounds__(64 * W) void k_tile2d(StepArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// Tile heights (rows = RW * W), by precision.  A taller tile recomputes less halo, a shorter one
-// gives more blocks: the tallest whose tiles number at least `blocks` is taken, else the
-// shortest (16 rows; with 8 steps per launch the next one, since 2k halo rows must leave owned
-// ones).  Measured, us per step: C32K, k = 4: 300^2 16 rows 2.0, 32 rows 2.9; 500^2 3.6 and 3.1;
-// 1024^2 32 rows 8.2, 40 rows 8.5; 1500^2 13.9 and 13.0; 4096^2 82 and 74.  REF32: 24 rows gain
-// nothing up to 4096^2 (97 and 96); C32 spills at 40 rows (4096^2 32 rows 112, 40 rows 142).
-// FP64 tiles of 16 rows hold two blocks on a CU (126 registers), of 24 rows one, so 24 rows win
-// where their tiles fill the CUs once or twice (k = 3, 16 and 24 rows: 300^2 2.9 and 3.6, 500^2
-// 4.4 and 3.8, 700^2 7.3 and 6.9) and lose beyond (1024^2 13.0 and 13.6, 2048^2 42 and 44; k = 2:
-// 12.1 and 13.6, 38 and 45), but for the halo of 4 steps, which leaves 8 of 16 rows (4096^2 189
-// and 183).  Tiles of 32 rows, one block of 16 wavefronts, k = 2 and 3: 1024^2 13.7 and 12.7,
-// 2048^2 42 and 40, behind the two blocks of 16 rows at k = 2.
+// Tile heights (rows = RW * W), by precision: the first of the list that the number of its tiles
+// allows, else the last that leaves owned rows beside the 2k of the halo.  Measured, us per step.
+//
+// 12 rows, one per wavefront, while its tiles find a compute unit each: a block's step is bound
+// by the issue of its own SIMDs, so fewer rows to a block are a shorter step (k = 4, 16 and 12
+// rows: 128^2 REF32 1.74 and 1.51, FP64 2.48 and 1.98, C32K 1.72 and 1.50, C32 2.31 and 1.82;
+// 180^2 REF32 1.75 and 1.56; 256^2, more tiles than units, 1.77 and 2.19).  16 rows of one per
+// wavefront are no better than of two (1.75).
+//
+// Then a taller tile recomputes less halo and a shorter one gives more blocks.  C32K, k = 4:
+// 300^2 16 rows 2.0, 32 rows 2.9; 500^2 3.6 and 3.1; 1024^2 32 rows 8.2, 40 rows 8.5; 1500^2
+// 13.9 and 13.0; 4096^2 82 and 74.  REF32: 24 rows gain nothing up to 4096^2 (97 and 96); C32
+// spills at 40 rows (4096^2 32 rows 112, 40 rows 142).  FP64 tiles of 16 rows hold two blocks on
+// a CU (126 registers), of 24 rows one, so 24 rows win where their tiles fill the CUs once or
+// twice (k = 3, 16 and 24 rows: 300^2 2.9 and 3.6, 500^2 4.4 and 3.8, 700^2 7.3 and 6.9) and
+// lose beyond (1024^2 13.0 and 13.6, 2048^2 42 and 44; k = 2: 12.1 and 13.6, 38 and 45), but for
+// the halo of 4 steps, which leaves 8 of 16 rows (4096^2 189 and 183).  FP64 tiles of 32 rows,
+// one block of 16 wavefronts, k = 2 and 3: 1024^2 13.7 and 12.7, 2048^2 42 and 40, behind the
+// two blocks of 16 rows at k = 2.
 // ---------------------------------------------------------------------------
 struct TileRows {
-    int rows, blocks, most;  // from `blocks` tiles on; up to `most` (0: any) at less than 4 steps
+    int rows, least;   // taken from `least` tiles on
+    int most, most4;   // up to this many tiles per compute unit, below 4 steps and from 4 on (0: any)
 };
 static const TileRows* tile_rows(int prec) {
-    static const TileRows f64[] = {{24, 200, 500}, {16, 0, 0}, {0, 0, 0}};
-    static const TileRows ref32[] = {{24, 1 << 30, 0}, {16, 0, 0}, {0, 0, 0}};
-    static const TileRows c32[] = {{32, 150, 0}, {16, 0, 0}, {0, 0, 0}};
-    static const TileRows c32k[] = {{40, 1000, 0}, {32, 150, 0}, {16, 0, 0}, {0, 0, 0}};
+    static const TileRows f64[] = {{12, 0, 1, 1}, {24, 200, 2, 0}, {16, 0, 0, 0}, {0, 0, 0, 0}};
+    static const TileRows ref32[] = {{12, 0, 1, 1}, {24, 1 << 30, 0, 0}, {16, 0, 0, 0}, {0, 0, 0, 0}};
+    static const TileRows c32[] = {{12, 0, 1, 1}, {32, 150, 0, 0}, {16, 0, 0, 0}, {0, 0, 0, 0}};
+    static const TileRows c32k[] = {{12, 0, 1, 1}, {40, 1000, 0, 0}, {32, 150, 0, 0}, {16, 0, 0, 0}, {0, 0, 0, 0}};
     return prec == PREC_F64 ? f64 : prec == PREC_REF32 ? ref32 : prec == PREC_C32 ? c32 : c32k;
 }
 
-// rows of the tiles for k steps per launch, 0 if none fits; tiles(owned): the number of tiles
-// that own that many rows
-int tile2d_rows(int prec, int k, int64_t (*tiles)(const void*, int), const void* arg) {
+// rows of the tiles for k steps per launch on cus compute units, 0 if none fits; tiles(owned):
+// the number of tiles that own that many rows
+int tile2d_rows(int prec, int k, int cus, int64_t (*tiles)(const void*, int), const void* arg) {
     int rows = 0;
     for (const TileRows* t = tile_rows(prec); t->rows > 0; ++t) {
-        if (t->rows <= 2 * k) break;
+        if (t->rows <= 2 * k) continue;
         rows = t->rows;
         const int64_t n = tiles(arg, rows - 2 * k);
-        if (n >= t->blocks && (t->most == 0 || n <= t->most || k >= 4)) break;
+        const int most = k < 4 ? t->most : t->most4;
+        if (n >= t->least && (most == 0 || n <= (int64_t)most * cus)) break;
     }
     return rows;
 }
@@ -311,12 +320,16 @@ hipError_t launch_tile2d(int prec, int rows, int n_items, hipStream_t s, const S
     const int nblocks = xcd_grid(n_items);
     if (nblocks <= 0) return hipSuccess;
     switch (prec * 64 + rows) {
+    case PREC_F64 * 64 + 12: return launch_tile<PREC_F64, 1, 12>(nblocks, s, a);
     case PREC_F64 * 64 + 16: return launch_tile<PREC_F64, 2, 8>(nblocks, s, a);
     case PREC_F64 * 64 + 24: return launch_tile<PREC_F64, 2, 12>(nblocks, s, a);
+    case PREC_REF32 * 64 + 12: return launch_tile<PREC_REF32, 1, 12>(nblocks, s, a);
     case PREC_REF32 * 64 + 16: return launch_tile<PREC_REF32, 2, 8>(nblocks, s, a);
     case PREC_REF32 * 64 + 24: return launch_tile<PREC_REF32, 2, 12>(nblocks, s, a);
+    case PREC_C32 * 64 + 12: return launch_tile<PREC_C32, 1, 12>(nblocks, s, a);
     case PREC_C32 * 64 + 16: return launch_tile<PREC_C32, 2, 8>(nblocks, s, a);
     case PREC_C32 * 64 + 32: return launch_tile<PREC_C32, 4, 8>(nblocks, s, a);
+    case PREC_C32K * 64 + 12: return launch_tile<PREC_C32K, 1, 12>(nblocks, s, a);
     case PREC_C32K * 64 + 16: return launch_tile<PREC_C32K, 2, 8>(nblocks, s, a);
     case PREC_C32K * 64 + 32: return launch_tile<PREC_C32K, 4, 8>(nblocks, s, a);
     case PREC_C32K * 64 + 40: return launch_tile<PREC_C32K, 5, 8>(nblocks, s, a);

@@ -39,3 +39,25 @@ def test_f64_heights_on_many_tiles(orc, k):
     ic = icgen.random_2d(1003, 701, 12, block=7)
     banner("F64 heights", k)
     assert_same(pb, gpu_run(pb, ic, 2 * k + 1, (1, k, 4, 0)), oracle_run(orc, pb, ic, 2 * k + 1), "F64 heights")
+
+
+@pytest.mark.parametrize("prec", [S.F64, S.REF32, S.C32, S.C32K])
+@pytest.mark.parametrize("shape,k", [((10, 62), 1), ((11, 63), 1), ((8, 61), 2), ((17, 66), 2), ((6, 64), 3), ((13, 59), 3),
+                                     ((4, 60), 4), ((5, 57), 4), ((9, 121), 4)])
+def test_one_row_per_wavefront(orc, prec, shape, k):
+    """Few tiles: 12 rows, of which 12 - 2k are owned, at one row or column more or less."""
+    pb = S.problem(2, 1, *shape, precision=prec, lx=1.0, ly=shape[1] / shape[0])
+    ic = icgen.random_2d(*shape, 5 + k, block=3)
+    banner("12 rows", prec, shape, k)
+    assert_same(pb, gpu_run(pb, ic, 2 * k + 1, (1, k, 4, 0)), oracle_run(orc, pb, ic, 2 * k + 1), "12 rows")
+
+
+@pytest.mark.parametrize("prec", [S.F64, S.REF32, S.C32, S.C32K])
+@pytest.mark.parametrize("shape,k", [((2049, 3), 4), ((4321, 4), 1), ((4001, 5), 2), ((6017, 3), 4), ((9000, 3), 3),
+                                     ((9300, 3), 3), ((32001, 2), 4)])
+def test_heights_of_long_domains(orc, prec, shape, k):
+    """Many tiles of a few columns: the taller tiles, with a last one of few rows."""
+    pb = S.problem(2, 1, *shape, precision=prec, lx=1.0, ly=shape[1] / shape[0])
+    ic = icgen.random_2d(*shape, 6 + k, block=5)
+    banner("long", prec, shape, k)
+    assert_same(pb, gpu_run(pb, ic, k + 1, (1, k, 4, 0)), oracle_run(orc, pb, ic, k + 1), "long domains")
