@@ -111,10 +111,19 @@ def bytes_per_update(dim, prec):
     return 2 * nv * s
 
 
+def kernel_first_order_2d(prec, lau):
+    """The first-order kernel of the benchmark's 2D problems (FP64 states beyond the last-level
+    cache: the row pipeline)."""
+    import shll_amd as S
+    if prec == S.F64 and lau[1] <= 2:
+        return "shll::k_step2d_tb<%d, %d> (first order, %d steps per launch)" % (lau[1], lau[2], lau[1])
+    return "shll::k_tile2d<%d, ...> (first order, register tiles, %d steps per launch)" % (prec, lau[1])
+
+
 def rows_per_item(lau):
-    """2D: owned rows per work item of a launch shape (its first value; 0 or 1: the
-    default for its steps per launch)."""
-    return lau[0] if lau[0] > 1 else {1: 16, 2: 32}.get(lau[1], 64)
+    """2D: owned rows per work item that a launch shape asks for (its first value; None: the
+    library's own choice)."""
+    return lau[0] if lau[0] > 1 else None
 
 
 def profile_figure(summary, key, shape):
@@ -703,8 +712,7 @@ def main_domains(S, args):
                "nonfinite_domains": int((b.check_state() > 0).sum() + (ref.check_state() > 0).sum())}
         ref.close()
     b.close()
-    kern = ("shll::k_step2d_tb<%d, %d, %d> (first order, %d steps per launch)" % (prec, lau[1], lau[2], lau[1])
-            if lau[1] > 1 else "shll::k_step2d<%d, 1, %d, 0>" % (prec, lau[2]))
+    kern = kernel_first_order_2d(prec, lau)
     result = {
         "metric": METRIC, "value": upd / wall, "unit": "cell-updates/s", "n_gpus": 1, "steps": K,
         "warmup": args.warmup, "ms_per_step": wall * 1e3 / K, "higher_is_better": True, "scaling": "weak",
@@ -824,8 +832,7 @@ def main_circle4096(S, args):
     s.close()
     B = bytes_per_update(2, prec)
     k = lau[1]
-    kern = ("shll::k_step2d_tb<%d, %d, %d> (first order, %d steps per launch)" % (prec, k, lau[2], k)
-            if k > 1 else "shll::k_step2d<%d, 1, %d, 0>" % (prec, lau[2]))
+    kern = kernel_first_order_2d(prec, lau)
     tag = ("k_step2d_tb_%s_circle4096" % form) if k > 1 else ("k_step2d_%s_circle4096" % form)
     result = {
         "metric": METRIC, "value": upd / wall, "unit": "cell-updates/s", "n_gpus": 1, "steps": K,
@@ -886,7 +893,7 @@ def main_omp2d(S, args, ref_cpu):
     s.close()
     B = bytes_per_update(2, prec)
     k = lau[1]
-    kern = ("shll::k_step2d<%d, 2, %d, 1> (second order, MC limiter, one step per launch)" % (prec, lau[2])
+    kern = ("shll::k_row2d<%d, %d, 1> (second order, MC limiter, one step per launch)" % (prec, lau[2])
             if k == 1 else "shll::k_step2d_tb2<%d, 2, %d, 1> (second order, MC limiter, 2 steps per launch)"
             % (prec, lau[2]))
     tag = "k_step2d_%s_o2_mc1024" % form if k == 1 else "k_step2d_tb2_%s_o2_mc1024" % form
