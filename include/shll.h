@@ -176,7 +176,7 @@ void shll_free(shll_ctx *ctx);
 /* Launch shape of the step kernels.  cells_per_lane: 1D in {1,2,4,8}; 2D the owned rows
  * of a work item, the cells of its column each lane owns (2-4096; 0 or 1: the library's
  * choice; first-order items are register tiles of the library's height whatever is asked
- * for, except in SHLL_F64 at 1 or 2 steps per launch on more than about 4e6 cells),
+ * for, except in SHLL_F64 at 1 or 2 steps per launch on more than about 7e6 cells),
  * steps_per_launch >= 1 (temporal blocking; 2D: 1, 2, 3, 4 or 8 in first order; 1, or 2 for
  * SHLL_C32/SHLL_C32K in second order),
  * waves_per_block in {1,4} (1D, 4 with 2+ cells per lane: the block's wavefronts hold
@@ -192,8 +192,9 @@ shll_status shll_get_launch(const shll_ctx *ctx, int32_t out[4]);
  * $SHLL_TUNE_CACHE (if set).  Candidates: 1D cells per lane 1-8, 1-64 steps per launch,
  * 1 or 4 waves per block (and 256-4096 steps per launch when the whole tube fits one
  * segment or block, which then has no halo); 2D the valid steps per launch, 1 or 4
- * waves per block, work items of 3/4, 5/4 and 3/2 of the default rows, and shorter ones
- * (down to 1/8) when the default ones give fewer than 4 wavefronts per SIMD; graphs of
+ * waves per block, and where items have a height of their own (second order, and SHLL_F64
+ * in first order) 3/4, 5/4 and 3/2 of the default rows, and shorter ones (down to 1/8)
+ * when the default ones give fewer than 4 wavefronts per SIMD; graphs of
  * 128 (2D: 64) steps, or two launches if longer, and for a single instance also of 2048
  * (2D: 1024) steps and direct launches (graph_steps 0). */
 shll_status shll_autotune(shll_ctx *ctx, int32_t trial_steps);
