@@ -502,6 +502,80 @@ __device__ __forceinline__ void step_f64f(double (&u)[3][C], const Inst& in, int
 }
 
 // ---------------------------------------------------------------------------
+// A wavefront's 64*C cells between memory, where lane i moves cells i, 64 + i, ..., and the
+// registers, where lane i holds cells C*i .. C*i + C - 1: through a slab of LDS of its own, C
+// cells to a row of C + 1 (the odd row spreads the banks).  A wavefront's LDS accesses are
+// carried out in order, so one slab serves variable after variable without a wait or barrier;
+// the fences keep the compiler to that order.
+//
+// Where (ON): lanes that load and store their own cells touch a cache line each per access, C
+// times the lines a moved row touches.  With 8 doubles, 64 bytes from lane to lane, that held
+// up the start and end of every item: batch of 400 tubes, second order F64F, 85.5 ms so, 78.2
+// through LDS; first order 78.7 and 53.8; F64 second order 67.8 and 64.3.  With 4 doubles (32
+// bytes) both take the same (F64 62.1 and 61.9, F64F 77.9 and 77.4), with 2 or 1 and in the
+// 32-bit forms too or the LDS way is the slower one (65536-cell tube, F64, 0.835 and 0.845 us
+// per step; C32 in blocks of four 45.3 and 47.0), so those keep their own accesses.
+// ---------------------------------------------------------------------------
+template <class RT, int C>
+struct Turn {
+    static constexpr bool ON = sizeof(RT) == 8 && C == 8;
+    static constexpr int SLAB = ON ? 64 * (C + 1) : 1;
+    __device__ static __forceinline__ void fence() {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+    __device__ static __forceinline__ int pos(int i) { return i + i / C; }
+    // cells gw .. gw + 64 C - 1 of three planes P apart; those off the domain [0, n) get a state at rest
+    __device__ static __forceinline__ void load(const RT* __restrict__ p, int64_t P, int gw, int n, int lane, RT* slab,
+                                                RT (&u)[3][C]) {
+        if (gw >= 0 && gw + 64 * C <= n) {
+#pragma unroll
+            for (int v = 0; v < 3; ++v)
+#pragma unroll
+                for (int m = 0; m < C; ++m) u[v][m] = p[v * P + (gw + m * 64 + lane)];
+        } else {
+#pragma unroll
+            for (int m = 0; m < C; ++m) {
+                const int g = gw + m * 64 + lane;
+                const bool ok = g >= 0 && g < n;
+#pragma unroll
+                for (int v = 0; v < 3; ++v) u[v][m] = ok ? p[v * P + g] : (RT)(v == 0 ? 1.0 : (v == 1 ? 0.0 : 2.5));
+            }
+        }
+#pragma unroll
+        for (int v = 0; v < 3; ++v) {
+#pragma unroll
+            for (int m = 0; m < C; ++m) slab[pos(m * 64 + lane)] = u[v][m];
+            fence();
+#pragma unroll
+            for (int m = 0; m < C; ++m) u[v][m] = slab[lane * (C + 1) + m];
+            fence();
+        }
+    }
+    // the item's owned cells
+    __device__ static __forceinline__ void store(RT* __restrict__ p, int64_t P, const Item1& it, int gw, int lane,
+                                                 RT* slab, RT (&u)[3][C]) {
+#pragma unroll
+        for (int v = 0; v < 3; ++v) {
+#pragma unroll
+            for (int m = 0; m < C; ++m) slab[lane * (C + 1) + m] = u[v][m];
+            fence();
+#pragma unroll
+            for (int m = 0; m < C; ++m) u[v][m] = slab[pos(m * 64 + lane)];
+            fence();
+        }
+#pragma unroll
+        for (int m = 0; m < C; ++m) {
+            const int g = gw + m * 64 + lane;
+            if (g >= it.x0 && g < it.x0 + it.w) {
+#pragma unroll
+                for (int v = 0; v < 3; ++v) p[v * P + g] = u[v][m];
+            }
+        }
+    }
+};
+
+// ---------------------------------------------------------------------------
 // ns steps of one segment from registers, then the owned cells back to HBM.  Each
 // wall mode gets its own copy of loop and store, so the loop-carried state never
 // has to be moved between the copies' registers.
@@ -528,7 +602,7 @@ __device__ __forceinline__ void advance_c32(float (&hi)[3][C], float (&lo)[3][C]
 
 template <int ORDER, int C, int WM, int LIM, int XW>
 __device__ __forceinline__ void advance_f64f(double (&u)[3][C], const Inst& in, const Item1& it, int gl, int ns,
-                                             const StepArgs& a, const Coop<double, XW>& x) {
+                                             const StepArgs& a, const Coop<double, XW>& x, double* slab) {
     // the limiter's clamped form (F64FArith) where it holds for the whole launch: second order,
     // density and energy of every cell in [2^-200, 2^400] and at most 64 steps, so that no flux
     // reaches 2^512 or falls where scaling it by 2^-512 costs digits
@@ -543,6 +617,10 @@ __device__ __forceinline__ void advance_f64f(double (&u)[3][C], const Inst& in, 
     }
     double* __restrict__ ou = (double*)a.out0 + in.off;
     const int64_t P = a.plane;
+    if constexpr (Turn<double, C>::ON) {
+        Turn<double, C>::store(ou, P, it, gl - x.lane * C, x.lane, slab, u);
+        return;
+    }
 #pragma unroll
     for (int m = 0; m < C; ++m) {
         const int g = gl + m;
@@ -556,11 +634,16 @@ __device__ __forceinline__ void advance_f64f(double (&u)[3][C], const Inst& in, 
 template <int PREC, int ORDER, int C, int WM, int LIM, int XW>
 __device__ __forceinline__ void advance_ref(typename Real<PREC>::T (&u)[3][C], const Inst& in, const Item1& it,
                                             int gl, int ns, const StepArgs& a,
-                                            const Coop<typename Real<PREC>::T, XW>& x) {
+                                            const Coop<typename Real<PREC>::T, XW>& x,
+                                            typename Real<PREC>::T* slab) {
     using RT = typename Real<PREC>::T;
     for (int s = 0; s < ns; ++s) step_ref<PREC, ORDER, C, WM, LIM, XW>(u, in, gl, x, s & 1);
     RT* __restrict__ ou = (RT*)a.out0 + in.off;
     const int64_t P = a.plane;
+    if constexpr (Turn<RT, C>::ON) {
+        Turn<RT, C>::store(ou, P, it, gl - x.lane * C, x.lane, slab, u);
+        return;
+    }
 #pragma unroll
     for (int m = 0; m < C; ++m) {
         const int g = gl + m;
@@ -591,7 +674,9 @@ void k_step1d(StepArgs a) {
     // per block, one segment of 64*C cells per wavefront
     constexpr int XW = WPB > 1 && C >= 2 ? WPB : 1;
     __shared__ __align__(16) RT xlds[XW > 1 ? 2 * XW * CoopSlots<RT>::WAVE : 1];
+    __shared__ RT slabs[WPB * Turn<RT, C>::SLAB];
     const int wib = uniform((int)threadIdx.x >> 6);
+    RT* const slab = slabs + wib * Turn<RT, C>::SLAB;
     const LaunchView lv = launch_view(a);
     constexpr int IPB = XW > 1 ? 1 : WPB;  // items per block
     const int blk = xcd_work((int)blockIdx.x, (lv.n_items + IPB - 1) / IPB);
@@ -636,21 +721,25 @@ void k_step1d(StepArgs a) {
     } else {
         const RT* __restrict__ iu = (const RT*)a.in0 + in.off;
         RT u[3][C];
+        if constexpr (Turn<RT, C>::ON) {
+            Turn<RT, C>::load(iu, P, gw, n, lane, slab, u);
+        } else {
 #pragma unroll
-        for (int m = 0; m < C; ++m) {
-            const int g = gl + m;
-            const bool ok = g >= 0 && g < n;
+            for (int m = 0; m < C; ++m) {
+                const int g = gl + m;
+                const bool ok = g >= 0 && g < n;
 #pragma unroll
-            for (int v = 0; v < 3; ++v) u[v][m] = ok ? iu[v * P + g] : (RT)(v == 0 ? 1.0 : (v == 1 ? 0.0 : 2.5));
+                for (int v = 0; v < 3; ++v) u[v][m] = ok ? iu[v * P + g] : (RT)(v == 0 ? 1.0 : (v == 1 ? 0.0 : 2.5));
+            }
         }
         if constexpr (PREC == PREC_F64F) {
-            if (wm == WM_NONE) advance_f64f<ORDER, C, WM_NONE, LIM, XW>(u, in, it, gl, ns, a, x);
-            else if (ORDER == 1 || wm == WM_GHOST) advance_f64f<ORDER, C, WM_GHOST, LIM, XW>(u, in, it, gl, ns, a, x);
-            else advance_f64f<ORDER, C, WR, LIM, XW>(u, in, it, gl, ns, a, x);
+            if (wm == WM_NONE) advance_f64f<ORDER, C, WM_NONE, LIM, XW>(u, in, it, gl, ns, a, x, slab);
+            else if (ORDER == 1 || wm == WM_GHOST) advance_f64f<ORDER, C, WM_GHOST, LIM, XW>(u, in, it, gl, ns, a, x, slab);
+            else advance_f64f<ORDER, C, WR, LIM, XW>(u, in, it, gl, ns, a, x, slab);
         } else {
-            if (wm == WM_NONE) advance_ref<PREC, ORDER, C, WM_NONE, LIM, XW>(u, in, it, gl, ns, a, x);
-            else if (ORDER == 1 || wm == WM_GHOST) advance_ref<PREC, ORDER, C, WM_GHOST, LIM, XW>(u, in, it, gl, ns, a, x);
-            else advance_ref<PREC, ORDER, C, WR, LIM, XW>(u, in, it, gl, ns, a, x);
+            if (wm == WM_NONE) advance_ref<PREC, ORDER, C, WM_NONE, LIM, XW>(u, in, it, gl, ns, a, x, slab);
+            else if (ORDER == 1 || wm == WM_GHOST) advance_ref<PREC, ORDER, C, WM_GHOST, LIM, XW>(u, in, it, gl, ns, a, x, slab);
+            else advance_ref<PREC, ORDER, C, WR, LIM, XW>(u, in, it, gl, ns, a, x, slab);
         }
     }
 }
