@@ -359,8 +359,7 @@ static void tile2d(int32_t inst, int64_t nx, int64_t ny, int order, int k, int r
     for (int64_t ix0 = 0; ix0 < nx; ix0 += rows) {
         const int64_t iw = std::min<int64_t>(rows, nx - ix0);
         for (const Strip& s : strips)
-            out.push_back(Item2{inst, s.j0, s.jx0, s.jw, (int32_t)(ix0 - H), (int32_t)ix0, (int32_t)iw,
-                                (int32_t)(iw + 2 * H)});
+            out.push_back(Item2{inst, s.j0, s.jx0, s.jw, (int32_t)ix0, (int32_t)iw});
     }
 }
 

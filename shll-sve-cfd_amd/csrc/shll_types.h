@@ -49,13 +49,12 @@ struct Item1 {
     int32_t w;
 };
 
-// One wavefront's share of a 2D launch: a strip of columns j in [j0, j0 + 64)
-// (owned [jx0, jx0 + jw)) streamed along rows i in [i0, i0 + ilen) (owned
-// [ix0, ix0 + iw)).
+// One wavefront's (tiles: one block's) share of a 2D launch: a strip of columns j in
+// [j0, j0 + 64), owned [jx0, jx0 + jw), and its owned rows [ix0, ix0 + iw).
 struct Item2 {
     int32_t inst;
     int32_t j0, jx0, jw;
-    int32_t i0, ix0, iw, ilen;
+    int32_t ix0, iw;
 };
 
 struct StepArgs {
