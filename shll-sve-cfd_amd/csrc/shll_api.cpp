@@ -1132,7 +1132,11 @@ static void default_launch(Engine* E, int64_t max_cells) {
         if (E->order == 2) E->L.k = E->prec == SHLL_C32K && !in_cache(E) ? 2 : 1;
         else if (comp || cells < 150000) E->L.k = 4;
         else E->L.k = E->prec == SHLL_F64 && cells < 500000 ? 3 : 2;
-        E->L.wpb = 4;
+        // FP64 second order: one wavefront per block, so a block's items need not start together on
+        // one CU (us per step, 4 and 1 per block: 777x613 15.3 and 14.7, 1024^2 22.3 and 22.3,
+        // 3000^2 159.6 and 156.9); the 32-bit forms gain nothing (REF32 777x613 10.3 and 10.5) and
+        // beyond the last-level cache lose (C32 3000^2 149 and 157)
+        E->L.wpb = E->order == 2 && E->prec == SHLL_F64 ? 1 : 4;
         E->L.rows = default_rows2d(E, E->L.k);
         // first-order launches of a single instance last 7 us or more and are submitted directly
         E->L.graph = E->batch || E->order == 2 ? 64 : 0;
