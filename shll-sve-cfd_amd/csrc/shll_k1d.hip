@@ -605,13 +605,16 @@ __device__ __forceinline__ void advance_f64f(double (&u)[3][C], const Inst& in, 
                                              const StepArgs& a, const Coop<double, XW>& x, double* slab) {
     // the limiter's clamped form (F64FArith) where it holds for the whole launch: second order,
     // density and energy of every cell in [2^-200, 2^400] and at most 64 steps, so that no flux
-    // reaches 2^512 or falls where scaling it by 2^-512 costs digits
-    bool unit = ORDER == 2 && ns <= 64;
+    // reaches 2^512 or falls where scaling it by 2^-512 costs digits.  Independent wavefronts only:
+    // those of a cooperative block read each other's fluxes, so all have to scale them alike, and
+    // the general form is the scale that holds for any of them
+    constexpr bool MAY = ORDER == 2 && XW == 1;
+    bool unit = MAY && ns <= 64;
 #pragma unroll
     for (int m = 0; m < C; ++m)
         unit = unit && u[0][m] >= 0x1p-200 && u[0][m] <= 0x1p400 && u[2][m] >= 0x1p-200 && u[2][m] <= 0x1p400;
-    if (ORDER == 2 && __all(unit)) {
-        for (int s = 0; s < ns; ++s) step_f64f<ORDER, C, WM, LIM, XW, ORDER == 2>(u, in, gl, x, s & 1);
+    if (MAY && __all(unit)) {
+        for (int s = 0; s < ns; ++s) step_f64f<ORDER, C, WM, LIM, XW, MAY>(u, in, gl, x, s & 1);
     } else {
         for (int s = 0; s < ns; ++s) step_f64f<ORDER, C, WM, LIM, XW, false>(u, in, gl, x, s & 1);
     }
