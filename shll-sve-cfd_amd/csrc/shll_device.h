@@ -238,17 +238,18 @@ __device__ __forceinline__ double rsq_nr2(double x) {
 //   - (float)sqrt((double)x) of a float x is the float square root (rounding twice is
 //     harmless from 53 to 24 bits), so REF32 takes it in float;
 //   - a quotient of +-0 comes out as +0, a zero whose sign no sum here keeps.
-// Two tests per cell cover all of it:
-//   - the radicand x = gamma R T in [XLO, XHI] (else false: the cell takes prim*_exact).  T > 0
-//     then bounds e = cv T + kin below and a away from the ends of the range; non-finite states
-//     fail here;
-//   - every velocity |v| >= VLO or exactly zero (else *tiny: the caller divides again with the
-//     operator).  Only the velocity itself needs it: with |v| below VLO, M/2 +- 1/2 is +-1/2
-//     and 1 - M^2 is 1 whatever M's last bits, and v^2 vanishes in kin.  Transverse velocities
-//     ahead of a front square from cell to cell (1e-9, 1e-18, 1e-36, 0), so a wavefront that
-//     holds a front nearly always has such a lane: REF32 at 128^2, four steps per launch, 10.7
-//     us with the whole cell redone there, 8.4 us with the divisions only, 7.6 us once the
-//     fronts are gone.
+// A quotient is right to the last bit while it and the reciprocal are normal and its remainder is
+// exact, the dividend 48 (FP64: 106) binary orders above the smallest denormal.  What covers that:
+//   - RefSpan: the radicand x = gamma R T and the density within [LO, HI) (else the cell takes
+//     prim*_exact).  T > 0 then bounds e = cv T + kin below, the energy with it, and a away from
+//     the ends of the range; non-finite states fail here;
+//   - then only a velocity of |M| < 2^-35 (FP64: 2^-500), of a momentum |u| < ULO, can be off: M/2 +-
+//     1/2 is +-1/2 and 1 - M^2 is 1 all the same, and next to the sound speed nothing of it is left
+//     in the fluxes, except in the transverse momentum's (rho u v).  So 2D divides again with the
+//     operator where a momentum is below ULO and not zero (*tiny).  Transverse velocities ahead of a
+//     front square from cell to cell (1e-9, 1e-18, 1e-36, 0), so a wavefront that holds a front
+//     often has such a lane: REF32 at 128^2, four steps per launch, 10.7 us with the whole cell
+//     redone there, 8.4 us with the divisions only, 7.6 us once the fronts are gone.
 // Before, each of the five (2D: seven) operations carried its own compare and branch, and a
 // gas at rest (u = 0) took the slow path of two of them: 1D first order FP64, 1024 cells,
 // 5.43 us per 8-step launch, 4.2 us now; second order, 4 cells per lane: 894 VALU instructions per
@@ -256,10 +257,27 @@ __device__ __forceinline__ double rsq_nr2(double x) {
 // ---------------------------------------------------------------------------
 template <class RT> struct RefRange;
 template <> struct RefRange<double> {
-    static constexpr double XLO = 0x1p-700, XHI = 0x1p+700, VLO = 0x1p-900;
+    static constexpr double ULO = 0x1p-800;
+    static constexpr int LO = (1023 - 200) << 20, HI = (1023 + 200) << 20;  // 2^-200, 2^200
+    __device__ static __forceinline__ int bits(double x) { return __double2hiint(x); }
 };
 template <> struct RefRange<float> {
-    static constexpr float XLO = 0x1p-30f, XHI = 0x1p+60f, VLO = 0x1p-64f;
+    static constexpr float ULO = 0x1p-80f;
+    static constexpr int LO = (127 - 30) << 23, HI = (127 + 40) << 23;  // 2^-30, 2^40
+    __device__ static __forceinline__ int bits(float x) { return __float_as_int(x); }
+};
+// Radicands and densities of any number of cells within [LO, HI): their (high) words as integers,
+// which order like the values; a negative value is below, a NaN below or above.  Two full-rate
+// instructions per cell.
+template <class RT>
+struct RefSpan {
+    using R = RefRange<RT>;
+    int top = R::LO, low = R::LO;
+    __device__ __forceinline__ void take(RT x, RT rho) {
+        top = max(top, max(R::bits(x), R::bits(rho)));
+        low = min(low, min(R::bits(x), R::bits(rho)));
+    }
+    __device__ __forceinline__ bool ok() const { return low >= R::LO && top < R::HI; }
 };
 
 template <class RT>
@@ -276,8 +294,8 @@ struct RefArith {
         a = (RT)sqrt((double)(gR * T));
         M = vx / a;
     }
-    __device__ static __forceinline__ bool prim1_fast(RT u0, RT u1, RT u2, int ke, RT cv, double rcv, RT gR, RT& vx,
-                                                      RT& T, RT& a, RT& M, bool& tiny) {
+    __device__ static __forceinline__ void prim1_fast(RT u0, RT u1, RT u2, int ke, RT cv, double rcv, RT gR, RT& vx,
+                                                      RT& T, RT& a, RT& M, RefSpan<RT>& span) {
         RT y;
         if constexpr (F32) y = rcp_fast(u0);
         else y = rcp_2n(u0);
@@ -285,20 +303,14 @@ struct RefArith {
         const double e = (double)quot(u2, u0, y);
         const double vv = ke == 0 && F32 ? (double)vx * (double)vx : (double)(vx * vx);
         T = (RT)quot(__builtin_fma(-0.5, vv, e), (double)cv, rcv);
-        tiny |= small(vx, u1);
-        return sound(T, gR, vx, a, M, y);
-    }
-    // a = sqrt(gamma R T), y = 1/a, M = v/a and the range test on x
-    __device__ static __forceinline__ bool sound(RT T, RT gR, RT v, RT& a, RT& M, RT& y) {
-        using R = RefRange<RT>;
         const RT x = gR * T;
         sqrt_rcp(x, a, y);
-        M = quot(v, a, y);
-        return x >= R::XLO && x <= R::XHI;
+        M = quot(vx, a, y);
+        span.take(x, u0);
     }
-    // the range test on a velocity (um: its momentum)
-    __device__ static __forceinline__ bool small(RT v, RT um) {
-        return !(fabs(v) >= RefRange<RT>::VLO || um == (RT)0);
+    // the range test on a momentum
+    __device__ static __forceinline__ bool small(RT um) {
+        return !(fabs(um) >= RefRange<RT>::ULO || um == (RT)0);
     }
     // Compute_P_from_U, 2D (base_shll_2d.c:313-317), and the two Mach numbers
     __device__ static __forceinline__ void prim2_exact(RT u0, RT u1, RT u2, RT u3, RT cv, RT gR, RT& vx, RT& vy,
@@ -310,8 +322,9 @@ struct RefArith {
         Mx = vx / a;
         My = vy / a;
     }
-    __device__ static __forceinline__ bool prim2_fast(RT u0, RT u1, RT u2, RT u3, RT cv, double rcv, RT gR, RT& vx,
-                                                      RT& vy, RT& T, RT& a, RT& Mx, RT& My, bool& tiny) {
+    __device__ static __forceinline__ void prim2_fast(RT u0, RT u1, RT u2, RT u3, RT cv, double rcv, RT gR, RT& vx,
+                                                      RT& vy, RT& T, RT& a, RT& Mx, RT& My, RefSpan<RT>& span,
+                                                      bool& tiny) {
         RT y;
         if constexpr (F32) y = rcp_fast(u0);
         else y = rcp_2n(u0);
@@ -319,10 +332,12 @@ struct RefArith {
         vy = quot(u2, u0, y);
         const double e = (double)quot(u3, u0, y);
         T = (RT)quot(__builtin_fma(-0.5, (double)(vx * vx + vy * vy), e), (double)cv, rcv);
-        const bool ok = sound(T, gR, vx, a, Mx, y);
+        const RT x = gR * T;
+        sqrt_rcp(x, a, y);
+        Mx = quot(vx, a, y);
         My = quot(vy, a, y);
-        tiny |= small(vx, u1) || small(vy, u2);
-        return ok;
+        span.take(x, u0);
+        tiny |= small(u1) || small(u2);
     }
     // Z invariants (base_shll.c:137-139): 0.5*(M +- 1) in double, stored to RT, is M/2 +- 1/2
     // rounded once: M/2 is exact, and for a float M the double sum is exact or nowhere near the

@@ -26,15 +26,14 @@ __device__ __forceinline__ void ref_consts(const Inst& in, RT& cv, double& rcv, 
         gR = in.k.f_gR;
     }
 }
-// Compute_P_from_U of one cell: the fast form (false: take the exact one; tiny: divide for the
-// velocity again), the exact form
+// Compute_P_from_U of one cell: the fast form (for cells that pass span), the exact form
 template <class RT>
-__device__ __forceinline__ bool ref_prim1(RT u0, RT u1, RT u2, const Inst& in, RT& vx, RT& T, RT& a, RT& M,
-                                          bool& tiny) {
+__device__ __forceinline__ void ref_prim1(RT u0, RT u1, RT u2, const Inst& in, RT& vx, RT& T, RT& a, RT& M,
+                                          RefSpan<RT>& span) {
     RT cv, gR;
     double rcv;
     ref_consts<RT>(in, cv, rcv, gR);
-    return RefArith<RT>::prim1_fast(u0, u1, u2, in.ke, cv, rcv, gR, vx, T, a, M, tiny);
+    RefArith<RT>::prim1_fast(u0, u1, u2, in.ke, cv, rcv, gR, vx, T, a, M, span);
 }
 template <class RT>
 __device__ __forceinline__ void ref_prim1_exact(RT u0, RT u1, RT u2, const Inst& in, RT& vx, RT& T, RT& a, RT& M) {
@@ -107,24 +106,25 @@ __device__ __forceinline__ void flux1(RT u0, RT u1, RT u2, const Inst& in, RT (&
         split_c32(f2, u2, z1, z2, z3, fp[2], fm[2]);
     } else {
         RT M;
-        bool tiny = false;
-        if (!ref_prim1<RT>(u0, u1, u2, in, vx, T, a, M, tiny)) ref_prim1_exact<RT>(u0, u1, u2, in, vx, T, a, M);
-        else if (tiny) vx = u1 / u0;
+        RefSpan<RT> span;
+        ref_prim1<RT>(u0, u1, u2, in, vx, T, a, M, span);
+        if (!span.ok()) ref_prim1_exact<RT>(u0, u1, u2, in, vx, T, a, M);
         ref_flux1<RT>(u0, u1, u2, vx, T, a, M, fp, fm);
     }
 }
 
-// 2D reference forms: Compute_P_from_U of one cell and the Mach numbers (as ref_prim1)
+// 2D reference forms: Compute_P_from_U of one cell and the Mach numbers (as ref_prim1; tiny: divide
+// for the velocities again)
 template <class RT>
 struct Prim2 {
     RT vx, vy, T, a, Mx, My;
 };
 template <class RT>
-__device__ __forceinline__ bool ref_prim2(const RT (&U)[4], const Inst& in, Prim2<RT>& q, bool& tiny) {
+__device__ __forceinline__ void ref_prim2(const RT (&U)[4], const Inst& in, Prim2<RT>& q, RefSpan<RT>& span, bool& tiny) {
     RT cv, gR;
     double rcv;
     ref_consts<RT>(in, cv, rcv, gR);
-    return RefArith<RT>::prim2_fast(U[0], U[1], U[2], U[3], cv, rcv, gR, q.vx, q.vy, q.T, q.a, q.Mx, q.My, tiny);
+    RefArith<RT>::prim2_fast(U[0], U[1], U[2], U[3], cv, rcv, gR, q.vx, q.vy, q.T, q.a, q.Mx, q.My, span, tiny);
 }
 template <class RT>
 __device__ __forceinline__ void ref_prim2_exact(const RT (&U)[4], const Inst& in, Prim2<RT>& q) {
@@ -133,7 +133,7 @@ __device__ __forceinline__ void ref_prim2_exact(const RT (&U)[4], const Inst& in
     ref_consts<RT>(in, cv, rcv, gR);
     RefArith<RT>::prim2_exact(U[0], U[1], U[2], U[3], cv, gR, q.vx, q.vy, q.T, q.a, q.Mx, q.My);
 }
-// redo what the fast form could not: ok, tiny as ref_prim2 says
+// redo what the fast form could not (ok: span's)
 template <class RT>
 __device__ __forceinline__ void ref_prim2_redo(const RT (&U)[4], const Inst& in, bool ok, Prim2<RT>& q) {
     if (!ok) {
@@ -204,7 +204,9 @@ __device__ __forceinline__ void fluxes2(const RT (&U)[4], const Inst& in, RT (&x
     } else {
         Prim2<RT> q;
         bool tiny = false;
-        const bool ok = ref_prim2<RT>(U, in, q, tiny);
+        RefSpan<RT> span;
+        ref_prim2<RT>(U, in, q, span, tiny);
+        const bool ok = span.ok();
         if (__builtin_expect(!ok || tiny, 0)) ref_prim2_redo<RT>(U, in, ok, q);
         ref_flux2<RT>(U, q, xp, xm, yp, ym);
         a = q.a;

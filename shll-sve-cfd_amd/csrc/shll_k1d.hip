@@ -278,15 +278,12 @@ __device__ __forceinline__ void step_ref(typename Real<PREC>::T (&u)[3][C], cons
     // primitives of all cells, then one branch for the lanes with a cell outside the fast
     // form's range, so the cells' dependent chains overlap
     RT vx[C], T[C], sa[C], M[C];
-    bool ok = true, tiny = false;
+    RefSpan<RT> span;
 #pragma unroll
-    for (int m = 0; m < C; ++m) ok &= ref_prim1<RT>(u[0][m], u[1][m], u[2][m], in, vx[m], T[m], sa[m], M[m], tiny);
-    if (__builtin_expect(!ok || tiny, 0)) {
+    for (int m = 0; m < C; ++m) ref_prim1<RT>(u[0][m], u[1][m], u[2][m], in, vx[m], T[m], sa[m], M[m], span);
+    if (__builtin_expect(!span.ok(), 0)) {
 #pragma unroll
-        for (int m = 0; m < C; ++m) {
-            if (!ok) ref_prim1_exact<RT>(u[0][m], u[1][m], u[2][m], in, vx[m], T[m], sa[m], M[m]);
-            else vx[m] = u[1][m] / u[0][m];
-        }
+        for (int m = 0; m < C; ++m) ref_prim1_exact<RT>(u[0][m], u[1][m], u[2][m], in, vx[m], T[m], sa[m], M[m]);
     }
 #pragma unroll
     for (int m = 0; m < C; ++m) {

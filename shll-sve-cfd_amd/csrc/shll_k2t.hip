@@ -91,9 +91,11 @@ struct Tile2 {
             // primitives of all rows, then one branch for the lanes with a cell outside the
             // fast form's range, so the rows' dependent chains overlap
             Prim2<RT> q[RW];
-            bool ok = true, tiny = false;
+            RefSpan<RT> span;
+            bool tiny = false;
 #pragma unroll
-            for (int r = 0; r < RW; ++r) ok &= ref_prim2<RT>(u[r], in, q[r], tiny);
+            for (int r = 0; r < RW; ++r) ref_prim2<RT>(u[r], in, q[r], span, tiny);
+            const bool ok = span.ok();
             if (__builtin_expect(!ok || tiny, 0)) {
 #pragma unroll
                 for (int r = 0; r < RW; ++r) ref_prim2_redo<RT>(u[r], in, ok, q[r]);
