@@ -256,20 +256,12 @@ __device__ __forceinline__ void ghost_cells(RT (&q)[3][C], int gl, int n, bool r
 // ---------------------------------------------------------------------------
 // F64 / REF32: the reference association, cell by cell
 // ---------------------------------------------------------------------------
-// u - k*x in one fused multiply-add: for k a power of two (k*x is exact) the bits of the two
-// operations
-template <class RT>
-__device__ __forceinline__ RT fms(RT k, RT x, RT u) { return __builtin_elementwise_fma(-k, x, u); }
-
 template <int PREC, int ORDER, int C, int WM, int LIM, int XW>
 __device__ __forceinline__ void step_ref(typename Real<PREC>::T (&u)[3][C], const Inst& in, int gl,
                                          const Coop<typename Real<PREC>::T, XW>& x, int parity) {
     using RT = typename Real<PREC>::T;
     using A = RefArith<RT>;
-    // DT/DX = CFL/(R + 1) = 1/8 (base_shll.c:18,84): products with it and its half are exact, so
-    // u - lam*x and the second-order term (formed in double by the reference, then stored to
-    // float: harmless twice-rounding of a sum of two floats) are fused multiply-adds
-    constexpr RT lam = (RT)0.125, hlam = (RT)0.0625;
+    constexpr RT lam = (RT)0.125;  // DT/DX = CFL/(R + 1) (base_shll.c:18,84)
     const RT th = PREC == PREC_F64 ? (RT)in.k.d_theta : (RT)in.k.f_theta;
     const int n = in.nx;
     const bool refl = in.bc == BC_REFLECT;
@@ -305,8 +297,8 @@ __device__ __forceinline__ void step_ref(typename Real<PREC>::T (&u)[3][C], cons
             for (int m = 0; m < C; ++m) {
                 // F+ of the left neighbour, F- of the right one; own slopes, the left
                 // neighbour's F+ slope and the right neighbour's F- slope
-                const RT uu = fms(lam, fp[v][m] - fm[v][m] + w.FM[m + 2] - w.FP[m], u[v][m]);
-                u[v][m] = fms(hlam, w.sp(m + 1) + w.sm(m) - w.sm(m + 1) - w.sp(m), uu);
+                const RT uu = u[v][m] - lam * (fp[v][m] - fm[v][m] + w.FM[m + 2] - w.FP[m]);
+                u[v][m] = ref_second<true>(uu, lam, w.sp(m + 1) + w.sm(m) - w.sm(m + 1) - w.sp(m));
             }
         }
         return;
@@ -328,7 +320,7 @@ __device__ __forceinline__ void step_ref(typename Real<PREC>::T (&u)[3][C], cons
         for (int m = 0; m < C; ++m) {
             const int g = gl + m;
             // FL = F+ of the left neighbour, FR = F- of the right one (ghosts at the walls)
-            RT uu = fms(lam, fp[v][m] - fm[v][m] + FM[m + 3] - FP[m + 1], u[v][m]);
+            RT uu = u[v][m] - lam * (fp[v][m] - fm[v][m] + FM[m + 3] - FP[m + 1]);
             if constexpr (ORDER == 2) {
                 // own slopes, the left neighbour's F+ slope and the right neighbour's F-
                 // slope; every slope of a boundary or ghost cell is zero
@@ -336,7 +328,7 @@ __device__ __forceinline__ void step_ref(typename Real<PREC>::T (&u)[3][C], cons
                 RT dm = slope_at<A, WM, LIM>(FM, m, g, n, th);
                 RT Ldf = slope_at<A, WM, LIM>(FP, m - 1, g - 1, n, th);
                 RT Rdf = slope_at<A, WM, LIM>(FM, m + 1, g + 1, n, th);
-                uu = fms(hlam, dp + dm - Rdf - Ldf, uu);
+                uu = ref_second<true>(uu, lam, dp + dm - Rdf - Ldf);
             }
             u[v][m] = uu;
         }

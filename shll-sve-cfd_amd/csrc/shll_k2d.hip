@@ -171,13 +171,12 @@ __device__ __forceinline__ void rows2(const StepArgs& a, const Item2& it, const 
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 if constexpr (!CMP) {
-                    using U = RefUpdate<RT>;
                     RT R = rb.xm[v];
                     if constexpr (!INNER) R = c == nx - 1 ? (refl ? (RT)sgn_x(v) * ra.xp[v] : ra.xm[v]) : R;
-                    RT uu = U::template first<true>(v == 2, ra.u[v], lamx, ra.xp[v] - ra.xm[v] + R - L[v]);
-                    uu = U::template second<true>(v == 2, uu, lamx, sP[v] + sM[v] - nM[v] - sPl[v]);
-                    uu = U::template first<SQ>(v == 1, uu, lamy, ra.y1[v]);
-                    uu = U::template second<SQ>(v == 1, uu, lamy, ra.y2[v]);
+                    RT uu = ra.u[v] - lamx * (ra.xp[v] - ra.xm[v] + R - L[v]);
+                    uu = ref_second<true>(uu, lamx, sP[v] + sM[v] - nM[v] - sPl[v]);
+                    uu = uu - lamy * ra.y1[v];
+                    uu = ref_second<SQ>(uu, lamy, ra.y2[v]);
                     if (jown) q0[v * P + o] = uu;
                 } else {
                     RT hi = ra.u[v], lo = ra.l[v], e;
@@ -276,11 +275,11 @@ void k_row2d(StepArgs a) {
     const Item2 it = ((const Item2*)a.items)[wave];
     const Inst in = a.inst[it.inst];
     if (in.nsteps - lv.step_base <= 0) return;
-    // strips away from both y walls take the copy without wall choices, square cells the one
-    // with DT/DY = 1/8
+    // strips away from both y walls take the copy without wall choices, REF32 on square cells the
+    // one with DT/DY = 1/8 (ref_second)
     const bool yw = it.j0 <= 0 || it.j0 + 64 >= in.ny;
-    if constexpr (PREC == PREC_F64 || PREC == PREC_REF32) {
-        const bool sq = PREC == PREC_F64 ? in.k.d_lamy == 0.125 : in.k.f_lamy == 0.125f;
+    if constexpr (PREC == PREC_REF32) {
+        const bool sq = in.k.f_lamy == 0.125f;
         if (yw) {
             if (sq) rows2<PREC, LIM, true, true>(a, it, in, lane);
             else rows2<PREC, LIM, true, false>(a, it, in, lane);
@@ -350,7 +349,7 @@ __device__ __forceinline__ void stage2(Held2& h, double (&io)[4], int mode, bool
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             const double Rv = mode == ST_DRAIN && refl ? sgn_x(v) * h.fp[v] : xm[v];
-            const double uu = RefUpdate<double>::first<true>(v == 2, h.u[v], lamx, h.d[v] + Rv - h.tl[v]);
+            const double uu = h.u[v] - lamx * (h.d[v] + Rv - h.tl[v]);
             io[v] = uu - lamy * h.yb[v];
         }
     }

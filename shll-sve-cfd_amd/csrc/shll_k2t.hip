@@ -31,8 +31,8 @@ __device__ __forceinline__ RT wall_x(int v, RT f) { return v == 1 ? f : -f; }
 template <class RT>
 __device__ __forceinline__ RT wall_y(int v, RT f) { return v == 2 ? f : -f; }
 
-// One wavefront's rows.  EDGE: the tile touches a wall; SQ: DT/DY = 1/8 (reference forms).
-template <int PREC, int RW, int W, bool EDGE, bool SQ>
+// One wavefront's rows.  EDGE: the tile touches a wall.
+template <int PREC, int RW, int W, bool EDGE>
 struct Tile2 {
     using RT = typename Real<PREC>::T;
     static constexpr bool CMP = PREC == PREC_C32 || PREC == PREC_C32K;  // (hi, lo) state
@@ -175,9 +175,8 @@ struct Tile2 {
                         L = g0 + r == 0 ? (refl ? wall_x(v, xm[r][v]) : xp[r][v]) : L;
                         R = g0 + r == in.nx - 1 ? (refl ? wall_x(v, xp[r][v]) : xm[r][v]) : R;
                     }
-                    using U = RefUpdate<RT>;
-                    const RT uu = U::template first<true>(v == 2, u[r][v], lamx, xp[r][v] - xm[r][v] + R - L);
-                    u[r][v] = U::template first<SQ>(v == 1, uu, lamy, Y1[r][v]);
+                    const RT uu = u[r][v] - lamx * (xp[r][v] - xm[r][v] + R - L);
+                    u[r][v] = uu - lamy * Y1[r][v];
                 }
             }
         }
@@ -185,10 +184,10 @@ struct Tile2 {
 };
 
 // ns steps of rows [i0, i0 + W*RW), of which the item's are stored
-template <int PREC, int RW, int W, bool EDGE, bool SQ>
+template <int PREC, int RW, int W, bool EDGE>
 __device__ __forceinline__ void tile_steps(const StepArgs& a, const Item2& it, const Inst& in, int i0, int ns,
                                            typename Real<PREC>::T* lds) {
-    using T = Tile2<PREC, RW, W, EDGE, SQ>;
+    using T = Tile2<PREC, RW, W, EDGE>;
     using RT = typename T::RT;
     constexpr bool CMP = T::CMP;
     const int wib = uniform((int)threadIdx.x >> 6), lane = (int)threadIdx.x & 63;
@@ -249,19 +248,8 @@ __global__ __launch_bounds__(64 * W) void k_tile2d(StepArgs a) {
     // walls, the halo (the host makes no item of more than W*RW - 2k rows)
     const int i0 = it.ix0 - a.ksteps < 0 ? 0 : it.ix0 - a.ksteps;
     const bool edge = i0 <= 0 || i0 + W * RW >= in.nx || it.j0 <= 0 || it.j0 + 64 >= in.ny;
-    if constexpr (PREC == PREC_F64 || PREC == PREC_REF32) {
-        const bool sq = PREC == PREC_F64 ? in.k.d_lamy == 0.125 : in.k.f_lamy == 0.125f;
-        if (edge) {
-            if (sq) tile_steps<PREC, RW, W, true, true>(a, it, in, i0, ns, lds);
-            else tile_steps<PREC, RW, W, true, false>(a, it, in, i0, ns, lds);
-        } else {
-            if (sq) tile_steps<PREC, RW, W, false, true>(a, it, in, i0, ns, lds);
-            else tile_steps<PREC, RW, W, false, false>(a, it, in, i0, ns, lds);
-        }
-    } else {
-        if (edge) tile_steps<PREC, RW, W, true, false>(a, it, in, i0, ns, lds);
-        else tile_steps<PREC, RW, W, false, false>(a, it, in, i0, ns, lds);
-    }
+    if (edge) tile_steps<PREC, RW, W, true>(a, it, in, i0, ns, lds);
+    else tile_steps<PREC, RW, W, false>(a, it, in, i0, ns, lds);
 }
 
 // ---------------------------------------------------------------------------
