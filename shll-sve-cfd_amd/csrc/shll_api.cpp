@@ -903,6 +903,10 @@ static shll_status engine_init_state(Engine* E, const double* const* prims) {
         if (e != hipSuccess) return fail(SHLL_EDEVICE, "upload: %s", hipGetErrorString(e));
         e = convert(E->d_prim);
         const hipError_t w = hipStreamSynchronize(E->stream);
+        // as large as a buffer of an FP64 state: a solver that is only stepped, or a batch that takes
+        // its snapshot next, does not hold it (a first large read allocates it again)
+        (void)hipFree(E->d_prim);
+        E->d_prim = nullptr;
         if (e != hipSuccess || w != hipSuccess)
             return fail(SHLL_EDEVICE, "init kernel: %s", hipGetErrorString(e != hipSuccess ? e : w));
     }
