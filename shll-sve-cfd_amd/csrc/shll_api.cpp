@@ -83,6 +83,7 @@ extern "C" const char* shll_version(void) { return "shll_amd 0.1 (gfx950)"; }
 // MiB that are kept between calls: up to 4 MiB the output kernels write straight into one slab
 // (no copy command, one synchronisation), beyond that up to eight threads each take the next
 // piece, copy it between its slab and the caller's memory, and have a second piece in flight.
+// Where no memory can be pinned, ordinary memory takes a slab's place, at the runtime's pace.
 // Measured (16-core host), before and now: 24 KB of primitives 48 and 14 us, 111 MB of 400 tubes
 // one by one 24 and 11.8 ms, 537 MB 51.5 and 12.5 ms; constructing a 128^2 context 183 and 96 us.
 // ---------------------------------------------------------------------------
@@ -98,6 +99,7 @@ size_t g_nslabs = 0;
 
 struct Slab {
     char* p = nullptr;
+    bool pinned = true;  // a kernel may write to it
     Slab() {
         {
             std::lock_guard<std::mutex> lock(g_slab_mu);
@@ -106,11 +108,17 @@ struct Slab {
                 return;
             }
         }
-        if (hipHostMalloc((void**)&p, kSlabBytes, hipHostMallocPortable) != hipSuccess) p = nullptr;
+        if (hipHostMalloc((void**)&p, kSlabBytes, hipHostMallocPortable) == hipSuccess) return;
+        (void)hipGetLastError();  // launches report the last error
+        pinned = false;
+        p = (char*)std::malloc(kSlabBytes);
     }
     // its last use by the device must have completed
     ~Slab() {
-        if (!p) return;
+        if (!pinned) {
+            std::free(p);
+            return;
+        }
         {
             std::lock_guard<std::mutex> lock(g_slab_mu);
             if (g_nslabs < kSlabsKept) {
@@ -881,15 +889,19 @@ static shll_status engine_init_state(Engine* E, const double* const* prims) {
         return launch_init(E->prec, E->dim, elem_blocks(maxcells), (int)E->h_inst.size(), E->stream, E->d_inst, src,
                            E->buf[0][0], E->buf[0][1], E->plane);
     };
+    bool done = false;
     if (total <= kSlabBytes) {
         Slab slab;
-        if (!slab.p) return fail(SHLL_ENOMEM, "hipHostMalloc(%zu) for the initial data", kSlabBytes);
-        gather(slab.p, 0, total);
-        const hipError_t e = convert((const double*)slab.p);
-        const hipError_t w = hipStreamSynchronize(E->stream);
-        if (e != hipSuccess || w != hipSuccess)
-            return fail(SHLL_EDEVICE, "init kernel: %s", hipGetErrorString(e != hipSuccess ? e : w));
-    } else {
+        if (slab.pinned) {
+            gather(slab.p, 0, total);
+            const hipError_t e = convert((const double*)slab.p);
+            const hipError_t w = hipStreamSynchronize(E->stream);
+            if (e != hipSuccess || w != hipSuccess)
+                return fail(SHLL_EDEVICE, "init kernel: %s", hipGetErrorString(e != hipSuccess ? e : w));
+            done = true;
+        }
+    }
+    if (!done) {
         shll_status st = ensure_prim(E);
         if (st != SHLL_OK) return st;
         auto len = [&](size_t i) { return std::min(kSlabBytes, total - i * kSlabBytes); };
@@ -955,13 +967,14 @@ static shll_status engine_get(Engine* E, int64_t i, double* prim, double* cons) 
     };
     if (bytes <= kSlabBytes) {
         Slab slab;
-        if (!slab.p) return fail(SHLL_ENOMEM, "hipHostMalloc(%zu)", kSlabBytes);
-        const hipError_t e = output((double*)slab.p);
-        const hipError_t w = hipStreamSynchronize(E->stream);
-        HIPCHECK(e);
-        HIPCHECK(w);
-        std::memcpy(dst, slab.p, bytes);
-        return SHLL_OK;
+        if (slab.pinned) {
+            const hipError_t e = output((double*)slab.p);
+            const hipError_t w = hipStreamSynchronize(E->stream);
+            HIPCHECK(e);
+            HIPCHECK(w);
+            std::memcpy(dst, slab.p, bytes);
+            return SHLL_OK;
+        }
     }
     shll_status st = ensure_prim(E);
     if (st != SHLL_OK) return st;
@@ -987,7 +1000,8 @@ static shll_status engine_sums(Engine* E, std::vector<double>& out) {
     const size_t n = (size_t)ninst * nb * 6;
     out.assign((size_t)ninst * 5, 0.0);
     // few partials: the kernel writes them into a pinned slab
-    const bool small = n * sizeof(double) <= kSlabBytes;
+    Slab slab;
+    const bool small = n * sizeof(double) <= kSlabBytes && slab.pinned;
     std::vector<double> part(small ? 0 : n);
     // instances may sit in different buffers: launch per parity group
     for (int p = 0; p < 2; ++p) {
@@ -1009,8 +1023,6 @@ static shll_status engine_sums(Engine* E, std::vector<double>& out) {
             }
         };
         if (small) {
-            Slab slab;
-            if (!slab.p) return fail(SHLL_ENOMEM, "hipHostMalloc(%zu)", kSlabBytes);
             const hipError_t e = sums((double*)slab.p);
             const hipError_t w = hipStreamSynchronize(E->stream);
             HIPCHECK(e);
