@@ -89,13 +89,16 @@ extern "C" const char* shll_version(void) { return "shll_amd 0.1 (gfx950)"; }
 // ---------------------------------------------------------------------------
 namespace {
 constexpr size_t kSlabBytes = 4u << 20;
-constexpr size_t kSlabsKept = 16;
+constexpr size_t kSlabsKept = 16, kSlabsIdle = 2;
 
-// The slabs not in use: at most kSlabsKept stay allocated for the process, the others are freed
-// when they are returned.  Portable, so any device may use any slab.
+// The slabs not in use: at most kSlabsKept stay allocated while there is a context or batch, the
+// others are freed when they are returned; when the last context goes, all but kSlabsIdle (what a
+// program needs that makes small contexts one after another) are freed.  Portable, so any device
+// may use any slab.
 std::mutex g_slab_mu;
 char* g_slabs[kSlabsKept];
 size_t g_nslabs = 0;
+int64_t g_engines = 0;  // contexts and batches
 
 struct Slab {
     char* p = nullptr;
@@ -121,7 +124,7 @@ struct Slab {
         }
         {
             std::lock_guard<std::mutex> lock(g_slab_mu);
-            if (g_nslabs < kSlabsKept) {
+            if (g_nslabs < (g_engines > 0 ? kSlabsKept : kSlabsIdle)) {
                 g_slabs[g_nslabs++] = p;
                 return;
             }
@@ -131,6 +134,17 @@ struct Slab {
     Slab(const Slab&) = delete;
     Slab& operator=(const Slab&) = delete;
 };
+
+void slabs_engine(int64_t d) {
+    char* idle[kSlabsKept];
+    size_t n = 0;
+    {
+        std::lock_guard<std::mutex> lock(g_slab_mu);
+        g_engines += d;
+        while (g_engines == 0 && g_nslabs > kSlabsIdle) idle[n++] = g_slabs[--g_nslabs];
+    }
+    while (n > 0) (void)hipHostFree(idle[--n]);
+}
 
 // Pieces [0, n) of a transfer.  start(i, slab): enqueue the copy between slab and device (an
 // upload fills the slab first); finish(i, slab): after it has completed.  Every piece is done by
@@ -529,6 +543,7 @@ static void engine_free(Engine* E) {
     if (E->ev1) (void)hipEventDestroy(E->ev1);
     if (E->stream) (void)hipStreamDestroy(E->stream);
     delete E;
+    slabs_engine(-1);
 }
 
 static int radius(const Engine* E) { return E->order; }
@@ -1050,6 +1065,7 @@ struct shll_ctx {
 
 static Engine* engine_new(int dim, int order, int prec, int lim) {
     Engine* E = new Engine();
+    slabs_engine(1);
     E->dim = dim;
     E->order = order;
     E->prec = prec;

@@ -1,6 +1,6 @@
 """GPU: transfers where the process can pin no memory.  A shim in front of the runtime's
 hipHostMalloc, in a process of its own, refuses; construction, reads, restarts and sums go on through
-ordinary memory, with the same values."""
+ordinary memory, with the same values.  And what stays pinned once no solver is left (the shim counts)."""
 import os
 import subprocess
 import sys
@@ -75,5 +75,29 @@ for a, b in zip(without, [values(n) for n in (64, 700)]):
     for x, y in zip(a, b):
         np.testing.assert_array_equal(x, y)
 assert made.value > 0
+print("done")
+""")
+
+
+def test_pinned_memory_is_given_back(tmp_path):
+    """Large transfers pin a piece or two per thread; of those, two stay when the last solver goes."""
+    banner("pinned memory given back")
+    run(tmp_path, """
+n = 1500
+ic = icgen.random_2d(n, n, 5, block=8)
+pb = S.problem(2, 1, n, n, precision=S.F64)
+small = S.Solver(S.problem(1, 1, 100, precision=S.F64), S.ic_tube(100))
+with S.Solver(pb, ic) as s:
+    s.primitives()
+assert made.value > 2 and freed.value == 0, (made.value, freed.value)
+small.conserved()
+small.close()
+assert made.value - freed.value == 2, (made.value, freed.value)
+pinned = made.value
+for _ in range(3):
+    with S.Solver(S.problem(2, 1, 100, 100, precision=S.F64), S.ic_circle(100, 100)) as s:
+        s.step(3)
+        s.primitives()
+assert made.value == pinned
 print("done")
 """)
