@@ -180,7 +180,8 @@ void shll_free(shll_ctx *ctx);
  * steps_per_launch >= 1 (temporal blocking; 2D: 1, 2, 3, 4 or 8 in first order; 1, or 2 for
  * SHLL_C32/SHLL_C32K in second order),
  * waves_per_block in {1,4} (1D, 4 with 2+ cells per lane: the block's wavefronts hold
- * one segment and share their edge fluxes), graph_steps: steps captured per HIP graph
+ * one segment and share their edge fluxes; register tiles have blocks of their own, whatever
+ * is asked for), graph_steps: steps captured per HIP graph
  * (0 = no graph; at most 4096 launches per graph; a single instance's graphs are captured
  * when the shape is set).  shll_get_launch returns the values as set (a 2D 0 reads back as 1).
  * Results do not depend on the launch shape (bitwise). */
@@ -191,10 +192,10 @@ shll_status shll_get_launch(const shll_ctx *ctx, int32_t out[4]);
  * keep the fastest; the choice is cached per (device, kernel, shape class) in
  * $SHLL_TUNE_CACHE (if set).  Candidates: 1D cells per lane 1-8, 1-64 steps per launch,
  * 1 or 4 waves per block (and 256-4096 steps per launch when the whole tube fits one
- * segment or block, which then has no halo); 2D the valid steps per launch, 1 or 4
- * waves per block, and where items have a height of their own (second order, and SHLL_F64
- * in first order) 3/4, 5/4 and 3/2 of the default rows, and shorter ones (down to 1/8)
- * when the default ones give fewer than 4 wavefronts per SIMD; graphs of
+ * segment or block, which then has no halo); 2D the valid steps per launch, and where they
+ * do not run on register tiles 1 or 4 waves per block, 3/4, 5/4 and 3/2 of the default rows,
+ * and in second order shorter ones (down to 1/8) when the default ones give fewer than 4
+ * wavefronts per SIMD; graphs of
  * 128 (2D: 64) steps, or two launches if longer, and for a single instance also of 2048
  * (2D: 1024) steps and direct launches (graph_steps 0). */
 shll_status shll_autotune(shll_ctx *ctx, int32_t trial_steps);

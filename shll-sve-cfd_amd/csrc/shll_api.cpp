@@ -501,11 +501,13 @@ static bool in_cache(const Engine* E) { return state_bytes(E) <= (256LL << 20); 
 // 2D first order: rows of the register tiles, 0 for the row pipelines, which FP64 keeps at 1 and
 // 2 steps per launch on domains well beyond the last-level cache (us per step at k = 2, pipeline
 // and tiles: 2048^2, 256 MB, 58 and 38; 2500^2, 400 MB, 66 and 61; 3072^2, 604 MB, 86 and 90;
-// 4096^2 147 and 151; 8192^2 530 and 588).  An item is one tile, whatever rows the launch shape
-// asks for.
+// 4096^2 147 and 151; 8192^2 530 and 588).  An item is one tile and its block has the wavefronts
+// of that, whatever rows and waves per block the launch shape asks for.
+static bool use_tiles2d(const Engine* E, int k) {
+    return E->dim == 2 && E->order == 1 && !(E->prec == SHLL_F64 && k <= 2 && state_bytes(E) > (448LL << 20));
+}
 static int pick_tile2d(const Engine* E) {
-    if (E->dim != 2 || E->order != 1) return 0;
-    if (E->prec == SHLL_F64 && E->L.k <= 2 && state_bytes(E) > (448LL << 20)) return 0;
+    if (!use_tiles2d(E, E->L.k)) return 0;
     return tile2d_rows(
         E->prec, E->L.k, (int)(simd_count(E) / 4),
         [](const void* e, int rows) { return items2d((const Engine*)e, ((const Engine*)e)->L.k, rows); }, E);
@@ -1664,6 +1666,9 @@ static shll_status engine_autotune(Engine* E, int32_t trial_steps, int64_t shape
         for (int k : {1, 2, 3, 4, 8})
             for (int w : {1, 4}) {
                 if (!step2d_supported(E->prec, E->order, k)) continue;
+                // register tiles have a height and a block of their own: one candidate
+                const bool tiles = use_tiles2d(E, k);
+                if (tiles && w != 4) continue;
                 // items a little longer or shorter than the default change how many rounds
                 // of resident wavefronts a launch takes, whose last round may run part-empty;
                 // much shorter items when the default ones give fewer than 4 wavefronts per
@@ -1671,7 +1676,7 @@ static shll_status engine_autotune(Engine* E, int32_t trial_steps, int64_t shape
                 // items is latency-bound, and more items trade halo rows for parallelism
                 const int rd = rows2d(k);
                 std::vector<int> rows = {1};
-                if (E->order == 2 || E->prec == SHLL_F64) rows = {1, rd * 3 / 4, rd * 5 / 4, rd * 3 / 2};
+                if (!tiles) rows = {1, rd * 3 / 4, rd * 5 / 4, rd * 3 / 2};
                 if (E->order == 2 && items2d(E, k, rd) < 4 * simd_count(E))
                     for (int r : {rd / 2, rd * 3 / 8, rd / 4, rd * 3 / 16, rd / 8})
                         if (r >= 2) rows.push_back(r);
