@@ -93,20 +93,19 @@ __device__ __forceinline__ double from_right_or(double x, double e) {
 __device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
 
 // ---------------------------------------------------------------------------
-// Correctly rounded division and square root.  The fast paths (div_fast, sqrt_fast)
-// are the instruction sequences the compiler emits for IEEE '/', sqrtf and sqrt
-// (-fhip-fp32-correctly-rounded-divide-sqrt; FP64 is always IEEE) minus their range
-// handling -- the exponent pre-scaling of v_div_scale / v_div_fmas, the special-value
-// pass of v_div_fixup, the square roots' pre-scaling of tiny radicands and their
-// pass-through of 0 and inf.  With operands and results of moderate size (no
+// Correctly rounded division and square root.  The fast paths are the instruction sequences the
+// compiler emits for IEEE '/', sqrtf and sqrt (-fhip-fp32-correctly-rounded-divide-sqrt; FP64 is
+// always IEEE) minus their range handling -- the exponent pre-scaling of v_div_scale /
+// v_div_fmas, the special-value pass of v_div_fixup, the square roots' pre-scaling of tiny
+// radicands and their pass-through of 0 and inf.  With operands and results of moderate size (no
 // intermediate leaves the normal range) they give the same bits as the operators.
 // The reference forms (F64, REF32) call them through RefArith::prim1_fast / prim2_fast, which
-// say per cell whether every intermediate stayed in that range (one test per cell, below), and
-// hand the other cells -- a vacuum, a tiny velocity, a non-finite state -- to the operators
-// themselves (prim1_exact / prim2_exact), so they are always bitwise '/' and sqrt.  The
-// compensated scheme calls the fast paths directly: its divisors (density, sound speed) and
-// radicand (gamma*R*T) are of order one, and its one possibly tiny quotient, the Mach number
-// M, only enters as M/2 +- 1/2 and 1 - M^2, which absorb any last-place difference of a tiny M.
+// say whether every intermediate stayed in that range (below), and hand the other cells -- a
+// vacuum, a tiny velocity, a non-finite state -- to the operators themselves (prim1_exact /
+// prim2_exact), so they are always bitwise '/' and sqrt.  The compensated scheme calls the fast
+// paths directly: its divisors (density, sound speed) and radicand (gamma*R*T) are of order one,
+// and its one possibly tiny quotient, the Mach number M, only enters as M/2 +- 1/2 and 1 - M^2,
+// which absorb any last-place difference of a tiny M.
 // ---------------------------------------------------------------------------
 // rcp_fast(b): 1/b correctly rounded -- v_rcp_f32 (within 1 ulp) and one Newton step with
 // fused multiply-adds.  Checked against IEEE 1.0f/b on the MI355X for every normal float b
@@ -116,25 +115,16 @@ __device__ __forceinline__ float rcp_fast(float b) {
     const float e = __builtin_fmaf(-b, r, 1.0f);
     return __builtin_fmaf(e, r, r);
 }
-// a/b from the correctly rounded reciprocal y: q = a*y is within one ulp of a/b, the
-// residual a - b*q is exact in one fma, and q + residual*y is the correctly rounded
-// quotient (Markstein's theorem; also checked against IEEE a/b on 2^31 random pairs)
-__device__ __forceinline__ float div_fast(float a, float b) {
-    const float y = rcp_fast(b);
-    const float q = a * y;
-    const float d = __builtin_fmaf(-b, q, a);
-    return __builtin_fmaf(d, y, q);
+// a/b from its correctly rounded reciprocal y: q = a*y is within one ulp of a/b, the residual
+// a - b*q is exact in one fma, and q + residual*y is the correctly rounded quotient (Markstein's
+// theorem; also checked against IEEE a/b on 2^31 random float and 2^28 random double pairs)
+template <class RT>
+__device__ __forceinline__ RT quot(RT a, RT b, RT y) {
+    const RT q = a * y;
+    const RT d = __builtin_elementwise_fma(-b, q, a);
+    return __builtin_elementwise_fma(d, y, q);
 }
-__device__ __forceinline__ double div_fast(double a, double b) {
-    double r = __builtin_amdgcn_rcp(b);
-    double e = __builtin_fma(-b, r, 1.0);
-    r = __builtin_fma(r, e, r);
-    e = __builtin_fma(-b, r, 1.0);
-    r = __builtin_fma(r, e, r);            // two Newton steps on 1/b
-    const double q = a * r;
-    const double d = __builtin_fma(-b, q, a);
-    return __builtin_fma(d, r, q);
-}
+__device__ __forceinline__ float div_fast(float a, float b) { return quot(a, b, rcp_fast(b)); }
 __device__ __forceinline__ float sqrt_fast(float x) {
     float s = __builtin_amdgcn_sqrtf(x);   // within 1 ulp
     const float sdn = __int_as_float(__float_as_int(s) - 1);
@@ -144,37 +134,22 @@ __device__ __forceinline__ float sqrt_fast(float x) {
     s = rdn <= 0.0f ? sdn : s;
     return rup > 0.0f ? sup : s;
 }
-__device__ __forceinline__ double sqrt_fast(double x) {
-    const double y = __builtin_amdgcn_rsq(x);
-    double g = x * y, h = y * 0.5;         // sqrt(x) and 1/(2 sqrt(x)) estimates
-    const double r = __builtin_fma(-h, g, 0.5);
-    g = __builtin_fma(g, r, g);
-    double d = __builtin_fma(-g, g, x);
-    h = __builtin_fma(h, r, h);
-    g = __builtin_fma(d, h, g);
-    d = __builtin_fma(-g, g, x);
-    return __builtin_fma(d, h, g);
-}
-// a/b given y = 1/b correctly rounded (the last three operations of div_fast)
-template <class RT>
-__device__ __forceinline__ RT quot(RT a, RT b, RT y) {
-    const RT q = a * y;
-    const RT d = __builtin_elementwise_fma(-b, q, a);
-    return __builtin_elementwise_fma(d, y, q);
-}
-// 1/b as div_fast's two Newton steps give it
-__device__ __forceinline__ double rcp_2n(double b) {
+// 1/b: the hardware's seed (v_rcp_f64, relative error about 2^-24, measured) and two Newton steps;
+// equal to the correctly rounded 1/b on each of 8e8 random arguments with exponents -1000..1000
+// (MI355X).  Zero gives NaN (not inf).
+__device__ __forceinline__ double rcp_nr2(double b) {
     double r = __builtin_amdgcn_rcp(b);
     double e = __builtin_fma(-b, r, 1.0);
     r = __builtin_fma(r, e, r);
     e = __builtin_fma(-b, r, 1.0);
     return __builtin_fma(r, e, r);
 }
-// s = sqrt(x) as sqrt_fast gives it, and y = 1/s: the square root's iteration already holds
+// s = sqrt(x) correctly rounded, and y = 1/s: the square root's iteration already holds
 // h = 1/(2 sqrt(x)) to about 2^-46, so one Newton step on 2h replaces a reciprocal seed and two
+// (checked with quot against IEEE sqrt and v/sqrt(x) on 2^28 random arguments)
 __device__ __forceinline__ void sqrt_rcp(double x, double& s, double& y) {
     const double q = __builtin_amdgcn_rsq(x);
-    double g = x * q, h = q * 0.5;
+    double g = x * q, h = q * 0.5;  // sqrt(x) and 1/(2 sqrt(x)) estimates
     const double r = __builtin_fma(-h, g, 0.5);
     g = __builtin_fma(g, r, g);
     h = __builtin_fma(h, r, h);
@@ -191,24 +166,14 @@ __device__ __forceinline__ void sqrt_rcp(float x, float& s, float& y) {
     y = rcp_fast(s);
 }
 
-// Faithful FP64 reciprocal and reciprocal square root (the F64F form): the hardware seeds
-// (v_rcp_f64, v_rsq_f64; relative error about 2^-24, measured) and a correction each.
-//   rcp_nr2(b): r <- r + r(1 - b r); equal to the correctly rounded 1/b on each of 8e8
-//               random arguments with exponents -1000..1000 (MI355X)
-//   rsq_nr2(x): one third-order step y <- y (1 + e/2 + 3 e^2/8), e = 1 - x y^2 (its remainder
-//               is 5/16 e^3, about 2^-73; two Newton steps took one operation more and rounded
-//               twice); within 2 ulp of 1.0/sqrt(x) on the same arguments.  rsq_sqrt also
-//               gives sqrt(x) from the same correction, in one operation
-// Neither is correctly rounded by construction, and the seeds are the hardware's, so the
-// F64F results are reproduced on a CPU to within round-off, not bit for bit.  A zero argument
-// gives NaN (not inf); negative and NaN arguments give NaN.
-__device__ __forceinline__ double rcp_nr2(double b) {
-    double r = __builtin_amdgcn_rcp(b);
-    double e = __builtin_fma(-b, r, 1.0);
-    r = __builtin_fma(r, e, r);
-    e = __builtin_fma(-b, r, 1.0);
-    return __builtin_fma(r, e, r);
-}
+// Faithful FP64 reciprocal square root and square root (the F64F form, with rcp_nr2): the hardware
+// seed (v_rsq_f64, relative error about 2^-24, measured) and one third-order step
+// y <- y (1 + e/2 + 3 e^2/8), e = 1 - x y^2 (its remainder is 5/16 e^3, about 2^-73; two Newton steps
+// took one operation more and rounded twice), and the same correction of x y for the root.  y is
+// within 2 ulp of 1.0/sqrt(x), s within 1 of sqrt(x) on random arguments with exponents -1000..1000
+// (MI355X); neither is correctly rounded, and the seeds are the hardware's, so the F64F results are
+// reproduced on a CPU to within round-off, not bit for bit.  Zero, negative and NaN arguments
+// give NaN.
 __device__ __forceinline__ void rsq_sqrt(double x, double& y, double& s) {
     const double q = __builtin_amdgcn_rsq(x);
     const double g = x * q;
@@ -298,7 +263,7 @@ struct RefArith {
                                                       RT& T, RT& a, RT& M, RefSpan<RT>& span) {
         RT y;
         if constexpr (F32) y = rcp_fast(u0);
-        else y = rcp_2n(u0);
+        else y = rcp_nr2(u0);
         vx = quot(u1, u0, y);
         const double e = (double)quot(u2, u0, y);
         const double vv = ke == 0 && F32 ? (double)vx * (double)vx : (double)(vx * vx);
@@ -327,7 +292,7 @@ struct RefArith {
                                                       bool& tiny) {
         RT y;
         if constexpr (F32) y = rcp_fast(u0);
-        else y = rcp_2n(u0);
+        else y = rcp_nr2(u0);
         vx = quot(u1, u0, y);
         vy = quot(u2, u0, y);
         const double e = (double)quot(u3, u0, y);
