@@ -244,6 +244,21 @@ struct RefSpan {
     }
     __device__ __forceinline__ bool ok() const { return low >= R::LO && top < R::HI; }
 };
+// The same by the smallest magnitude, as floats, which order alike and pass over a NaN, and the
+// largest unsigned integer, where a negative value or a NaN is above any other: thin() is true only of
+// a magnitude below LO, not of a cell without a temperature.
+template <class RT>
+struct ThinSpan {
+    using R = RefRange<RT>;
+    unsigned top = 0;
+    float low = __builtin_inff();
+    __device__ __forceinline__ void take(RT x, RT rho) {
+        top = max(top, max((unsigned)R::bits(x), (unsigned)R::bits(rho)));
+        asm("v_min3_f32 %0, %0, |%1|, |%2|" : "+v"(low) : "v"(R::bits(x)), "v"(R::bits(rho)));
+    }
+    __device__ __forceinline__ bool thin() const { return __float_as_int(low) < R::LO; }
+    __device__ __forceinline__ bool ok() const { return !thin() && top < (unsigned)R::HI; }
+};
 
 template <class RT>
 struct RefArith {
@@ -259,8 +274,9 @@ struct RefArith {
         a = (RT)sqrt((double)(gR * T));
         M = vx / a;
     }
+    template <class Span>
     __device__ static __forceinline__ void prim1_fast(RT u0, RT u1, RT u2, int ke, RT cv, double rcv, RT gR, RT& vx,
-                                                      RT& T, RT& a, RT& M, RefSpan<RT>& span) {
+                                                      RT& T, RT& a, RT& M, Span& span) {
         RT y;
         if constexpr (F32) y = rcp_fast(u0);
         else y = rcp_nr2(u0);

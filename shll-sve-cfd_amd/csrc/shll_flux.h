@@ -27,9 +27,9 @@ __device__ __forceinline__ void ref_consts(const Inst& in, RT& cv, double& rcv, 
     }
 }
 // Compute_P_from_U of one cell: the fast form (for cells that pass span), the exact form
-template <class RT>
+template <class RT, class Span>
 __device__ __forceinline__ void ref_prim1(RT u0, RT u1, RT u2, const Inst& in, RT& vx, RT& T, RT& a, RT& M,
-                                          RefSpan<RT>& span) {
+                                          Span& span) {
     RT cv, gR;
     double rcv;
     ref_consts<RT>(in, cv, rcv, gR);
@@ -161,16 +161,25 @@ __device__ __forceinline__ void ref_flux2(const RT (&U)[4], const Prim2<RT>& q, 
     split<RT>(q.vy * (U[3] + P), U[3], z1, z2, z3, yp[3], ym[3]);
 }
 
-// The reference's second-order update term, u - 0.5*lam*x formed in double and stored to RT.
-// EIGHTH: lam = CFL/(R + 1) = 1/8 (DT/DX always, base_shll.c:18,84; DT/DY on square cells).  Then a
-// float x's product is exact in double, and rounding the difference to double first is harmless, so
-// one fused multiply-add gives the same bits.  In one type (FP64, and the first-order term
-// u - lam*x in either) a product below the normal range rounds by itself and is left to: fused, the
-// second-order 2D runs were 1.3-1.5% faster, 1D ones 0.7-1.9%, and states thinner than about
-// 1e-36 (FP64: 1e-306) off in the last bit.
-template <bool EIGHTH, class RT>
+// The reference's update terms: u - lam*x, and the second-order u - 0.5*lam*x formed in double and
+// stored to RT.
+//   EIGHTH: lam = CFL/(R + 1) = 1/8 (DT/DX always, base_shll.c:18,84; DT/DY on square cells).  A
+//     float x's second-order product is exact in double, and rounding the difference to double first
+//     is harmless, so one fused multiply-add gives the same bits.
+//   FUSED: so does it in one type while the product is exact, which a product with bits below the
+//     denormal range is not.  The caller has seen that no cell is thin (ThinSpan).  Then a flux has no
+//     bits below 2^-510 (float: 2^-126): it is a sum of two products, of which one at least has
+//     factors of the order of density, energy or pressure and of the sound speed or M +- 1; and x
+//     is a sum of such fluxes, or of their limited slopes.  (In 2D the transverse momentum's flux
+//     has none of them, and the wavefronts of a tile meet each other's rows: two operations.)
+template <bool FUSED, class RT>
+__device__ __forceinline__ RT ref_first(RT u, RT lam, RT x) {
+    if constexpr (FUSED) return __builtin_elementwise_fma((RT)-0.125, x, u);
+    else return u - lam * x;
+}
+template <bool EIGHTH, bool FUSED = false, class RT>
 __device__ __forceinline__ RT ref_second(RT u, RT lam, RT x) {
-    if constexpr (EIGHTH && sizeof(RT) == 4) return __builtin_elementwise_fma((RT)-0.0625, x, u);
+    if constexpr (FUSED || (EIGHTH && sizeof(RT) == 4)) return __builtin_elementwise_fma((RT)-0.0625, x, u);
     else return (RT)((double)u - 0.5 * (double)lam * (double)x);
 }
 
