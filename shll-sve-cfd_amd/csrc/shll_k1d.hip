@@ -659,11 +659,12 @@ __device__ __forceinline__ void advance_f64f(double (&u)[3][C], const Inst& in, 
                 step_f64f<ORDER, C, WM, LIM, XW, true>(u, in, gl, x, s & 1);
             }
             unit = __all(all.in_range());
-            if (!unit) load_cells<C>((const double*)a.in0 + in.off, a.plane, gl, x.lane, in.nx, slab, u);
         }
     }
-    if (!unit)
+    if (!MAY || __builtin_expect(!unit, 0)) {
+        if constexpr (MAY) load_cells<C>((const double*)a.in0 + in.off, a.plane, gl, x.lane, in.nx, slab, u);
         for (int s = 0; s < ns; ++s) step_f64f<ORDER, C, WM, LIM, XW, false>(u, in, gl, x, s & 1);
+    }
     double* __restrict__ ou = (double*)a.out0 + in.off;
     const int64_t P = a.plane;
     if constexpr (Turn<double, C>::ON) {
