@@ -1101,7 +1101,12 @@ static shll_status engine_create_stream(Engine* E) {
 //   first order   F64 2,16,4 10.5, 2,16,1 7.9; 2,16,4 40.0, 4,16,1 36.0
 //                 C32K 2,16,4 6.8, 2,16,1 6.1; 2,16,4 23.7, 4,16,1 27.8
 // and the largest batches take the autotuner's choices for the 4.7e7-cell one.
-static void default_launch1d(Engine* E, int64_t max_cells) {
+// A single tube beyond 65536 cells takes 2,16,4, the fastest of the shapes tried for the 32-bit forms
+// from 4e5 cells on (us per step, second order, 2,16,4 and 2,16,1 and 4,8,1: REF32 4e5 cells 2.20, 3.65,
+// 2.33, 2e6 7.9, 15.3, 8.2; C32K 1.92, 2.53, 1.95 and 6.8, 10.3, 6.4).  It is not the fastest up to
+// 131072 cells (REF32 1.50, 1.23, 1.49; F64F 1.57, 0.95, 1.18; F64 first order, 65537 cells, 0.98, 0.60,
+// 1.12), nor for the FP64 forms beyond (F64 2e6 cells 12.2, 17.5, 10.2).
+static void default_launch1d(Engine* E) {
     int64_t cells = 0;
     for (int64_t c : E->inst_cells) cells += c;
     const bool f64 = word_bytes(E->prec) == 8;
@@ -1132,7 +1137,7 @@ static void default_launch1d(Engine* E, int64_t max_cells) {
     if (!E->batch) {
         E->L.C = 2;
         E->L.k = 16;
-        E->L.wpb = max_cells <= 65536 ? 1 : 4;
+        E->L.wpb = 4;
         return;
     }
     // {C, k, waves per block} for up to 1e6, up to 2e7 and more cells
@@ -1148,7 +1153,7 @@ static void default_launch1d(Engine* E, int64_t max_cells) {
     E->L.wpb = t[z].w;
 }
 
-static void default_launch(Engine* E, int64_t max_cells) {
+static void default_launch(Engine* E) {
     if (E->dim == 2) {
         // First order: the compensated forms take 4 steps per launch; F64 and REF32 4 on small
         // domains, where a launch costs as much as its steps, and 2 (F64 in between 3) on large
@@ -1172,11 +1177,11 @@ static void default_launch(Engine* E, int64_t max_cells) {
         // beyond the last-level cache lose (C32 3000^2 149 and 157)
         E->L.wpb = E->order == 2 && E->prec == SHLL_F64 ? 1 : 4;
         E->L.rows = default_rows2d(E, E->L.k);
-        // first-order launches of a single instance last 7 us or more and are submitted directly
+        // first-order launches of a single instance last 6 us or more and are submitted directly
         E->L.graph = E->batch || E->order == 2 ? 64 : 0;
         return;
     }
-    default_launch1d(E, max_cells);
+    default_launch1d(E);
 }
 
 extern "C" shll_status shll_init(const shll_problem* pb, const double* prim_soa, shll_ctx** out) {
@@ -1201,7 +1206,7 @@ extern "C" shll_status shll_init(const shll_problem* pb, const double* prim_soa,
     const int64_t cells = pb->nx * pb->ny;
     E->inst_cells.push_back(cells);
     E->order_idx.push_back(0);
-    default_launch(E, cells);
+    default_launch(E);
     if ((st = engine_alloc(E, (cells + 63) / 64 * 64)) != SHLL_OK) { engine_free(E); return st; }
     const double* prims[1] = {prim_soa};
     if ((st = engine_init_state(E, prims)) != SHLL_OK) { engine_free(E); return st; }
@@ -1768,7 +1773,7 @@ extern "C" shll_status shll_batch_init(const shll_problem* items, const double* 
     Engine* E = engine_new(items[0].dim, items[0].order, items[0].precision, items[0].limiter);
     E->batch = true;
     if ((st = engine_create_stream(E)) != SHLL_OK) { engine_free(E); return st; }
-    int64_t off = 0, maxcells = 0, total = 0;
+    int64_t off = 0, total = 0;
     for (int32_t i = 0; i < n; ++i) {
         Inst in;
         std::memset(&in, 0, sizeof(in));
@@ -1784,14 +1789,13 @@ extern "C" shll_status shll_batch_init(const shll_problem* items, const double* 
         E->h_inst.push_back(in);
         E->inst_cells.push_back(cells);
         off += (cells + 63) / 64 * 64;
-        maxcells = std::max(maxcells, cells);
         total += cells * nsteps[i];
     }
     E->order_idx.resize(n);
     for (int32_t i = 0; i < n; ++i) E->order_idx[i] = i;
     std::stable_sort(E->order_idx.begin(), E->order_idx.end(),
                      [&](int64_t a, int64_t b) { return E->h_inst[a].nsteps > E->h_inst[b].nsteps; });
-    default_launch(E, maxcells);
+    default_launch(E);
     if ((st = engine_alloc(E, off)) != SHLL_OK) { engine_free(E); return st; }
     if ((st = engine_init_state(E, prims)) != SHLL_OK) { engine_free(E); return st; }
     if ((st = engine_snapshot(E, true)) != SHLL_OK) { engine_free(E); return st; }

@@ -218,7 +218,7 @@ __device__ __forceinline__ double rsq_nr2(double x) {
 // Before, each of the five (2D: seven) operations carried its own compare and branch, and a
 // gas at rest (u = 0) took the slow path of two of them: 1D first order FP64, 1024 cells,
 // 5.43 us per 8-step launch, 4.2 us now; second order, 4 cells per lane: 894 VALU instructions per
-// step, 582 now; the whole 2D second-order REF32 run at 1024^2 1.12x.
+// step, 581 now; the whole 2D second-order REF32 run at 1024^2 1.12x.
 // ---------------------------------------------------------------------------
 template <class RT> struct RefRange;
 template <> struct RefRange<double> {

@@ -62,8 +62,8 @@ __device__ __forceinline__ void ref_flux1(RT u0, RT u1, RT u2, RT vx, RT T, RT a
 //   Mh = SC M/2 = (u y) SC/(2 sqrt c),  Z1 = Mh + SC/2,  Z3 = Mh - SC/2
 //   Z2 = SC (a/2)(1 - M^2) = s SC sqrt(c)/2 - Mh u
 // 32 FP64 operations and two seeds (36 with p, a^2 and 1 - M^2 formed).  With the limiter's
-// three-instruction form the step of 8 cells issues 659 VALU instructions instead of 715, and a
-// batch of 400 tubes runs in 85.8 instead of 92.6 ms.  Rounding error of a step against 80-bit
+// three-instruction form the step of 8 cells issues 626 VALU instructions instead of 715 (and 12
+// that bound the scaled fluxes, Extremes), and a batch of 400 tubes ran in 85.8 instead of 92.6 ms.  Rounding error of a step against 80-bit
 // arithmetic (rho, m, E relative): 9.6e-18, 1.22e-16, 1.00e-17 before, 9.4e-18, 1.17e-16,
 // 9.8e-18 now; after 20 steps 3.4e-17, 4.7e-16, 2.6e-17 and the same within 5%.
 template <bool UNIT>

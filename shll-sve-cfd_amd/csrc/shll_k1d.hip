@@ -9,7 +9,8 @@
 //   boundary cells and the conservative update in registers         (Update_U_from_F)
 // so a launch of k steps reads the state from HBM once and writes it once; the
 // segment's outer order*k cells on each side are recomputed halo (temporal
-// blocking without LDS and without barriers: wavefronts never wait on each other).
+// blocking without barriers: wavefronts never wait on each other; 8 doubles per lane
+// pass through a wavefront's own LDS on the way from and to memory, Turn).
 // With 4 wavefronts per block and at least 2 cells per lane the block's wavefronts
 // instead hold consecutive segments of one item and swap their edge fluxes through LDS
 // once a step (one barrier), so only the block's ends carry halo.
