@@ -234,8 +234,10 @@ static Consts make_consts(int64_t nx, int64_t ny, double lx, double ly, double t
         k.d_lamx = CFL / (R + 1.0);
         k.d_lamy = DT / DY;
         k.d_rcv = 1.0 / k.d_cv;
-        k.d_sc = std::sqrt(k.d_gR / k.d_cv);
-        k.d_rsc = std::sqrt(k.d_cv / k.d_gR);
+        // the nearest doubles: formed in double, the first would be 0.92 x 2^-53 off in every flux
+        const long double c = (long double)k.d_gR / (long double)k.d_cv;
+        k.d_sc = (double)sqrtl(c);
+        k.d_rsc = (double)(1.0L / sqrtl(c));
         k.u_hsc = std::ldexp(k.d_sc, -513);
         k.u_hrc = std::ldexp(k.d_rsc, -513);
     }
