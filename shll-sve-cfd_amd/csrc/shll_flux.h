@@ -63,9 +63,10 @@ __device__ __forceinline__ void ref_flux1(RT u0, RT u1, RT u2, RT vx, RT T, RT a
 //   Z2 = SC (a/2)(1 - M^2) = s SC sqrt(c)/2 - Mh u
 // 32 FP64 operations and two seeds (36 with p, a^2 and 1 - M^2 formed).  With the limiter's
 // three-instruction form the step of 8 cells issues 626 VALU instructions instead of 715 (and 12
-// that bound the scaled fluxes, Extremes), and a batch of 400 tubes ran in 85.8 instead of 92.6 ms.  Rounding error of a step against 80-bit
-// arithmetic (rho, m, E relative): 9.6e-18, 1.22e-16, 1.00e-17 before, 9.4e-18, 1.17e-16,
-// 9.8e-18 now; after 20 steps 3.4e-17, 4.7e-16, 2.6e-17 and the same within 5%.
+// that bound the scaled fluxes, Extremes), and a batch of 400 tubes ran in 85.8 instead of 92.6 ms.
+// Rounding error of a step against 80-bit arithmetic (rho, m, E relative): 9.6e-18, 1.22e-16,
+// 1.00e-17 with 36 operations, 9.4e-18, 1.22e-16, 9.8e-18 so; after 20 steps 3.42e-17, 4.73e-16,
+// 2.64e-17 and 3.29e-17, 4.42e-16, 2.58e-17.  sqrt c and its reciprocal are the nearest doubles (host).
 template <bool UNIT>
 __device__ __forceinline__ void flux1_f64f(double u0, double u1, double u2, const Inst& in, double (&fp)[3],
                                            double (&fm)[3], double& a) {
