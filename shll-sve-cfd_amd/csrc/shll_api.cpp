@@ -32,7 +32,7 @@ bool step2d_supported(int prec, int order, int k);
 int tile2d_rows(int prec, int k, int cus, int64_t (*tiles)(const void*, int), const void* arg);
 hipError_t launch_tile2d(int prec, int rows, int n_items, hipStream_t s, const StepArgs& a);
 hipError_t launch_init(int prec, int dim, int nblocks, int n_inst, hipStream_t st, const Inst* insts,
-                       const double* prim, void* o0, void* o1, int64_t plane);
+                       const double* prim, int64_t width, int64_t c0, void* o0, void* o1, int64_t plane);
 hipError_t launch_stage(int prec, int dim, int nblocks, hipStream_t st, const Inst* inst, const void* s0,
                         int64_t plane, double* out);
 hipError_t launch_output(int prec, int dim, int nblocks, int n_inst, hipStream_t st, const Inst* insts,
@@ -880,67 +880,69 @@ static shll_status ensure_prim(Engine* E) {
     return SHLL_OK;
 }
 
-// upload primitives of all instances and convert them (k_init) into buffer 0
+// Upload primitives of all instances and convert them (k_init) into buffer 0.  Large ones wait on
+// the device in buffer 1, which is free until the first step: as doubles they fill it once, or in the
+// 32-bit forms twice, half of the cells at a time.
 static shll_status engine_init_state(Engine* E, const double* const* prims) {
     const size_t total = (size_t)E->plane * E->nv * sizeof(double);
     int64_t maxcells = 0;
     for (int64_t c : E->inst_cells) maxcells = std::max(maxcells, c);
-    // bytes [at, at + len) of the device layout (planes of all instances, each padded to 64 cells)
-    auto gather = [&](char* dst, size_t at, size_t len) {
-        size_t g = at / sizeof(double);
-        const size_t end = (at + len) / sizeof(double);
-        while (g < end) {
-            const size_t v = g / (size_t)E->plane, o = g % (size_t)E->plane;
-            // the instance at offset o: the last one that starts at or before it
+    // doubles [at, at + n) of cells [c0, c0 + width) of the device layout (the instances one after the
+    // other, each padded to 64 cells), a plane of `width` per variable
+    auto gather = [&](double* dst, size_t at, size_t n, size_t c0, size_t width) {
+        const size_t end = at + n;
+        for (size_t g = at; g < end;) {
+            const size_t v = g / width, o = c0 + g % width;
+            const size_t last = std::min(end, (v + 1) * width);  // of this variable
+            // the instance at cell o: the last one that starts at or before it
             size_t i = std::upper_bound(E->h_inst.begin(), E->h_inst.end(), (int64_t)o,
                                         [](int64_t x, const Inst& in) { return x < in.off; }) - E->h_inst.begin() - 1;
-            for (; i < E->h_inst.size() && g < end && g / (size_t)E->plane == v; ++i) {
+            for (; g < last; ++i) {
                 const size_t off = (size_t)E->h_inst[i].off, nc = (size_t)E->inst_cells[i];
                 const size_t stop = i + 1 < E->h_inst.size() ? (size_t)E->h_inst[i + 1].off : (size_t)E->plane;
-                const size_t from = g - v * (size_t)E->plane - off;  // cell within the instance, or its padding
-                const size_t take = from < nc ? std::min(nc - from, end - g) : 0;
-                std::memcpy(dst + g * sizeof(double) - at, prims[i] + v * nc + from, take * sizeof(double));
-                g = std::min(end, v * (size_t)E->plane + stop);
+                const size_t from = c0 + g - v * width - off;  // cell within the instance, or its padding
+                const size_t take = from < nc ? std::min(nc - from, last - g) : 0;
+                std::memcpy(dst + (g - at), prims[i] + v * nc + from, take * sizeof(double));
+                g = std::min(last, v * width + stop - c0);
             }
         }
     };
-    auto convert = [&](const double* src) {
+    auto convert = [&](const double* src, size_t c0, size_t width) {
         return launch_init(E->prec, E->dim, elem_blocks(maxcells), (int)E->h_inst.size(), E->stream, E->d_inst, src,
-                           E->buf[0][0], E->buf[0][1], E->plane);
+                           (int64_t)width, (int64_t)c0, E->buf[0][0], E->buf[0][1], E->plane);
     };
+    hipError_t e = hipSuccess;
     bool done = false;
     if (total <= kSlabBytes) {
         Slab slab;
         if (slab.pinned) {
-            gather(slab.p, 0, total);
-            const hipError_t e = convert((const double*)slab.p);
+            gather((double*)slab.p, 0, total / sizeof(double), 0, (size_t)E->plane);
+            e = convert((const double*)slab.p, 0, (size_t)E->plane);
             const hipError_t w = hipStreamSynchronize(E->stream);
-            if (e != hipSuccess || w != hipSuccess)
-                return fail(SHLL_EDEVICE, "init kernel: %s", hipGetErrorString(e != hipSuccess ? e : w));
+            if (e == hipSuccess) e = w;
             done = true;
         }
     }
     if (!done) {
-        shll_status st = ensure_prim(E);
-        if (st != SHLL_OK) return st;
-        auto len = [&](size_t i) { return std::min(kSlabBytes, total - i * kSlabBytes); };
-        hipError_t e = transfer(
-            E->device, E->stream, (total + kSlabBytes - 1) / kSlabBytes,
-            [&](size_t i, char* slab) {
-                gather(slab, i * kSlabBytes, len(i));
-                return hipMemcpyAsync((char*)E->d_prim + i * kSlabBytes, slab, len(i), hipMemcpyHostToDevice, E->stream);
-            },
-            [](size_t, const char*) {});
-        if (e != hipSuccess) return fail(SHLL_EDEVICE, "upload: %s", hipGetErrorString(e));
-        e = convert(E->d_prim);
+        constexpr size_t piece = kSlabBytes / sizeof(double);
+        double* const dev = (double*)E->buf[1][0];
+        const size_t width = (size_t)E->plane * word_bytes(E->prec) / sizeof(double), n = width * E->nv;
+        for (size_t c0 = 0; c0 < (size_t)E->plane && e == hipSuccess; c0 += width) {
+            e = transfer(
+                E->device, E->stream, (n + piece - 1) / piece,
+                [&](size_t i, char* slab) {
+                    const size_t at = i * piece, len = std::min(piece, n - at);
+                    gather((double*)slab, at, len, c0, width);
+                    return hipMemcpyAsync(dev + at, slab, len * sizeof(double), hipMemcpyHostToDevice, E->stream);
+                },
+                [](size_t, const char*) {});
+            if (e != hipSuccess) return fail(SHLL_EDEVICE, "upload: %s", hipGetErrorString(e));
+            e = convert(dev, c0, width);
+        }
         const hipError_t w = hipStreamSynchronize(E->stream);
-        // as large as a buffer of an FP64 state: a solver that is only stepped, or a batch that takes
-        // its snapshot next, does not hold it (a first large read allocates it again)
-        (void)hipFree(E->d_prim);
-        E->d_prim = nullptr;
-        if (e != hipSuccess || w != hipSuccess)
-            return fail(SHLL_EDEVICE, "init kernel: %s", hipGetErrorString(e != hipSuccess ? e : w));
+        if (e == hipSuccess) e = w;
     }
+    if (e != hipSuccess) return fail(SHLL_EDEVICE, "init kernel: %s", hipGetErrorString(e));
     engine_rewind(E);
     return SHLL_OK;
 }

@@ -18,18 +18,21 @@
 
 namespace shll {
 
-// primitives (rho, u, (v), T) -> conserved, per precision
+// primitives (rho, u, (v), T) -> conserved, per precision.  prim holds cells [c0, c0 + width) of the
+// state's layout, a plane of `width` per variable; the others are left alone.
 template <int PREC, int DIM>
-__global__ __launch_bounds__(256) void k_init(const Inst* insts, const double* __restrict__ prim, void* out0,
-                                              void* out1, int64_t plane) {
+__global__ __launch_bounds__(256) void k_init(const Inst* insts, const double* __restrict__ prim, int64_t width,
+                                              int64_t c0, void* out0, void* out1, int64_t plane) {
     const Inst in = insts[blockIdx.y];
     const int64_t ncell = (int64_t)in.nx * in.ny;
     for (int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; c < ncell;
          c += (int64_t)gridDim.x * blockDim.x) {
         const int64_t o = in.off + c;
-        const double r = prim[o], vx = prim[plane + o];
-        const double vy = DIM == 2 ? prim[2 * plane + o] : 0.0;
-        const double T = prim[(DIM == 2 ? 3 : 2) * plane + o];
+        const int64_t i = o - c0;
+        if (i < 0 || i >= width) continue;
+        const double r = prim[i], vx = prim[width + i];
+        const double vy = DIM == 2 ? prim[2 * width + i] : 0.0;
+        const double T = prim[(DIM == 2 ? 3 : 2) * width + i];
         double U[4];
         if constexpr (PREC == PREC_REF32) {
             const float rf = (float)r, vxf = (float)vx, vyf = (float)vy, Tf = (float)T, cv = in.k.f_cv;
@@ -251,20 +254,21 @@ hipError_t launch_ctl(hipStream_t st, int64_t* ctl, int64_t v0, int64_t v1, int6
 
 // ---------------------------------------------------------------------------
 template <int PREC>
-static hipError_t init_p(int dim, dim3 g, hipStream_t st, const Inst* insts, const double* prim, void* o0,
-                         void* o1, int64_t plane) {
-    if (dim == 1) hipLaunchKernelGGL((k_init<PREC, 1>), g, dim3(256), 0, st, insts, prim, o0, o1, plane);
-    else hipLaunchKernelGGL((k_init<PREC, 2>), g, dim3(256), 0, st, insts, prim, o0, o1, plane);
+static hipError_t init_p(int dim, dim3 g, hipStream_t st, const Inst* insts, const double* prim, int64_t width,
+                         int64_t c0, void* o0, void* o1, int64_t plane) {
+    if (dim == 1) hipLaunchKernelGGL((k_init<PREC, 1>), g, dim3(256), 0, st, insts, prim, width, c0, o0, o1, plane);
+    else hipLaunchKernelGGL((k_init<PREC, 2>), g, dim3(256), 0, st, insts, prim, width, c0, o0, o1, plane);
     return hipGetLastError();
 }
 
 hipError_t launch_init(int prec, int dim, int nblocks, int n_inst, hipStream_t st, const Inst* insts,
-                       const double* prim, void* o0, void* o1, int64_t plane) {
+                       const double* prim, int64_t width, int64_t c0, void* o0, void* o1, int64_t plane) {
     dim3 g(nblocks, n_inst);
     // F64F keeps its state as F64 does (one double plane per variable, same initial values)
-    if (prec == PREC_F64 || prec == PREC_F64F) return init_p<PREC_F64>(dim, g, st, insts, prim, o0, o1, plane);
-    if (prec == PREC_REF32) return init_p<PREC_REF32>(dim, g, st, insts, prim, o0, o1, plane);
-    return init_p<PREC_C32>(dim, g, st, insts, prim, o0, o1, plane);
+    if (prec == PREC_F64 || prec == PREC_F64F)
+        return init_p<PREC_F64>(dim, g, st, insts, prim, width, c0, o0, o1, plane);
+    if (prec == PREC_REF32) return init_p<PREC_REF32>(dim, g, st, insts, prim, width, c0, o0, o1, plane);
+    return init_p<PREC_C32>(dim, g, st, insts, prim, width, c0, o0, o1, plane);
 }
 
 // sound speed a and split fluxes (x: fp, fm; y: hp, hm) of every cell of one instance;

@@ -46,6 +46,26 @@ def test_initial_data_are_not_kept(prec, words, batch):
             break
         time.sleep(0.02)
     assert used < most, "used %d, state buffers %d" % (used, held)
-    got = s.primitives(0) if batch else s.primitives()
-    assert np.isfinite(got).all()
+    first = s.primitives(0) if batch else s.primitives()
+    assert np.isfinite(first).all()
     s.close()
+
+
+@pytest.mark.parametrize("prec", [S.F64F, S.REF32, S.C32, S.C32K])
+def test_initial_data_of_uneven_batches(prec):
+    """Large initial data pass through the second state buffer, in the 32-bit forms half of the cells at
+    a time: halves and transfers end inside instances, in their padding and between them.  Each
+    instance is that of a solver of its own, whose data fit one transfer."""
+    for sizes in ([3, 100003, 64, 170000, 5, 160001, 1000, 130001], [100000] * 4, [64, 128, 174700, 174700, 64, 128], [350000, 2]):
+        ics = [icgen.random_1d(n, 20 + i, block=500) for i, n in enumerate(sizes)]
+        pbs = [S.problem(1, 1, n, precision=prec) for n in sizes]
+        banner("initial data", prec, sizes)
+        b = S.Batch(pbs, ics, [1] * len(sizes))
+        for i, n in enumerate(sizes):
+            part = min(n, 170000)  # 4 MB
+            with S.Solver(S.problem(1, 1, part, precision=prec), np.array(ics[i]).reshape(3, n)[:, :part].reshape(-1)) as s:
+                np.testing.assert_array_equal(b.conserved(i)[:, :part], s.conserved(), err_msg="n=%d" % n)
+            if part < n:
+                with S.Solver(S.problem(1, 1, n - part, precision=prec), np.array(ics[i]).reshape(3, n)[:, part:].reshape(-1)) as s:
+                    np.testing.assert_array_equal(b.conserved(i)[:, part:], s.conserved(), err_msg="n=%d" % n)
+        b.close()
