@@ -82,19 +82,22 @@ extern "C" const char* shll_version(void) { return "shll_amd 0.1 (gfx950)"; }
 // pinning a buffer per call costs 0.1 ms to 40 ms.  So transfers go through pinned slabs of 4
 // MiB that are kept between calls: up to 4 MiB the output kernels write straight into one slab
 // (no copy command, one synchronisation), beyond that up to eight threads each take the next
-// piece, copy it between its slab and the caller's memory, and have a second piece in flight.
+// piece, copy it between its slab and the caller's memory, and have a second piece in flight: in the
+// slab's other half, and from 128 MiB on in a second slab (537 MB 14.1 ms in halves, 12.5 in whole
+// slabs; below, pinning the second ones, 0.1 to 0.2 ms each, takes longer than they save).
 // Where no memory can be pinned, ordinary memory takes a slab's place, at the runtime's pace.
 // Measured (16-core host), before and now: 24 KB of primitives 48 and 14 us, 111 MB of 400 tubes
 // one by one 24 and 11.8 ms, 537 MB 51.5 and 12.5 ms; constructing a 128^2 context 183 and 96 us.
 // ---------------------------------------------------------------------------
 namespace {
 constexpr size_t kSlabBytes = 4u << 20;
-constexpr size_t kSlabsKept = 16, kSlabsIdle = 2;
+constexpr size_t kLargeTransfer = 128u << 20;
+constexpr size_t kSlabsKept = 16, kSlabsIdle = 4;
 
 // The slabs not in use: at most kSlabsKept stay allocated while there is a context or batch, the
-// others are freed when they are returned; when the last context goes, all but kSlabsIdle (what a
-// program needs that makes small contexts one after another) are freed.  Portable, so any device
-// may use any slab.
+// others are freed when they are returned; when the last context goes, all but kSlabsIdle are freed, so
+// that a program that makes contexts one after another pins few or none each time.  Portable, so
+// any device may use any slab.
 std::mutex g_slab_mu;
 char* g_slabs[kSlabsKept];
 size_t g_nslabs = 0;
@@ -103,7 +106,8 @@ int64_t g_engines = 0;  // contexts and batches
 struct Slab {
     char* p = nullptr;
     bool pinned = true;  // a kernel may write to it
-    Slab() {
+    explicit Slab(bool none = false) {
+        if (none) return;
         {
             std::lock_guard<std::mutex> lock(g_slab_mu);
             if (g_nslabs > 0) {
@@ -118,6 +122,7 @@ struct Slab {
     }
     // its last use by the device must have completed
     ~Slab() {
+        if (!p) return;
         if (!pinned) {
             std::free(p);
             return;
@@ -146,34 +151,36 @@ void slabs_engine(int64_t d) {
     while (n > 0) (void)hipHostFree(idle[--n]);
 }
 
-// Pieces [0, n) of a transfer.  start(i, slab): enqueue the copy between slab and device (an
-// upload fills the slab first); finish(i, slab): after it has completed.  Every piece is done by
-// the time this returns; the first error wins.
+// A transfer of `bytes` in pieces.  start(at, len, slab): enqueue the copy of a piece between slab
+// and device (an upload fills the slab first); finish(at, len, slab): after it has completed.  Every
+// piece is done by the time this returns; the first error wins.
 template <class Start, class Finish>
-hipError_t transfer(int device, hipStream_t stream, size_t n, const Start& start, const Finish& finish) {
+hipError_t transfer(int device, hipStream_t stream, size_t bytes, const Start& start, const Finish& finish) {
+    const bool large = bytes >= kLargeTransfer;
+    const size_t piece = large ? kSlabBytes : kSlabBytes / 2, n = (bytes + piece - 1) / piece;
+    auto len = [&](size_t i) { return std::min(piece, bytes - i * piece); };
     std::atomic<size_t> next{0};
     std::atomic<int> error{(int)hipSuccess};
     auto work = [&]() {
         hipError_t e = hipSetDevice(device);
-        Slab slab[2];
+        Slab first, second(!large);
+        char* const room[2] = {first.p, large ? second.p : first.p + piece};
+        if (!first.p || !room[1]) e = hipErrorOutOfMemory;
         hipEvent_t ev[2] = {nullptr, nullptr};
-        for (int q = 0; q < 2 && e == hipSuccess; ++q) {
-            if (!slab[q].p) e = hipErrorOutOfMemory;
-            else e = hipEventCreateWithFlags(&ev[q], hipEventDisableTiming);
-        }
+        for (int q = 0; q < 2 && e == hipSuccess; ++q) e = hipEventCreateWithFlags(&ev[q], hipEventDisableTiming);
         size_t at[2];
         bool busy[2] = {false, false};
         for (int q = 0;; q ^= 1) {
             if (busy[q]) {
                 const hipError_t w = hipEventSynchronize(ev[q]);
                 busy[q] = false;
-                if (w == hipSuccess) finish(at[q], slab[q].p);
+                if (w == hipSuccess) finish(at[q] * piece, len(at[q]), room[q]);
                 else if (e == hipSuccess) e = w;
             }
             const size_t i = e == hipSuccess && error.load() == (int)hipSuccess ? next.fetch_add(1) : n;
             if (i < n) {
                 at[q] = i;
-                const hipError_t c = start(i, slab[q].p);
+                const hipError_t c = start(i * piece, len(i), room[q]);
                 const hipError_t r = hipEventRecord(ev[q], stream);
                 busy[q] = true;  // waited for even after an error, so the slab is idle when it goes back
                 e = c != hipSuccess ? c : r;
@@ -924,20 +931,19 @@ static shll_status engine_init_state(Engine* E, const double* const* prims) {
         }
     }
     if (!done) {
-        constexpr size_t piece = kSlabBytes / sizeof(double);
-        double* const dev = (double*)E->buf[1][0];
-        const size_t width = (size_t)E->plane * word_bytes(E->prec) / sizeof(double), n = width * E->nv;
+        constexpr size_t D = sizeof(double);
+        char* const dev = (char*)E->buf[1][0];
+        const size_t width = (size_t)E->plane * word_bytes(E->prec) / D;
         for (size_t c0 = 0; c0 < (size_t)E->plane && e == hipSuccess; c0 += width) {
             e = transfer(
-                E->device, E->stream, (n + piece - 1) / piece,
-                [&](size_t i, char* slab) {
-                    const size_t at = i * piece, len = std::min(piece, n - at);
-                    gather((double*)slab, at, len, c0, width);
-                    return hipMemcpyAsync(dev + at, slab, len * sizeof(double), hipMemcpyHostToDevice, E->stream);
+                E->device, E->stream, width * E->nv * D,
+                [&](size_t at, size_t len, char* slab) {
+                    gather((double*)slab, at / D, len / D, c0, width);
+                    return hipMemcpyAsync(dev + at, slab, len, hipMemcpyHostToDevice, E->stream);
                 },
-                [](size_t, const char*) {});
+                [](size_t, size_t, const char*) {});
             if (e != hipSuccess) return fail(SHLL_EDEVICE, "upload: %s", hipGetErrorString(e));
-            e = convert(dev, c0, width);
+            e = convert((const double*)dev, c0, width);
         }
         const hipError_t w = hipStreamSynchronize(E->stream);
         if (e == hipSuccess) e = w;
@@ -964,14 +970,12 @@ static shll_status engine_snapshot(Engine* E, bool save) {
 
 // contiguous device memory to the caller's
 static shll_status download(Engine* E, void* dst, const void* src, size_t bytes) {
-    const size_t n = (bytes + kSlabBytes - 1) / kSlabBytes;
-    auto len = [&](size_t i) { return std::min(kSlabBytes, bytes - i * kSlabBytes); };
     HIPCHECK(transfer(
-        E->device, E->stream, n,
-        [&](size_t i, char* slab) {
-            return hipMemcpyAsync(slab, (const char*)src + i * kSlabBytes, len(i), hipMemcpyDeviceToHost, E->stream);
+        E->device, E->stream, bytes,
+        [&](size_t at, size_t len, char* slab) {
+            return hipMemcpyAsync(slab, (const char*)src + at, len, hipMemcpyDeviceToHost, E->stream);
         },
-        [&](size_t i, const char* slab) { std::memcpy((char*)dst + i * kSlabBytes, slab, len(i)); }));
+        [&](size_t at, size_t len, const char* slab) { std::memcpy((char*)dst + at, slab, len); }));
     return SHLL_OK;
 }
 
