@@ -539,8 +539,7 @@ static void engine_free(Engine* E) {
     if (E->stream) (void)hipStreamSynchronize(E->stream);
     engine_drop_graphs(E);
     for (int b = 0; b < 2; ++b)
-        for (int w = 0; w < 2; ++w)
-            if (E->buf[b][w]) (void)hipFree(E->buf[b][w]);
+        if (E->buf[b][0]) (void)hipFree(E->buf[b][0]);
     for (int w = 0; w < 2; ++w)
         if (E->init_copy[w]) (void)hipFree(E->init_copy[w]);
     if (E->d_inst) (void)hipFree(E->d_inst);
@@ -865,12 +864,14 @@ static int inst_parity(const Engine* E, int64_t i) {
 static shll_status engine_alloc(Engine* E, int64_t plane) {
     E->plane = plane;
     const size_t bytes = (size_t)plane * E->nv * word_bytes(E->prec);
-    for (int b = 0; b < 2; ++b)
-        for (int w = 0; w < nwords(E->prec); ++w) {
-            hipError_t e = hipMalloc(&E->buf[b][w], bytes);
-            if (e != hipSuccess) return fail(SHLL_ENOMEM, "hipMalloc(%zu) for the state: %s", bytes, hipGetErrorString(e));
-            HIPCHECK(hipMemsetAsync(E->buf[b][w], 0, bytes, E->stream));
-        }
+    // a buffer's words lie one after the other
+    const size_t all = bytes * nwords(E->prec);
+    for (int b = 0; b < 2; ++b) {
+        hipError_t e = hipMalloc(&E->buf[b][0], all);
+        if (e != hipSuccess) return fail(SHLL_ENOMEM, "hipMalloc(%zu) for the state: %s", all, hipGetErrorString(e));
+        HIPCHECK(hipMemsetAsync(E->buf[b][0], 0, all, E->stream));
+        if (nwords(E->prec) == 2) E->buf[b][1] = (char*)E->buf[b][0] + bytes;
+    }
     const size_t inst_bytes = E->h_inst.size() * sizeof(Inst);
     HIPCHECK(hipMalloc(&E->d_inst, inst_bytes));
     HIPCHECK(hipMemcpyAsync(E->d_inst, E->h_inst.data(), inst_bytes, hipMemcpyHostToDevice, E->stream));
@@ -888,8 +889,8 @@ static shll_status ensure_prim(Engine* E) {
 }
 
 // Upload primitives of all instances and convert them (k_init) into buffer 0.  Large ones wait on
-// the device in buffer 1, which is free until the first step: as doubles they fill it once, or in the
-// 32-bit forms twice, half of the cells at a time.
+// the device in buffer 1, which is free until the first step: as doubles they fill it once, in REF32
+// twice, half of the cells at a time.
 static shll_status engine_init_state(Engine* E, const double* const* prims) {
     const size_t total = (size_t)E->plane * E->nv * sizeof(double);
     int64_t maxcells = 0;
@@ -933,7 +934,7 @@ static shll_status engine_init_state(Engine* E, const double* const* prims) {
     if (!done) {
         constexpr size_t D = sizeof(double);
         char* const dev = (char*)E->buf[1][0];
-        const size_t width = (size_t)E->plane * word_bytes(E->prec) / D;
+        const size_t width = (size_t)E->plane * word_bytes(E->prec) * nwords(E->prec) / D;
         for (size_t c0 = 0; c0 < (size_t)E->plane && e == hipSuccess; c0 += width) {
             e = transfer(
                 E->device, E->stream, width * E->nv * D,
@@ -1001,10 +1002,16 @@ static shll_status engine_get(Engine* E, int64_t i, double* prim, double* cons) 
             return SHLL_OK;
         }
     }
-    shll_status st = ensure_prim(E);
-    if (st != SHLL_OK) return st;
-    HIPCHECK(output(E->d_prim));
-    return download(E, dst, E->d_prim, bytes);
+    // the doubles wait on the device in the buffer that the next step writes, if they fit it (a batch's
+    // holds the states of instances that took fewer launches)
+    double* stage = (double*)E->buf[p ^ 1][0];
+    if (E->batch || word_bytes(E->prec) * nwords(E->prec) < sizeof(double)) {
+        shll_status st = ensure_prim(E);
+        if (st != SHLL_OK) return st;
+        stage = E->d_prim;
+    }
+    HIPCHECK(output(stage));
+    return download(E, dst, stage, bytes);
 }
 
 static shll_status ensure_partial(Engine* E, size_t n) {

@@ -46,15 +46,26 @@ def test_initial_data_are_not_kept(prec, words, batch):
             break
         time.sleep(0.02)
     assert used < most, "used %d, state buffers %d" % (used, held)
+    # reads pass through that buffer too, between any steps
     first = s.primitives(0) if batch else s.primitives()
+    if not batch:
+        cons = s.conserved()
+        s.step(2)
+        s.primitives()
+        s.step(3)
+        with S.Solver(pb, ic) as t:
+            t.step(3)
+            np.testing.assert_array_equal(t.conserved(), cons)
+            t.step(5)
+            np.testing.assert_array_equal(t.state_raw(), s.state_raw())
     assert np.isfinite(first).all()
     s.close()
 
 
 @pytest.mark.parametrize("prec", [S.F64F, S.REF32, S.C32, S.C32K])
 def test_initial_data_of_uneven_batches(prec):
-    """Large initial data pass through the second state buffer, in the 32-bit forms half of the cells at
-    a time: halves and transfers end inside instances, in their padding and between them.  Each
+    """Large initial data pass through the second state buffer, in REF32 half of the cells at a time:
+    halves and transfers end inside instances, in their padding and between them.  Each
     instance is that of a solver of its own, whose data fit one transfer."""
     for sizes in ([3, 100003, 64, 170000, 5, 160001, 1000, 130001], [100000] * 4, [64, 128, 174700, 174700, 64, 128], [350000, 2]):
         ics = [icgen.random_1d(n, 20 + i, block=500) for i, n in enumerate(sizes)]
